@@ -11,15 +11,90 @@
 // solves, which then need only matrix-vector work per block.
 #include "common.h"
 #include "kernels.h"
+#include "mfma.h"
 #include "profile.h"
 
 namespace mbd {
 
 namespace {
 
+constexpr int DB = 32;                             // sub-block of a diagonal block
+constexpr int DNB = kCholNB / DB;                  // sub-blocks per edge
+constexpr int DTRI = DNB * (DNB + 1) / 2;
+static_assert(DNB == 4, "the inverse's doubling steps are written for 4 x 4 sub-blocks");
+
 template <typename T>
-__device__ inline T dev_sqrt(T x) {
-  return sqrt(x);
+using Sub = T[DB][DB + 1];  // row-major sub-block in LDS
+
+// LDS of k_potrf_diag: the lower sub-blocks, R^{-1} of the diagonal ones
+// (R = L^T), and two scratch blocks.
+template <typename T>
+struct DiagLds {
+  Sub<T> l[DTRI];
+  Sub<T> ri[DNB];
+  Sub<T> w[2];
+};
+
+__device__ constexpr int sub_index(int i, int j) { return i * (i + 1) / 2 + j; }
+
+// The 16 x 16 tile (wave >> 1, wave & 1) of op(A) op(B) added to acc, on
+// MFMA; op transposes where TA / TB is set.
+template <typename T, bool TA, bool TB>
+__device__ inline void sub_mm(typename Mfma<T>::acc_t &acc, const Sub<T> &A, const Sub<T> &Bm) {
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, lr = lane & 15, lk = lane >> 4;
+  const int r = 16 * (wv >> 1) + lr, c = 16 * (wv & 1) + lr;
+#pragma unroll
+  for (int k = 0; k < DB; k += 4) {
+    const T a = TA ? A[k + lk][r] : A[r][k + lk];
+    const T b = TB ? Bm[c][k + lk] : Bm[k + lk][c];
+    acc = Mfma<T>::mma(a, b, acc);
+  }
+}
+
+// C = alpha acc (+ C): each wave its tile.
+template <typename T, bool ADD>
+__device__ inline void sub_put(Sub<T> &C, const typename Mfma<T>::acc_t &acc, T alpha) {
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, lr = lane & 15, lk = lane >> 4;
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    T *p = &C[16 * (wv >> 1) + Mfma<T>::row(lk, v)][16 * (wv & 1) + lr];
+    *p = ADD ? *p + alpha * acc[v] : alpha * acc[v];
+  }
+}
+
+// Lower Cholesky of the 32 x 32 sub-block G (lower triangle read) by one
+// wave, without barriers: lanes 0..31 hold G's columns and lanes 32..63 the
+// identity's, step k applies the same row operations to both with pivot
+// column k read from lane k through the scalar unit, and the identity ends as
+// the inverse factor (32 steps at one barrier and one LDS round trip each
+// cost 20 us, this 9 us in FP64).  Writes L over G and L^{-T} to Ri, zeros
+// outside the triangles; returns the first non-positive pivot, or DB (such
+// steps divide by 1 and carry on).
+template <typename T>
+__device__ __forceinline__ int wave_chol(Sub<T> &G, Sub<T> &Ri) {
+  const int lane = threadIdx.x & 63, j = lane & (DB - 1);
+  const bool ih = lane >= DB;  // identity half
+  T x[DB];
+#pragma unroll
+  for (int i = 0; i < DB; ++i) x[i] = G[i > j ? i : j][i > j ? j : i];
+#pragma unroll
+  for (int i = 0; i < DB; ++i) x[i] = ih ? (i == j ? T(1) : T(0)) : x[i];
+  int bad = DB;
+#pragma unroll
+  for (int k = 0; k < DB; ++k) {
+    const T d = lane_value(x[k], k);
+    if (!(d > T(0)) && bad == DB) bad = k;
+    const T dd = d > T(0) ? d : T(1);
+    // column k of L and of L^{-T} are final
+    const bool in = ih ? (j <= k) : (k <= j);
+    T *p = ih ? &Ri[j][k] : &G[j][k];
+    *p = in ? x[k] * rsq_fast(dd) : T(0);
+    if (k == DB - 1) break;
+    const T a = (ih || j > k) ? x[k] * rcp_fast(dd) : T(0);
+#pragma unroll
+    for (int i = k + 1; i < DB; ++i) x[i] = fma(-lane_value(x[i], k), a, x[i]);
+  }
+  return bad;
 }
 
 }  // namespace
@@ -28,74 +103,136 @@ __device__ inline T dev_sqrt(T x) {
 // batch, write L11 back, and write inv(L11) (kb x kb, zero above the
 // diagonal) to inv + b * sinv with leading dimension NB.  info[b] records the
 // first non-positive pivot as k0 + j + 1 (LAPACK convention).
+//
+// One workgroup per matrix, so a chain of dependent steps bounds it: four
+// 32 x 32 factorisations by one wave each with the panel and trailing
+// sub-blocks on MFMA between them, then the inverse by doubling (2 + 6
+// products).  A column at a time with a barrier per step took 610 us for a
+// 128 x 128 block, FP32 and FP64 alike.
 template <typename T>
 __global__ __launch_bounds__(256) void k_potrf_diag(T *A, int lda, long sA,
                                                     int k0, int kb, T *inv,
                                                     long sinv, int *info) {
   extern __shared__ unsigned char smem_raw[];
-  T *L = reinterpret_cast<T *>(smem_raw);
-  const int ldl = kb + 1;
-  T *dg = L + (long)ldl * kb;   // diagonal of L, then of inv(L)
-  T *tmp = dg + kb;             // column scratch
+  DiagLds<T> &s = *reinterpret_cast<DiagLds<T> *>(smem_raw);
+  using acc_t = typename Mfma<T>::acc_t;
+  const acc_t zero = {0, 0, 0, 0};
   const int b = blockIdx.x, t = threadIdx.x;
   T *M = A + (long)b * sA + k0 + (long)k0 * lda;
 
-  for (int e = t; e < kb * kb; e += blockDim.x) {
-    const int r = e % kb, c = e / kb;
-    if (r >= c) L[c * ldl + r] = M[r + (long)c * lda];
+  // lower triangle into the sub-blocks, 16 columns in flight per thread
+  // (clamped addresses); the identity past kb
+  const int r = t & (kCholNB - 1), rc = min(r, kb - 1), ch = t >> 7;
+  for (int c0 = 0; c0 < kCholNB; c0 += 32) {
+    T v[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[i] = M[rc + (long)min(c0 + ch + 2 * i, kb - 1) * lda];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int c = c0 + ch + 2 * i;
+      if (r / DB >= c / DB)
+        s.l[sub_index(r / DB, c / DB)][r % DB][c % DB] =
+            (r < kb && c < kb) ? v[i] : (r == c ? T(1) : T(0));
+    }
   }
   __syncthreads();
-  for (int j = 0; j < kb; ++j) {
-    const T d = L[j * ldl + j];
-    const bool bad = !(d > T(0));
-    const T ljj = bad ? T(1) : dev_sqrt(d);
-    const T rinv = T(1) / ljj;
-    if (t == 0) {
-      dg[j] = ljj;
-      if (bad && info[b] == 0) info[b] = k0 + j + 1;
+  const int nb = (kb + DB - 1) / DB;
+  for (int k = 0; k < nb; ++k) {
+    if (t < 64) {
+      const int bad = wave_chol<T>(s.l[sub_index(k, k)], s.ri[k]);
+      if (t == 0 && bad < DB && info[b] == 0) info[b] = k0 + k * DB + bad + 1;
     }
-    for (int r = j + 1 + t; r < kb; r += blockDim.x) L[j * ldl + r] *= rinv;
     __syncthreads();
-    for (int c = j + 1 + (t >> 4); c < kb; c += 16) {
-      const T lc = L[j * ldl + c];
-      for (int r = c + (t & 15); r < kb; r += 16) L[c * ldl + r] -= L[j * ldl + r] * lc;
-    }
+    if (k + 1 == nb) break;
+    // sub-blocks below: L_ik = A_ik L_kk^{-T}
+    acc_t p[DNB - 1] = {zero, zero, zero};
+#pragma unroll
+    for (int i = 0; i < DNB - 1; ++i)
+      if (k + 1 + i < nb) sub_mm<T, false, false>(p[i], s.l[sub_index(k + 1 + i, k)], s.ri[k]);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < DNB - 1; ++i)
+      if (k + 1 + i < nb) sub_put<T, false>(s.l[sub_index(k + 1 + i, k)], p[i], T(1));
+    __syncthreads();
+    for (int i = k + 1; i < nb; ++i)
+      for (int j = k + 1; j <= i; ++j) {
+        acc_t q = zero;
+        sub_mm<T, false, true>(q, s.l[sub_index(i, k)], s.l[sub_index(j, k)]);
+        sub_put<T, true>(s.l[sub_index(i, j)], q, T(-1));
+      }
     __syncthreads();
   }
-  // write L11 (lower, with its diagonal)
-  for (int e = t; e < kb * kb; e += blockDim.x) {
-    const int r = e % kb, c = e / kb;
-    if (r > c)
-      M[r + (long)c * lda] = L[c * ldl + r];
-    else if (r == c)
-      M[r + (long)c * lda] = dg[r];
+  for (int c0 = 0; c0 < kCholNB; c0 += 2) {
+    const int c = c0 + ch;
+    if (r >= c && r < kb) M[r + (long)c * lda] = s.l[sub_index(r / DB, c / DB)][r % DB][c % DB];
   }
-  // in-place lower-triangular inverse, last column first
-  for (int j = kb - 1; j >= 0; --j) {
-    const T xjj = T(1) / dg[j];
-    for (int r = j + 1 + t; r < kb; r += blockDim.x) tmp[r] = L[j * ldl + r];
+  // inverse X of the factor, X_ii = ri_i^T, the others over L's sub-blocks
+  // (the unused ones past nb are formed from whatever LDS holds and dropped)
+  __syncthreads();
+  Sub<T> *L = s.l;
+  auto X = [&](int i, int j) -> Sub<T> & { return L[sub_index(i, j)]; };
+  if (nb > 1) {
+    // X_10 = -X_11 (L_10 X_00), X_32 = -X_33 (L_32 X_22)
+    acc_t a0 = zero, a1 = zero;
+    sub_mm<T, false, true>(a0, X(1, 0), s.ri[0]);
+    if (nb > 3) sub_mm<T, false, true>(a1, X(3, 2), s.ri[2]);
+    sub_put<T, false>(s.w[0], a0, T(1));
+    sub_put<T, false>(s.w[1], a1, T(1));
     __syncthreads();
-    for (int r = j + 1 + t; r < kb; r += blockDim.x) {
-      T s = T(0);
-      // (inv L22 * l)_r: columns p > j already hold the inverse below the
-      // diagonal, dg[r] (r > j) already holds 1 / L[r][r]
-      for (int p = j + 1; p < r; ++p) s += L[p * ldl + r] * tmp[p];
-      s += dg[r] * tmp[r];
-      L[j * ldl + r] = -xjj * s;
+    a0 = zero;
+    a1 = zero;
+    sub_mm<T, true, false>(a0, s.ri[1], s.w[0]);
+    if (nb > 3) sub_mm<T, true, false>(a1, s.ri[3], s.w[1]);
+    sub_put<T, false>(X(1, 0), a0, T(-1));
+    if (nb > 3) sub_put<T, false>(X(3, 2), a1, T(-1));
+    __syncthreads();
+  }
+  if (nb > 2) {
+    // W = [L_20 L_21; L_30 L_31] [X_00 0; X_10 X_11], then -[X_22 0; X_32 X_33] W
+    acc_t q[4] = {zero, zero, zero, zero};
+    sub_mm<T, false, true>(q[0], X(2, 0), s.ri[0]);
+    sub_mm<T, false, false>(q[0], X(2, 1), X(1, 0));
+    sub_mm<T, false, true>(q[1], X(2, 1), s.ri[1]);
+    if (nb > 3) {
+      sub_mm<T, false, true>(q[2], X(3, 0), s.ri[0]);
+      sub_mm<T, false, false>(q[2], X(3, 1), X(1, 0));
+      sub_mm<T, false, true>(q[3], X(3, 1), s.ri[1]);
     }
     __syncthreads();
-    if (t == 0) dg[j] = xjj;  // dg now holds the inverse diagonal
+    sub_put<T, false>(X(2, 0), q[0], T(1));
+    sub_put<T, false>(X(2, 1), q[1], T(1));
+    if (nb > 3) {
+      sub_put<T, false>(X(3, 0), q[2], T(1));
+      sub_put<T, false>(X(3, 1), q[3], T(1));
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; ++i) q[i] = zero;
+    sub_mm<T, true, false>(q[0], s.ri[2], X(2, 0));
+    sub_mm<T, true, false>(q[1], s.ri[2], X(2, 1));
+    if (nb > 3) {
+      sub_mm<T, false, false>(q[2], X(3, 2), X(2, 0));
+      sub_mm<T, true, false>(q[2], s.ri[3], X(3, 0));
+      sub_mm<T, false, false>(q[3], X(3, 2), X(2, 1));
+      sub_mm<T, true, false>(q[3], s.ri[3], X(3, 1));
+    }
+    __syncthreads();
+    sub_put<T, false>(X(2, 0), q[0], T(-1));
+    sub_put<T, false>(X(2, 1), q[1], T(-1));
+    if (nb > 3) {
+      sub_put<T, false>(X(3, 0), q[2], T(-1));
+      sub_put<T, false>(X(3, 1), q[3], T(-1));
+    }
     __syncthreads();
   }
   T *I = inv + (long)b * sinv;
-  for (int e = t; e < kb * kb; e += blockDim.x) {
-    const int r = e % kb, c = e / kb;
-    T v = T(0);
-    if (r > c)
-      v = L[c * ldl + r];
-    else if (r == c)
-      v = dg[r];
-    I[r + (long)c * kCholNB] = v;
+  for (int c0 = 0; c0 < kCholNB; c0 += 2) {
+    const int c = c0 + ch;
+    if (r < kb && c < kb)
+      I[r + (long)c * kCholNB] =
+          r < c ? T(0)
+                : (r / DB == c / DB ? s.ri[r / DB][c % DB][r % DB]
+                                    : s.l[sub_index(r / DB, c / DB)][r % DB][c % DB]);
   }
 }
 
@@ -103,7 +240,7 @@ template <typename T>
 void potrf_batched(hipStream_t s, int n, T *A, int lda, long sA, int batch,
                    T *inv, long sinv_blk, int *info) {
   const int NB = kCholNB;
-  const size_t smem = sizeof(T) * ((size_t)(NB + 1) * NB + 2 * NB);
+  const size_t smem = sizeof(DiagLds<T>);
   static bool attr_set = false;
   if (!attr_set) {
     MBD_HIP(hipFuncSetAttribute((const void *)k_potrf_diag<T>,
@@ -372,22 +509,29 @@ __device__ void sym3_eig(const double *P, double *w) {
   w[2] = e[2];
 }
 
-// Molecular C6 and the per-point eigenvalues (UTILS.f90:273-278, 288);
-// one thread.
+// Molecular C6 and the per-point eigenvalues (UTILS.f90:273-278, 288): one
+// lane per grid point (a Jacobi iteration is a chain of dependent divisions:
+// 600 us for the 21 points one after another), the sum in the reference's
+// order by one lane.
 __global__ void k_molpol(const double *P, const double *weight, double *eig,
                          double *c6_mol) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  double acc = 0.0;
-  for (int k = 0; k < kNumFreq; ++k) {
+  __shared__ double term[kNumFreq];
+  const int k = threadIdx.x;
+  if (k < kNumFreq) {
     double w[3];
     sym3_eig(P + 9 * k, w);
     eig[3 * k] = w[0];
     eig[3 * k + 1] = w[1];
     eig[3 * k + 2] = w[2];
     const double iso = (w[0] + w[1] + w[2]) / 3.0;
-    if (k >= 1) acc = acc + weight[k] * (iso * iso);
+    term[k] = weight[k] * (iso * iso);
   }
-  *c6_mol = kThreeOverPi * acc;
+  __syncthreads();
+  if (k == 0) {
+    double acc = 0.0;
+    for (int q = 1; q < kNumFreq; ++q) acc = acc + term[q];
+    *c6_mol = kThreeOverPi * acc;
+  }
 }
 
 // Per-atom C6 (UTILS.f90:302-313): alpha layout [k * N + i], k = 0..20.

@@ -21,32 +21,11 @@
 // 16-row block's loads of C together and stores only after every value of the
 // block is formed.
 #include "common.h"
+#include "mfma.h"
 
 namespace mbd {
 
 namespace {
-
-template <typename T>
-struct Mfma;
-template <>
-struct Mfma<double> {
-  using acc_t = v4d;
-  static constexpr bool kSwap = true;
-  // row of accumulator element v held by lane group g = lane / 16
-  __device__ static int row(int g, int v) { return g + 4 * v; }
-  __device__ static acc_t mma(double a, double b, acc_t c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-};
-template <>
-struct Mfma<float> {
-  using acc_t = v4f;
-  static constexpr bool kSwap = true;
-  __device__ static int row(int g, int v) { return 4 * g + v; }
-  __device__ static acc_t mma(float a, float b, acc_t c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-};
 
 constexpr int BM = 128, BN = 128, BK = 16, NT = 256;
 constexpr int PER_T = BM * BK / NT;  // elements of each operand per thread
@@ -133,8 +112,7 @@ __global__ __launch_bounds__(NT, 2) void k_gemm_nt(
       for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-          acc[i][j] = Mfma<T>::kSwap ? Mfma<T>::mma(bf[j], af[i], acc[i][j])
-                                     : Mfma<T>::mma(af[i], bf[j], acc[i][j]);
+          acc[i][j] = Mfma<T>::mma(bf[j], af[i], acc[i][j]);
     }
     if (kt + 1 < nk) sstore(cur ^ 1);
     __syncthreads();
@@ -150,8 +128,8 @@ __global__ __launch_bounds__(NT, 2) void k_gemm_nt(
     for (int j = 0; j < 4; ++j)
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const int r = row0 + wm * 64 + i * 16 + (Mfma<T>::kSwap ? lr : Mfma<T>::row(lk, v));
-        const int c = col0 + wn * 64 + j * 16 + (Mfma<T>::kSwap ? Mfma<T>::row(lk, v) : lr);
+        const int r = row0 + wm * 64 + i * 16 + lr;
+        const int c = col0 + wn * 64 + j * 16 + Mfma<T>::row(lk, v);
         const bool in = r < m && c < n && (!LOWER || r >= c);
         cv[j][v] = (beta != T(0) && in) ? C[r + (long)c * ldc] : T(0);
       }
@@ -169,8 +147,8 @@ __global__ __launch_bounds__(NT, 2) void k_gemm_nt(
     for (int j = 0; j < 4; ++j)
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const int r = row0 + wm * 64 + i * 16 + (Mfma<T>::kSwap ? lr : Mfma<T>::row(lk, v));
-        const int c = col0 + wn * 64 + j * 16 + (Mfma<T>::kSwap ? Mfma<T>::row(lk, v) : lr);
+        const int r = row0 + wm * 64 + i * 16 + lr;
+        const int c = col0 + wn * 64 + j * 16 + Mfma<T>::row(lk, v);
         if (r < m && c < n && (!LOWER || r >= c)) C[r + (long)c * ldc] = cv[j][v];
       }
   }

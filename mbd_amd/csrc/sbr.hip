@@ -32,6 +32,7 @@
 
 #include "common.h"
 #include "kernels.h"
+#include "mfma.h"
 #include "profile.h"
 
 namespace mbd {
@@ -467,31 +468,6 @@ __device__ inline double block_max(double v) {
   for (int i = 1; i < NT / 64; ++i) r = fmax(r, wm[i]);
   __syncthreads();
   return r;
-}
-
-// 1 / sqrt(x) and 1 / x for x > 0 from the hardware estimates refined by two
-// Newton steps each (a few ulp; the correctly rounded square root and
-// division are long dependent chains on the factorisations' critical path)
-__device__ inline double rsq_fast(double x) {
-  double y = __builtin_amdgcn_rsq(x);
-  const double h = 0.5 * x;
-  y = y * fma(-h, y * y, 1.5);
-  y = y * fma(-h, y * y, 1.5);
-  return y;
-}
-__device__ inline double rcp_fast(double x) {
-  double r = __builtin_amdgcn_rcp(x);
-  r = fma(r, fma(-x, r, 1.0), r);
-  r = fma(r, fma(-x, r, 1.0), r);
-  return r;
-}
-
-// The value of lane src, wave-uniform.
-__device__ inline double lane_value(double v, int src) {
-  const unsigned long long u = (unsigned long long)__double_as_longlong(v);
-  const unsigned lo = __builtin_amdgcn_readlane((unsigned)u, src);
-  const unsigned hi = __builtin_amdgcn_readlane((unsigned)(u >> 32), src);
-  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
 // true in the last of `total` workgroups to call it on cnt
