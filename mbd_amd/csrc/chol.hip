@@ -4,15 +4,23 @@
 // alpha_SCS and the molecular tensor (UTILS.f90:479-495), and the C6 sums
 // (UTILS.f90:273-276, 302-315).
 //
-// Right-looking, block size NB: per block column one workgroup per matrix
-// factors the NB x NB diagonal block in LDS and inverts it in place; the panel
-// below becomes A21 * inv(L11)^T and the trailing update A22 -= A21 A21^T, both
-// on the MFMA GEMM.  The inverted diagonal blocks are kept for the triangular
-// solves, which then need only matrix-vector work per block.
+// Right-looking with two block sizes: per block column of NB one workgroup per
+// matrix factors the NB x NB diagonal block in LDS and inverts it; the panel
+// below becomes A21 * inv(L11)^T, and its update A22 -= A21 A21^T reaches only
+// the rest of an outer block of NBO columns; the columns after that are
+// updated once per outer block, both on the MFMA GEMM.  An update of K
+// columns moves 2 sizeof(T) bytes per 2 K flops of the trailing triangle: at
+// K = NB that is as long as the MFMAs take (21 matrices of order 8709 in
+// FP64, trailing updates per factorisation with NBO = 128, 256, 512, 1024:
+// 109, 90, 83, 82 ms; order 12288 in FP32: 133, 115, 107, 106 ms).  The
+// inverted diagonal blocks are kept for the triangular solves, which then
+// need only matrix-vector work per block.
 #include "common.h"
 #include "kernels.h"
 #include "mfma.h"
 #include "profile.h"
+
+#include <algorithm>
 
 namespace mbd {
 
@@ -248,35 +256,45 @@ void potrf_batched(hipStream_t s, int n, T *A, int lda, long sA, int batch,
                                 (int)smem));
     attr_set = true;
   }
-  const int nblk = ceil_div(n, NB);
-  for (int kbk = 0; kbk < nblk; ++kbk) {
-    const int k0 = kbk * NB;
-    const int kb = (n - k0 < NB) ? n - k0 : NB;
-    T *invk = inv + (long)kbk * NB * NB;
-    {
-      ProfScope ps(K_CHOL_DIAG, s, 0.0, batch * (2.0 / 3.0) * kb * (double)kb * kb);
-      hipLaunchKernelGGL((k_potrf_diag<T>), dim3(batch), dim3(256), smem, s, A,
-                         lda, sA, k0, kb, invk, sinv_blk, info);
-      MBD_LAUNCH_CHECK();
+  constexpr int NBO = kCholNBO;
+  for (int o0 = 0; o0 < n; o0 += NBO) {
+    const int o1 = std::min(n, o0 + NBO);  // this outer block's end
+    for (int k0 = o0; k0 < o1; k0 += NB) {
+      const int kb = std::min(NB, n - k0);
+      T *invk = inv + (long)(k0 / NB) * NB * NB;
+      {
+        ProfScope ps(K_CHOL_DIAG, s, 0.0, batch * (2.0 / 3.0) * kb * (double)kb * kb);
+        hipLaunchKernelGGL((k_potrf_diag<T>), dim3(batch), dim3(256), smem, s, A,
+                           lda, sA, k0, kb, invk, sinv_blk, info);
+        MBD_LAUNCH_CHECK();
+      }
+      const int k1 = k0 + kb;
+      const int m2 = n - k1;
+      if (m2 <= 0) break;
+      T *A21 = A + k1 + (long)k0 * lda;
+      // A21 <- A21 inv(L11)^T (in place: one column tile per row tile);
+      // algorithmic work of the triangular solve: m2 kb^2 flops
+      {
+        ProfScope ps(K_CHOL_TRSM, s, 0.0, batch * (double)m2 * kb * kb);
+        gemm_nt(s, false, m2, kb, kb, T(1), A21, lda, sA, invk, NB, sinv_blk,
+                T(0), A21, lda, sA, batch);
+      }
+      // the rest of the outer block's columns, on and below the diagonal
+      const int w2 = o1 - k1;
+      if (w2 > 0) {
+        ProfScope ps(K_CHOL_SYRK, s, 0.0, batch * (double)kb * w2 * (2.0 * m2 - w2 + 1.0));
+        gemm_nt(s, true, m2, w2, kb, T(-1), A21, lda, sA, A21, lda, sA, T(1),
+                A + k1 + (long)k1 * lda, lda, sA, batch);
+      }
     }
-    const int k1 = k0 + kb;
-    const int m2 = n - k1;
+    // trailing A22 -= A21 A21^T on the lower triangle, A21 the outer block's
+    // columns below it: m2 (m2 + 1) (o1 - o0) flops
+    const int m2 = n - o1;
     if (m2 <= 0) break;
-    T *A21 = A + k1 + (long)k0 * lda;
-    T *A22 = A + k1 + (long)k1 * lda;
-    // A21 <- A21 inv(L11)^T (in place: one column tile per row tile);
-    // algorithmic work of the triangular solve: m2 kb^2 flops
-    {
-      ProfScope ps(K_CHOL_TRSM, s, 0.0, batch * (double)m2 * kb * kb);
-      gemm_nt(s, false, m2, kb, kb, T(1), A21, lda, sA, invk, NB, sinv_blk,
-              T(0), A21, lda, sA, batch);
-    }
-    // A22 -= A21 A21^T on the lower triangle: m2 (m2 + 1) kb flops
-    {
-      ProfScope ps(K_CHOL_SYRK, s, 0.0, batch * (double)m2 * (m2 + 1.0) * kb);
-      gemm_nt(s, true, m2, m2, kb, T(-1), A21, lda, sA, A21, lda, sA, T(1), A22,
-              lda, sA, batch);
-    }
+    const T *A21 = A + o1 + (long)o0 * lda;
+    ProfScope ps(K_CHOL_SYRK, s, 0.0, batch * (double)m2 * (m2 + 1.0) * (o1 - o0));
+    gemm_nt(s, true, m2, m2, o1 - o0, T(-1), A21, lda, sA, A21, lda, sA, T(1),
+            A + o1 + (long)o1 * lda, lda, sA, batch);
   }
 }
 template void potrf_batched<double>(hipStream_t, int, double *, int, long,

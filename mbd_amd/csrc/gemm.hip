@@ -5,21 +5,20 @@
 // symmetric rank-k update, and the two-sided Householder SYR2K of the
 // tridiagonalisation.  One 256-thread workgroup owns a 128 x 128 tile of C;
 // its four wave64s each own a 64 x 64 sub-tile held as 4 x 4 MFMA 16x16
-// accumulators.  K is staged through double-buffered LDS in steps of 16 with
-// the next global tile prefetched into registers while the MFMAs run.
+// accumulators (v_mfma_f64_16x16x4_f64, v_mfma_f32_16x16x4_f32).  K is staged
+// through double-buffered LDS in steps of 16 with the next global tile
+// prefetched into registers while the MFMAs run.
 //
-// FP64 uses v_mfma_f64_16x16x4_f64, FP32 uses v_mfma_f32_16x16x4_f32; both
-// take one A and one B element per lane per K=4 step:
-//   A operand: lane l -> A[row l%16][k l/16]
-//   B operand: lane l -> B^T[k l/16][col l%16]
-//   D (FP32):  lane l -> D[row 4*(l/16)+v][col l%16], v = 0..3
-//   D (FP64):  lane l -> D[row (l/16)+4*v][col l%16], v = 0..3
-// Both compute each 16 x 16 block transposed (the B tile as the MFMA's A
-// operand), so the 16 lanes of a group hold 16 consecutive rows of one column
-// of C and every epilogue access covers whole column segments (64 bytes in
-// FP32, 128 in FP64) instead of 16 scattered pieces; the epilogue issues a
-// 16-row block's loads of C together and stores only after every value of the
-// block is formed.
+// Rows are dealt to the 16 x 16 blocks so that a lane's blocks hold V
+// consecutive rows (V = 16 bytes of elements: 4 in FP32, 2 in FP64): block i
+// of a wave covers rows V (16 (i / V) + l) + i % V.  One 16-byte LDS read
+// then feeds V blocks, and with the blocks computed transposed (the B tile as
+// the MFMA's first operand) a lane holds V consecutive rows of each of its
+// columns of C, so global accesses are 16 bytes a lane on both sides.  The
+// matrix cores bound it: 56 TFLOP/s in FP64 and 121 in FP32 over the updates
+// of a 21-matrix Cholesky of order 8709 / 12288 (35 and 73 with 8-byte
+// accesses, branches between the loads and K = 128 updates), against 77 and
+// 155 of the MFMAs alone.
 #include "common.h"
 #include "mfma.h"
 
@@ -28,30 +27,51 @@ namespace mbd {
 namespace {
 
 constexpr int BM = 128, BN = 128, BK = 16, NT = 256;
-constexpr int PER_T = BM * BK / NT;  // elements of each operand per thread
+
+template <typename T>
+struct Vec16;  // 16 bytes of elements, element-aligned
+template <>
+struct Vec16<double> {
+  typedef double t __attribute__((ext_vector_type(2), aligned(8)));
+  static constexpr int n = 2;
+};
+template <>
+struct Vec16<float> {
+  typedef float t __attribute__((ext_vector_type(4), aligned(4)));
+  static constexpr int n = 4;
+};
 
 // Two waves per SIMD (launch bound): the FP64 form otherwise takes 202 VGPRs
 // plus 128 AGPRs, one workgroup per CU, and each workgroup's prologue,
-// barriers and epilogue stall the matrix cores; bounded it fits 214 VGPRs with
-// no spill, two workgroups share a CU, and the FP64 Cholesky and SYR2K updates
-// measured ~20 % faster.
-// ta: op(A)[r][k] = A[k + r lda] instead of A[r + k lda];
+// barriers and epilogue stall the matrix cores.
+// LOWER: the tiles on and below the diagonal of an m x n trapezoid (n <= m).
+// GEN: operands read an element at a time, for fewer than V rows or columns
+// and for ta: op(A)[r][k] = A[k + r lda] instead of A[r + k lda];
 // tb: op(B)[c][k] = B[k + c ldb] instead of B[c + k ldb].
-template <typename T, bool LOWER>
+// No load of the K loop sits under a branch: past the edges of A, B and K the
+// addresses are clamped and the values put right (uniform branch, edge tiles
+// only) before they go to LDS; branches between the loads had made the
+// compiler wait for each one.
+template <typename T, bool LOWER, bool GEN>
 __global__ __launch_bounds__(NT, 2) void k_gemm_nt(
     int m, int n, int k, T alpha, const T *__restrict__ A, int lda, long sA,
     const T *__restrict__ B, int ldb, long sB, T beta, T *__restrict__ C,
     int ldc, long sC, int tiles_n, int ta, int tb) {
+  using vec = typename Vec16<T>::t;
+  constexpr int V = Vec16<T>::n, G = 4 / V;  // row groups of a wave
+  constexpr int NV = BM * BK / V / NT;       // operand vectors per thread
+  constexpr int KS = NT / (BM / V);          // their distance in k
   int tm, tn;
   const int idx = blockIdx.x;
-  if (LOWER) {
+  if (LOWER && idx < tiles_n * (tiles_n + 1) / 2) {
     tm = (int)((sqrt(8.0 * idx + 1.0) - 1.0) * 0.5);
     while ((tm + 1) * (tm + 2) / 2 <= idx) ++tm;
     while (tm * (tm + 1) / 2 > idx) --tm;
     tn = idx - tm * (tm + 1) / 2;
   } else {
-    tm = idx / tiles_n;
-    tn = idx - tm * tiles_n;
+    const int rest = LOWER ? idx - tiles_n * (tiles_n + 1) / 2 : idx;
+    tm = rest / tiles_n + (LOWER ? tiles_n : 0);
+    tn = rest % tiles_n;
   }
   const long bz = blockIdx.z;
   A += bz * sA;
@@ -59,8 +79,8 @@ __global__ __launch_bounds__(NT, 2) void k_gemm_nt(
   C += bz * sC;
   const int row0 = tm * BM, col0 = tn * BN;
 
-  __shared__ T As[2][BK][BM];
-  __shared__ T Bs[2][BK][BN];
+  __shared__ __align__(16) T As[2][BK][BM];
+  __shared__ __align__(16) T Bs[2][BK][BN];
 
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int wm = wave >> 1, wn = wave & 1;
@@ -72,86 +92,158 @@ __global__ __launch_bounds__(NT, 2) void k_gemm_nt(
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = typename Mfma<T>::acc_t{0, 0, 0, 0};
 
-  T ra[PER_T], rb[PER_T];
+  // this thread's vectors: rows sr ... sr + V - 1 of the tiles, columns
+  // sk + KS i; at the edges the last V rows, shifted back into place below
+  const int sr = (t % (BM / V)) * V, sk = t / (BM / V);
+  const int ar = min(row0 + sr, m - V), br = min(col0 + sr, n - V);
+  const bool edge = row0 + BM > m || col0 + BN > n;
+  vec ra[NV], rb[NV];
   auto gload = [&](int k0) {
 #pragma unroll
-    for (int i = 0; i < PER_T; ++i) {
-      const int e = t + NT * i;
-      const int r = e & (BM - 1), kk = e / BM;
-      const int gk = k0 + kk;
-      const int gr = row0 + r, gc = col0 + r;
-      ra[i] = (gr < m && gk < k) ? (ta ? A[gk + (long)gr * lda] : A[gr + (long)gk * lda]) : T(0);
-      rb[i] = (gc < n && gk < k) ? (tb ? B[gk + (long)gc * ldb] : B[gc + (long)gk * ldb]) : T(0);
+    for (int i = 0; i < NV; ++i) {
+      const int kc = min(k0 + sk + KS * i, k - 1);
+      if (GEN) {
+#pragma unroll
+        for (int q = 0; q < V; ++q) {
+          const int r = min(row0 + sr + q, m - 1), c = min(col0 + sr + q, n - 1);
+          ra[i][q] = A[ta ? kc + (long)r * lda : r + (long)kc * lda];
+          rb[i][q] = B[tb ? kc + (long)c * ldb : c + (long)kc * ldb];
+        }
+      } else {
+        ra[i] = *(const vec *)(A + ar + (long)kc * lda);
+        rb[i] = *(const vec *)(B + br + (long)kc * ldb);
+      }
     }
   };
-  auto sstore = [&](int buf) {
+  auto sstore = [&](int buf, int k0) {
+    if (!GEN && edge) {
+      const int da = row0 + sr - ar, db = col0 + sr - br;
 #pragma unroll
-    for (int i = 0; i < PER_T; ++i) {
-      const int e = t + NT * i;
-      const int r = e & (BM - 1), kk = e / BM;
-      As[buf][kk][r] = ra[i];
-      Bs[buf][kk][r] = rb[i];
+      for (int i = 0; i < NV; ++i)
+#pragma unroll
+        for (int q = 0; q < V; ++q)
+#pragma unroll
+          for (int z = V - 1; z > q; --z) {
+            ra[i][q] = da == z - q ? ra[i][z] : ra[i][q];
+            rb[i][q] = db == z - q ? rb[i][z] : rb[i][q];
+          }
+    }
+    if (k0 + BK > k) {
+#pragma unroll
+      for (int i = 0; i < NV; ++i) {
+        const bool in = k0 + sk + KS * i < k;
+#pragma unroll
+        for (int q = 0; q < V; ++q) {
+          ra[i][q] = in ? ra[i][q] : T(0);
+          rb[i][q] = in ? rb[i][q] : T(0);
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      *(vec *)__builtin_assume_aligned(&As[buf][sk + KS * i][sr], 16) = ra[i];
+      *(vec *)__builtin_assume_aligned(&Bs[buf][sk + KS * i][sr], 16) = rb[i];
+    }
+  };
+  // the MFMAs of one staged K tile, the next step's fragments read ahead
+  auto compute = [&](int cur) {
+    vec af[2][G], bf[2][G];
+    auto frag = [&](int b, int kk) {
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        af[b][g] = *(const vec *)__builtin_assume_aligned(&As[cur][kk + lk][wm * 64 + V * (16 * g + lr)], 16);
+        bf[b][g] = *(const vec *)__builtin_assume_aligned(&Bs[cur][kk + lk][wn * 64 + V * (16 * g + lr)], 16);
+      }
+    };
+    frag(0, 0);
+#pragma unroll
+    for (int q = 0; q < BK / 4; ++q) {
+      if (q + 1 < BK / 4) frag((q + 1) & 1, 4 * (q + 1));
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          acc[i][j] = Mfma<T>::mma(bf[q & 1][j / V][j % V], af[q & 1][i / V][i % V], acc[i][j]);
     }
   };
 
   const int nk = (k + BK - 1) / BK;
   gload(0);
-  sstore(0);
+  sstore(0, 0);
   __syncthreads();
   for (int kt = 0; kt < nk; ++kt) {
-    const int cur = kt & 1;
     if (kt + 1 < nk) gload((kt + 1) * BK);
-#pragma unroll
-    for (int kk = 0; kk < BK; kk += 4) {
-      T af[4], bf[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) af[i] = As[cur][kk + lk][wm * 64 + i * 16 + lr];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) bf[j] = Bs[cur][kk + lk][wn * 64 + j * 16 + lr];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          acc[i][j] = Mfma<T>::mma(bf[j], af[i], acc[i][j]);
-    }
-    if (kt + 1 < nk) sstore(cur ^ 1);
+    compute(kt & 1);
+    if (kt + 1 < nk) sstore((kt & 1) ^ 1, (kt + 1) * BK);
     __syncthreads();
   }
 
-  // C in four row blocks of 16 x 64 per wave: a block's loads of C all issue
-  // before its first store (a load after a store to C, which may alias it,
-  // would otherwise wait for the previous element's round trip)
+  // C in G^2 blocks of 16 V rows by 16 V columns per wave: block (g, h) holds
+  // rows crow(g) ... + V - 1 and columns ccol(h, j, v) of the lane
+  auto crow = [&](int g) { return row0 + wm * 64 + V * (16 * g + lr); };
+  auto ccol = [&](int h, int j, int v) {
+    return col0 + wn * 64 + V * (16 * h + Mfma<T>::row(lk, v)) + j;
+  };
+  if (!edge && (!LOWER || tm > tn)) {
+    // a block's C is loaded while the block before it is stored
+    vec cv[2][V][4];
+    auto cload = [&](int b) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    T cv[4][4];
+      for (int j = 0; j < V; ++j)
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+        for (int v = 0; v < 4; ++v)
+          cv[b & 1][j][v] = *(const vec *)(C + crow(b / G) + (long)ccol(b % G, j, v) * ldc);
+    };
+    if (beta != T(0)) cload(0);
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int r = row0 + wm * 64 + i * 16 + lr;
-        const int c = col0 + wn * 64 + j * 16 + Mfma<T>::row(lk, v);
-        const bool in = r < m && c < n && (!LOWER || r >= c);
-        cv[j][v] = (beta != T(0) && in) ? C[r + (long)c * ldc] : T(0);
-      }
-    // every value before the first store, each in its own register (a store
-    // reads its data late, so a register it holds is not reused before it
-    // completes)
+    for (int b = 0; b < G * G; ++b) {
+      __builtin_amdgcn_sched_barrier(0);  // no earlier loads: their registers would spill
+      if (beta != T(0) && b + 1 < G * G) cload(b + 1);
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+      for (int j = 0; j < V; ++j)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        cv[j][v] = alpha * acc[i][j][v] + beta * cv[j][v];
-        asm volatile("" : "+v"(cv[j][v]));  // computed here, not sunk into the stores' branches
-      }
+        for (int v = 0; v < 4; ++v) {
+          vec x;
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int r = row0 + wm * 64 + i * 16 + lr;
-        const int c = col0 + wn * 64 + j * 16 + Mfma<T>::row(lk, v);
-        if (r < m && c < n && (!LOWER || r >= c)) C[r + (long)c * ldc] = cv[j][v];
-      }
+          for (int q = 0; q < V; ++q) {
+            const T p = alpha * acc[V * (b / G) + q][V * (b % G) + j][v];
+            x[q] = beta != T(0) ? p + beta * cv[b & 1][j][v][q] : p;
+          }
+          *(vec *)(C + crow(b / G) + (long)ccol(b % G, j, v) * ldc) = x;
+        }
+    }
+    return;
   }
+  // edge and diagonal tiles, an element at a time: a column group's loads
+  // before its first store (a load after a store to C, which may alias it,
+  // would wait for the previous element's round trip)
+#pragma unroll
+  for (int b = 0; b < G * G; ++b)
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+      __builtin_amdgcn_sched_barrier(0);
+      T x[4][V];
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+#pragma unroll
+        for (int q = 0; q < V; ++q)
+          x[v][q] = C[min(crow(b / G) + q, m - 1) + (long)min(ccol(b % G, j, v), n - 1) * ldc];
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+#pragma unroll
+        for (int q = 0; q < V; ++q) {
+          const T p = alpha * acc[V * (b / G) + q][V * (b % G) + j][v];
+          x[v][q] = beta != T(0) ? p + beta * x[v][q] : p;
+          asm volatile("" : "+v"(x[v][q]));  // computed here, not sunk into the stores' branches
+        }
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+#pragma unroll
+        for (int q = 0; q < V; ++q) {
+          const int r = crow(b / G) + q, c = ccol(b % G, j, v);
+          if (r < m && c < n && (!LOWER || r >= c)) C[r + (long)c * ldc] = x[v][q];
+        }
+    }
 }
 
 // Tall-skinny FP64 update C = alpha (A1 B1^T + A2 B2^T) + beta C for at most
@@ -249,17 +341,12 @@ void launch(hipStream_t s, bool lower, int m, int n, int k, T alpha,
             T beta, T *C, int ldc, long sC, int batch, int ta = 0, int tb = 0) {
   if (m <= 0 || n <= 0 || batch <= 0) return;
   const int tmn = ceil_div(m, BM), tnn = ceil_div(n, BN);
-  if (lower) {
-    // symmetric update: m == n, only tiles with row tile >= column tile
-    const int tiles = tmn * (tmn + 1) / 2;
-    dim3 grid(tiles, 1, batch);
-    hipLaunchKernelGGL((k_gemm_nt<T, true>), grid, dim3(NT), 0, s, m, n, k,
-                       alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, tnn, ta, tb);
-  } else {
-    dim3 grid(tmn * tnn, 1, batch);
-    hipLaunchKernelGGL((k_gemm_nt<T, false>), grid, dim3(NT), 0, s, m, n, k,
-                       alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, tnn, ta, tb);
-  }
+  const bool gen = ta || tb || m < Vec16<T>::n || n < Vec16<T>::n;
+  const dim3 grid(lower ? tnn * (tnn + 1) / 2 + (tmn - tnn) * tnn : tmn * tnn, 1, batch);
+  auto *f = lower ? (gen ? k_gemm_nt<T, true, true> : k_gemm_nt<T, true, false>)
+                  : (gen ? k_gemm_nt<T, false, true> : k_gemm_nt<T, false, false>);
+  hipLaunchKernelGGL(f, grid, dim3(NT), 0, s, m, n, k, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc,
+                     sC, tnn, ta, tb);
   MBD_LAUNCH_CHECK();
 }
 

@@ -6,6 +6,7 @@
 namespace mbd {
 
 constexpr int kCholNB = 128;   // Cholesky block size (diagonal block in LDS)
+constexpr int kCholNBO = 512;  // columns factored between two updates of the whole trailing triangle
 constexpr int kTrdNB = 64;     // Householder panel width
 constexpr int kTrdTail = 128;  // trailing order reduced by one workgroup
 constexpr int kTrdTile = 128;  // tile edge of the lower-triangle symv

@@ -29,3 +29,19 @@ def test_cholesky_reports_each_pivot(at):
     A[at - 1, at - 1] = -1.0
     _, info = engine.device_cholesky(A)
     assert info[0] == at
+
+
+# fewer rows or columns than a 16-byte vector, one short of and one past a
+# vector and a tile, odd leading dimensions, K remainders
+@pytest.mark.parametrize("fp32", [False, True])
+@pytest.mark.parametrize("m,n,k", [(1, 130, 5), (3, 200, 17), (130, 3, 15), (127, 129, 16),
+                                   (129, 127, 31), (131, 133, 1), (257, 255, 47), (256, 128, 64)])
+def test_gemm_edges(m, n, k, fp32):
+    from mbd_amd import engine
+    rng = np.random.default_rng(m * 1000 + n)
+    t = np.float32 if fp32 else np.float64
+    A, B, C = (rng.standard_normal(s).astype(t).astype(np.float64) for s in ((m, k), (n, k), (m, n)))
+    got = engine.device_gemm_nt(A, B, C, alpha=-1.0, beta_=1.0, fp32=fp32)
+    # k + 1 roundings of sums no larger than |A| |B|^T + |C|
+    eps = 6e-8 if fp32 else 1.2e-16
+    assert np.all(np.abs(got - (C - A @ B.T)) <= 2 * (k + 2) * eps * (np.abs(A) @ np.abs(B).T + np.abs(C)))
