@@ -22,6 +22,7 @@
 #include "kernels.h"
 #include "net.h"
 #include "batch.h"
+#include "logdet.h"
 #include "pcg.h"
 #include "profile.h"
 #include "refine.h"
@@ -237,6 +238,13 @@ struct mbd_handle {
   hipEvent_t sbr_fork = nullptr, sbr_join = nullptr;
   int eig_used = 1;
   int eig_flag = 0;
+  // log-determinant energy: shifted matrices and their inverted diagonal
+  // blocks share A64 / inv64; bounds and sums on the device and the host
+  DevBuf<double> ldHi, ldG;
+  DevBuf<int> ldInfo;
+  // result of the last run_energy
+  double e_val = 0.0;
+  int n_neg = 0;
   // instrumentation
   bool prof_on = false;
   Profiler prof;
@@ -573,6 +581,89 @@ void run_scs(mbd_handle *h, int mode, mbd_diag *d) {
   }
 }
 
+// The energy by log-determinants rather than eigenvalues: unless
+// MBD_EIG_METHOD asks for one of the eigenvalue methods.
+bool use_logdet(long nm) { return !getenv("MBD_EIG_METHOD") && nm <= kLdMaxOrder; }
+
+// E_MBD of the coupled matrix h->C (order nm, lower triangle) by
+// log-determinants into h->e_val.  false, with nothing decided, when C has an
+// eigenvalue below a thirtieth of the smallest omega^2 (negative ones among
+// them), a value that is not finite, or no room for one shifted matrix.
+bool energy_by_logdet(mbd_handle *h, long nm) {
+  hipStream_t s = h->stream;
+  const int N = h->N, n = (int)nm;
+  const int nblk = ceil_div(nm, 64), nd_max = kLdMaxNodes + 1;
+  const long sA = nm * nm, sinv = (long)ceil_div(nm, kCholNB) * kCholNB * kCholNB;
+  const size_t one = 8 * (size_t)(sA + sinv);
+  if (mem_budget() < one) return false;
+  h->ldHi.ensure(nblk);
+  h->ldG.ensure(nd_max);
+  h->ldInfo.ensure(nd_max);
+  std::vector<double> hi(nblk), om(N);
+  ld_bounds(s, n, h->C.p, nm, sA, 1, h->ldHi.p);
+  MBD_HIP(hipMemcpyAsync(hi.data(), h->ldHi.p, 8 * nblk, hipMemcpyDeviceToHost, s));
+  MBD_HIP(hipMemcpyAsync(om.data(), h->om_at.p, 8 * N, hipMemcpyDeviceToHost, s));
+  MBD_HIP(hipStreamSynchronize(s));
+  double top = 0.0, w2min = 1e300;
+  for (double v : hi) {
+    if (!std::isfinite(v)) return false;
+    top = std::max(top, v);
+  }
+  for (double w : om) {
+    if (!std::isfinite(w)) return false;
+    w2min = std::min(w2min, w * w);
+    top = std::max(top, w * w);
+  }
+  // the smallest eigenvalue is 0.38 (graphene) to 0.97 (water) of the
+  // smallest omega^2 on the reference's examples and the benchmark's systems
+  for (double frac : {0.3, 0.03}) {
+    LdNodes nd;
+    if (!ld_nodes(frac * w2min, top, nd)) return false;
+    const int all = nd.n + 1;
+    // matrices per pass: the SCS stage's memory budget, and what is free
+    int fit = (int)std::min<size_t>(mem_budget() / one, all);
+    if (h->A64.n < (size_t)fit * sA || h->inv64.n < (size_t)fit * sinv) {
+      size_t freeb = 0, total = 0;
+      MBD_HIP(hipMemGetInfo(&freeb, &total));
+      freeb = freeb / 10 * 9 + 8 * (h->A64.n + h->inv64.n);
+      fit = (int)std::min<size_t>(fit, freeb / one);
+      if (fit < 1) return false;
+      try {
+        h->A64.ensure((size_t)fit * sA);
+        h->inv64.ensure((size_t)fit * sinv);
+      } catch (const HipError &e) {
+        if (e.err != hipErrorOutOfMemory) throw;
+        (void)hipGetLastError();
+        return false;
+      }
+    }
+    batch_zero(s, h->ldInfo.p, all);
+    // the proof's shift is in the first pass, and a failure there ends it
+    std::vector<double> g(all);
+    std::vector<int> info(all, 0);
+    bool ok = true;
+    for (int end = all; end > 0 && ok;) {
+      const int nb = std::min(fit, end), b0 = end - nb;
+      end = b0;
+      ld_shift(s, n, h->C.p, nm, sA, 1, nd, b0, nb, h->A64.p, sA);
+      potrf_batched<double>(s, n, h->A64.p, n, sA, nb, h->inv64.p, sinv, h->ldInfo.p + b0, true);
+      ld_sums(s, n, h->A64.p, sA, 1, nd, b0, nb, h->om_at.p, N, h->ncell, h->ldG.p + b0);
+      MBD_HIP(hipMemcpyAsync(g.data() + b0, h->ldG.p + b0, 8 * nb, hipMemcpyDeviceToHost, s));
+      MBD_HIP(hipMemcpyAsync(info.data() + b0, h->ldInfo.p + b0, 4 * nb, hipMemcpyDeviceToHost, s));
+      MBD_HIP(hipStreamSynchronize(s));
+      for (int b = b0; b < b0 + nb; ++b) ok = ok && info[b] == 0;
+    }
+    if (!ok) continue;
+    double e = 0.0;
+    for (int b = 0; b < nd.n; ++b) e += nd.w[b] * g[b];
+    if (!std::isfinite(e)) return false;
+    h->e_val = e / h->ncell;
+    h->n_neg = 0;
+    return true;
+  }
+  return false;
+}
+
 // E_MBD from device alpha_eff / c6_eff.
 void run_energy(mbd_handle *h, const double *alpha_eff_d, const double *c6_d,
                 mbd_diag *d) {
@@ -586,6 +677,12 @@ void run_energy(mbd_handle *h, const double *alpha_eff_d, const double *c6_d,
   cfdm_build(s, N, h->ncell, h->xyz.p, h->cell.p, h->lat_d.p, h->nimg_cfdm,
              h->nimg_cfdm / 2, h->img_cfdm.p, h->rc_cfdm / kBohr, h->beta,
              alpha_eff_d, h->om_at.p, h->reff.p, h->C.p, nm, false);
+  if (d) {
+    d->info_eig = 0;
+    for (int k = 0; k < 3; ++k) d->supercell[k] = h->supercell[k];
+  }
+  h->eig_flag = 0;
+  if (use_logdet(nm) && energy_by_logdet(h, nm)) return;
   TrdWork wk;
   h->VW.ensure((size_t)nm * 3 * kTrdNB);
   h->tau.ensure(nm);
@@ -612,7 +709,6 @@ void run_energy(mbd_handle *h, const double *alpha_eff_d, const double *c6_d,
   wk.pb = h->pb.p;
   const int method = eig_method((int)nm);
   h->eig_used = method;
-  h->eig_flag = 0;
   SbrWork sw{};
   if (method == 2) {
     const SbrSizes z = sbr_sizes((int)nm);
@@ -714,10 +810,9 @@ void run_energy(mbd_handle *h, const double *alpha_eff_d, const double *c6_d,
   h->E.ensure(4);
   h->nneg.ensure(1);
   energy(s, (int)nm, h->lam.p, N, h->om_at.p, h->ncell, h->E.p, h->nneg.p);
-  if (d) {
-    d->info_eig = 0;
-    for (int k = 0; k < 3; ++k) d->supercell[k] = h->supercell[k];
-  }
+  MBD_HIP(hipMemcpyAsync(&h->e_val, h->E.p, sizeof(double), hipMemcpyDeviceToHost, s));
+  MBD_HIP(hipMemcpyAsync(&h->n_neg, h->nneg.p, sizeof(int), hipMemcpyDeviceToHost, s));
+  MBD_HIP(hipStreamSynchronize(s));
 }
 
 void fetch(mbd_handle *h, double *dst, const double *src, size_t count) {
@@ -833,6 +928,9 @@ int mbd_destroy(mbd_handle *h) {
   DevBuf<int> *sibufs[] = {&h->sbrCnt, &h->sbrMcnt, &h->sbrProg, &h->sbrFlag, &h->sbrCq};
   for (auto *b : sibufs) b->release();
   h->sbrMail.release();
+  h->ldHi.release();
+  h->ldG.release();
+  h->ldInfo.release();
   batch_release(h);
   if (h->trd_exec) (void)hipGraphExecDestroy(h->trd_exec);
   if (h->stream2) (void)hipStreamSynchronize(h->stream2);
@@ -1050,20 +1148,16 @@ int mbd_energy(mbd_handle *h, const double *alpha_eff, const double *c6_eff, dou
     run_energy(h, h->ext_alpha.p, h->ext_c6.p, d);
     tm.stop(h->stream);
     const double ms = tm.ms();
-    double E[4];
-    int nn = 0;
-    fetch(h, E, h->E.p, 3);
-    MBD_HIP(hipMemcpyAsync(&nn, h->nneg.p, sizeof(int), hipMemcpyDeviceToHost, h->stream));
     fetch(h, omega, h->om_at.p, N);
     fetch(h, reff, h->reff.p, N);
     MBD_HIP(hipStreamSynchronize(h->stream));
-    *e_mbd = E[0];
+    *e_mbd = h->e_val;
     if (h->eig_flag) {
       if (d) d->info_eig = 1;
       return MBD_ERR_EIG;
     }
     if (d) {
-      d->n_negative = nn;
+      d->n_negative = h->n_neg;
       d->t_mbd_ms = ms;
       d->t_total_ms = ms;
     }
@@ -1090,18 +1184,14 @@ int mbd_run(mbd_handle *h, int mode, double *e_mbd, double *alpha_eff, double *c
     t_mbd.stop(h->stream);
     t_all.stop(h->stream);
     const double ms_all = t_all.ms(), ms_mbd = t_mbd.ms();
-    double E[4];
-    int nn = 0;
-    fetch(h, E, h->E.p, 3);
-    MBD_HIP(hipMemcpyAsync(&nn, h->nneg.p, sizeof(int), hipMemcpyDeviceToHost, h->stream));
     fetch_scs_outputs(h, alpha_eff, coupled_pol, molpol_eig, c6_eff, c6_mol);
-    *e_mbd = E[0];
+    *e_mbd = h->e_val;
     if (h->eig_flag) {
       if (d) d->info_eig = 1;
       return MBD_ERR_EIG;
     }
     if (d) {
-      d->n_negative = nn;
+      d->n_negative = h->n_neg;
       d->t_total_ms = ms_all;
       d->t_mbd_ms = ms_mbd;
       d->t_scs_ms = ms_all - ms_mbd;

@@ -246,7 +246,7 @@ __global__ __launch_bounds__(256) void k_potrf_diag(T *A, int lda, long sA,
 
 template <typename T>
 void potrf_batched(hipStream_t s, int n, T *A, int lda, long sA, int batch,
-                   T *inv, long sinv_blk, int *info) {
+                   T *inv, long sinv_blk, int *info, bool energy) {
   const int NB = kCholNB;
   const size_t smem = sizeof(DiagLds<T>);
   static bool attr_set = false;
@@ -263,7 +263,7 @@ void potrf_batched(hipStream_t s, int n, T *A, int lda, long sA, int batch,
       const int kb = std::min(NB, n - k0);
       T *invk = inv + (long)(k0 / NB) * NB * NB;
       {
-        ProfScope ps(K_CHOL_DIAG, s, 0.0, batch * (2.0 / 3.0) * kb * (double)kb * kb);
+        ProfScope ps(energy ? K_LD_DIAG : K_CHOL_DIAG, s, 0.0, batch * (2.0 / 3.0) * kb * (double)kb * kb);
         hipLaunchKernelGGL((k_potrf_diag<T>), dim3(batch), dim3(256), smem, s, A,
                            lda, sA, k0, kb, invk, sinv_blk, info);
         MBD_LAUNCH_CHECK();
@@ -275,14 +275,14 @@ void potrf_batched(hipStream_t s, int n, T *A, int lda, long sA, int batch,
       // A21 <- A21 inv(L11)^T (in place: one column tile per row tile);
       // algorithmic work of the triangular solve: m2 kb^2 flops
       {
-        ProfScope ps(K_CHOL_TRSM, s, 0.0, batch * (double)m2 * kb * kb);
+        ProfScope ps(energy ? K_LD_TRSM : K_CHOL_TRSM, s, 0.0, batch * (double)m2 * kb * kb);
         gemm_nt(s, false, m2, kb, kb, T(1), A21, lda, sA, invk, NB, sinv_blk,
                 T(0), A21, lda, sA, batch);
       }
       // the rest of the outer block's columns, on and below the diagonal
       const int w2 = o1 - k1;
       if (w2 > 0) {
-        ProfScope ps(K_CHOL_SYRK, s, 0.0, batch * (double)kb * w2 * (2.0 * m2 - w2 + 1.0));
+        ProfScope ps(energy ? K_LD_SYRK : K_CHOL_SYRK, s, 0.0, batch * (double)kb * w2 * (2.0 * m2 - w2 + 1.0));
         gemm_nt(s, true, m2, w2, kb, T(-1), A21, lda, sA, A21, lda, sA, T(1),
                 A + k1 + (long)k1 * lda, lda, sA, batch);
       }
@@ -292,15 +292,15 @@ void potrf_batched(hipStream_t s, int n, T *A, int lda, long sA, int batch,
     const int m2 = n - o1;
     if (m2 <= 0) break;
     const T *A21 = A + o1 + (long)o0 * lda;
-    ProfScope ps(K_CHOL_SYRK, s, 0.0, batch * (double)m2 * (m2 + 1.0) * (o1 - o0));
+    ProfScope ps(energy ? K_LD_SYRK : K_CHOL_SYRK, s, 0.0, batch * (double)m2 * (m2 + 1.0) * (o1 - o0));
     gemm_nt(s, true, m2, m2, o1 - o0, T(-1), A21, lda, sA, A21, lda, sA, T(1),
             A + o1 + (long)o1 * lda, lda, sA, batch);
   }
 }
 template void potrf_batched<double>(hipStream_t, int, double *, int, long,
-                                    int, double *, long, int *);
+                                    int, double *, long, int *, bool);
 template void potrf_batched<float>(hipStream_t, int, float *, int, long, int,
-                                   float *, long, int *);
+                                   float *, long, int *, bool);
 
 // ---------------------------------------------------------------------------
 // Triangular solves with NRHS = 3, X column-major n x 3 (ldx) per matrix,

@@ -32,7 +32,7 @@ void cfdm_build(hipStream_t s, int N, int ncell, const double *xyz,
 // chol.hip
 template <typename T>
 void potrf_batched(hipStream_t s, int n, T *A, int lda, long sA, int batch,
-                   T *inv, long sinv_blk, int *info);
+                   T *inv, long sinv_blk, int *info, bool energy = false);
 template <typename T>
 void potrs3_batched(hipStream_t s, int n, const T *L, int lda, long sA,
                     int batch, const T *inv, long sinv_blk, double *X, int ldx,

@@ -1,0 +1,34 @@
+// E_MBD from Cholesky log-determinants (logdet.hip).
+#pragma once
+
+#include <vector>
+
+#include "common.h"
+
+namespace mbd {
+
+// Quadrature nodes of the energy: E = sum_b w[b] (ln det(C + t[b]) - ln det(D + t[b])) / cells with
+// D = diag(omega^2); one more entry, t = -lo without a weight, whose factorisation proves that
+// every eigenvalue of C lies above lo.
+constexpr int kLdMaxNodes = 20;
+constexpr long kLdMaxOrder = 16384;
+struct LdNodes {
+  int n = 0;  // nodes; entry n is the proof's shift
+  double t[kLdMaxNodes + 1];
+  double w[kLdMaxNodes + 1];
+};
+// Nodes for eigenvalues in [lo, hi]; false if more than kLdMaxNodes would be needed.
+bool ld_nodes(double lo, double hi, LdNodes &nd);
+
+// Gershgorin discs of `batch` symmetric n x n matrices (lower triangle read): hi[b nblk + i] is the
+// largest right end over rows 64 i ... 64 i + 63 of matrix b, nblk = ceil(n / 64).
+void ld_bounds(hipStream_t s, int n, const double *H, long ld, long sH, int batch, double *hi);
+// Lower triangle of H_r + t[b0 + b] I as matrix r nb + b of A (leading dimension n), r < batch, b < nb.
+void ld_shift(hipStream_t s, int n, const double *H, long ld, long sH, int batch, const LdNodes &nd,
+              int b0, int nb, double *A, long sA);
+// g[m] = ln det(A_m) - ln det(D + t) from the factor's diagonal, for m < batch nb; row r of a matrix
+// belongs to atom (r % (3 N cells)) / (3 cells).
+void ld_sums(hipStream_t s, int n, const double *L, long sA, int batch, const LdNodes &nd, int b0,
+             int nb, const double *omega, int N, int cells, double *g);
+
+}  // namespace mbd

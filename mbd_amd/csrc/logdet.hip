@@ -1,0 +1,208 @@
+// E_MBD without eigenvalues (the sum 1/2 sum sqrt(lambda) - 1/2 sum omega of
+// UTILS.f90:835-877, for a matrix whose eigenvalues are all positive).
+//
+// With D = diag(omega^2), sqrt(x) - sqrt(d) = 1/pi int_0^inf ln((x + y^2) /
+// (d + y^2)) dy, so
+//   E = 1/(2 pi) int_0^inf [ln det(C + y^2) - ln det(D + y^2)] dy,
+// and a Cholesky factor gives each log-determinant.  With all eigenvalues (and
+// omega^2) in [lo, hi], y = sqrt(lo) sc(u | k') with k^2 = lo / hi turns the
+// integrand into an even periodic function of u, analytic for |Im u| < K, and
+// the midpoint rule with N points on [0, K'] converges as
+// exp(-2 pi K N / K') = exp(-2 pi^2 N / ln(16 hi / lo)) (the substitution of
+// Hale, Higham and Trefethen for contour integrals of matrix functions; SIAM
+// J. Numer. Anal. 46, 2008).  8 to 11 factorisations of FP64 accuracy replace
+// the reduction to tridiagonal form and the bisection: (N + 1) n^3 / 3 flops
+// on the GEMM against 4 n^3 / 3 in panels, a bulge chase and Sturm counts
+// bound by latency.  hi is Gershgorin's bound; lo is a guess that one more
+// Cholesky factorisation, of C - lo I, proves (it exists exactly if every
+// eigenvalue exceeds lo); the caller takes the eigenvalue path when it does
+// not exist.
+#include <algorithm>
+#include <cmath>
+#include <vector>
+
+#include "common.h"
+#include "logdet.h"
+
+namespace mbd {
+
+namespace {
+
+double agm(double a, double b) {
+  for (int i = 0; i < 40 && std::fabs(a - b) > 1e-16 * a; ++i) {
+    const double t = 0.5 * (a + b);
+    b = std::sqrt(a * b);
+    a = t;
+  }
+  return 0.5 * (a + b);
+}
+
+// sn, cn, dn of u with complementary modulus kc, by the arithmetic-geometric
+// mean (Abramowitz and Stegun 16.4)
+void jacobi(double u, double kc, double &sn, double &cn, double &dn) {
+  constexpr int M = 16;
+  double a[M + 1], c[M + 1], b = kc;
+  a[0] = 1.0;
+  c[0] = std::sqrt((1.0 - kc) * (1.0 + kc));
+  int n = 0;
+  while (n < M && c[n] > 1e-17 * a[n]) {
+    a[n + 1] = 0.5 * (a[n] + b);
+    c[n + 1] = 0.5 * (a[n] - b);
+    b = std::sqrt(a[n] * b);
+    ++n;
+  }
+  double phi = std::ldexp(a[n] * u, n);
+  for (; n > 0; --n) phi = 0.5 * (phi + std::asin(c[n] / a[n] * std::sin(phi)));
+  sn = std::sin(phi);
+  cn = std::cos(phi);
+  dn = std::sqrt(cn * cn + kc * kc * sn * sn);
+}
+
+constexpr double kLdEps = 1e-14;  // the midpoint rule's relative error
+constexpr int GB = 64;            // rows of a bounds workgroup
+constexpr int GW = 8;             // its waves
+constexpr int SC = 8;             // columns of a shift workgroup
+
+}  // namespace
+
+bool ld_nodes(double lo, double hi, LdNodes &nd) {
+  if (!(lo > 0.0) || !(hi > lo) || !std::isfinite(hi)) return false;
+  const double pi = 3.14159265358979323846;
+  const double kc = std::sqrt(lo / hi);  // k: the complementary modulus of k'
+  const double Kp = pi / (2.0 * agm(1.0, kc));
+  const double K = pi / (2.0 * agm(1.0, std::sqrt((1.0 - kc) * (1.0 + kc))));
+  nd.n = std::max(2, (int)std::ceil(std::log(2.0 / kLdEps) * Kp / (2.0 * pi * K)));
+  if (nd.n > kLdMaxNodes) return false;
+  const double h = Kp / nd.n;
+  for (int b = 0; b < nd.n; ++b) {
+    double sn, cn, dn;
+    jacobi((b + 0.5) * h, kc, sn, cn, dn);
+    nd.t[b] = lo * (sn / cn) * (sn / cn);
+    nd.w[b] = h * std::sqrt(lo) * dn / (cn * cn) / (2.0 * pi);
+  }
+  nd.t[nd.n] = -lo;
+  nd.w[nd.n] = 0.0;
+  return true;
+}
+
+// Row sums of |H| for 64 rows: the part left of the diagonal block with lanes
+// on rows, the diagonal block, and the columns below it (the rows' part right
+// of the diagonal) with lanes down a column; every partial has one owner and
+// a fixed order.  Each element off the diagonal blocks is read twice; HBM
+// bound (0.4 ms at n = 12288).
+__global__ __launch_bounds__(64 * GW) void k_ld_bounds(int n, const double *__restrict__ H, long ld,
+                                                       long sH, double *__restrict__ hi) {
+  __shared__ double part[GW][GB], diag[GB], below[GB];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int r0 = blockIdx.x * GB, nr = min(GB, n - r0);
+  const double *M = H + (long)blockIdx.y * sH;
+  const int row = r0 + min(lane, nr - 1);
+  double s = 0.0;
+  for (int c = w; c < r0; c += 8 * GW) {
+    double v[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) v[q] = M[row + (long)min(c + q * GW, r0 - 1) * ld];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) s += (c + q * GW < r0) ? fabs(v[q]) : 0.0;
+  }
+  // the diagonal block: row `lane`, its columns dealt to the waves
+  for (int c = w; c < nr; c += GW) {
+    const int a = max(lane, c), b = min(lane, c);
+    const double v = M[r0 + min(a, nr - 1) + (long)(r0 + b) * ld];
+    s += (lane < nr && c != lane) ? fabs(v) : 0.0;
+    if (c == lane) diag[lane] = v;
+  }
+  part[w][lane] = s;
+  // columns r0 + w, r0 + w + GW, ... below the diagonal block
+  double q[GB / GW];
+#pragma unroll
+  for (int i = 0; i < GB / GW; ++i) q[i] = 0.0;
+  for (int r = r0 + GB + lane; r < n; r += 64) {
+#pragma unroll
+    for (int i = 0; i < GB / GW; ++i) q[i] += fabs(M[r + (long)min(r0 + w + i * GW, n - 1) * ld]);
+  }
+#pragma unroll
+  for (int i = 0; i < GB / GW; ++i) {
+    for (int o = 32; o > 0; o >>= 1) q[i] += __shfl_xor(q[i], o, 64);
+    if (lane == 0) below[w + i * GW] = q[i];
+  }
+  __syncthreads();
+  if (w == 0) {
+    double t = below[lane];
+    for (int i = 0; i < GW; ++i) t += part[i][lane];
+    t += lane < nr ? diag[lane] : 0.0;
+    // a NaN row must not be lost in the maximum
+    bool bad = lane < nr && !(t < 1e300);
+    double m = lane < nr ? t : -1e300;
+    for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o, 64));
+    if (__any(bad)) m = INFINITY;
+    if (lane == 0) hi[(long)blockIdx.y * gridDim.x + blockIdx.x] = m;
+  }
+}
+
+void ld_bounds(hipStream_t s, int n, const double *H, long ld, long sH, int batch, double *hi) {
+  hipLaunchKernelGGL(k_ld_bounds, dim3(ceil_div(n, GB), batch), dim3(64 * GW), 0, s, n, H, ld, sH, hi);
+  MBD_LAUNCH_CHECK();
+}
+
+// Each element of the lower triangle read once and written once per node.
+__global__ __launch_bounds__(256) void k_ld_shift(int n, const double *__restrict__ H, long ld,
+                                                  long sH, LdNodes nd, int b0, int nb,
+                                                  double *__restrict__ A, long sA) {
+  const int r = blockIdx.x * 256 + threadIdx.x, c0 = blockIdx.y * SC;
+  if (blockIdx.x * 256 + 255 < c0 || r >= n) return;
+  const double *M = H + (long)blockIdx.z * sH;
+  double v[SC];
+#pragma unroll
+  for (int i = 0; i < SC; ++i) v[i] = M[r + (long)min(c0 + i, n - 1) * ld];
+  double *out = A + (long)blockIdx.z * nb * sA + r;
+  for (int b = 0; b < nb; ++b, out += sA) {
+    const double t = nd.t[b0 + b];
+#pragma unroll
+    for (int i = 0; i < SC; ++i) {
+      const int c = c0 + i;
+      if (c <= r) out[(long)c * n] = r == c ? v[i] + t : v[i];
+    }
+  }
+}
+
+void ld_shift(hipStream_t s, int n, const double *H, long ld, long sH, int batch, const LdNodes &nd,
+              int b0, int nb, double *A, long sA) {
+  hipLaunchKernelGGL(k_ld_shift, dim3(ceil_div(n, 256), ceil_div(n, SC), batch), dim3(256), 0, s, n, H,
+                     ld, sH, nd, b0, nb, A, sA);
+  MBD_LAUNCH_CHECK();
+}
+
+// One workgroup per matrix: sum over the rows of ln(L_jj^2 / (omega_j^2 + t)),
+// terms near zero, in a fixed order.
+__global__ __launch_bounds__(1024) void k_ld_sums(int n, const double *__restrict__ L, long sA,
+                                                  LdNodes nd, int b0, int nb,
+                                                  const double *__restrict__ omega, int N, int cells,
+                                                  double *__restrict__ g) {
+  __shared__ double red[16];
+  const int m = blockIdx.x, t = threadIdx.x;
+  const double shift = nd.t[b0 + m % nb];
+  const double *M = L + (long)m * sA;
+  double s = 0.0;
+  for (int j = t; j < n; j += 1024) {
+    const double l = M[j + (long)j * n], w = omega[(j % (3 * N * cells)) / (3 * cells)];
+    s += log(l * l / (w * w + shift));
+  }
+  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+  if ((t & 63) == 0) red[t >> 6] = s;
+  __syncthreads();
+  if (t == 0) {
+    double a = 0.0;
+    for (int i = 0; i < 16; ++i) a += red[i];
+    g[m] = a;
+  }
+}
+
+void ld_sums(hipStream_t s, int n, const double *L, long sA, int batch, const LdNodes &nd, int b0,
+             int nb, const double *omega, int N, int cells, double *g) {
+  hipLaunchKernelGGL(k_ld_sums, dim3(batch * nb), dim3(1024), 0, s, n, L, sA, nd, b0, nb, omega, N,
+                     cells, g);
+  MBD_LAUNCH_CHECK();
+}
+
+}  // namespace mbd

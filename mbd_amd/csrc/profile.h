@@ -32,6 +32,9 @@ enum KernelClass {
   K_SBR_SYMM,
   K_SBR_CHASE,
   K_LU,
+  K_LD_DIAG,
+  K_LD_TRSM,
+  K_LD_SYRK,
   K_NUM_CLASSES
 };
 

@@ -10,7 +10,7 @@ const char *kernel_class_name(int cls) {
       "scs_build", "chol_diag", "chol_trsm_gemm", "chol_syrk_gemm", "trsv",
       "refine_residual", "cfdm_build", "trd_colupd", "trd_symv", "trd_wcol", "trd_syr2k_gemm",
       "trd_tail", "bisect", "pcg_symv", "pcg_small", "net_infer", "sbr_panel_qr", "sbr_symm", "sbr_chase",
-      "lu_fallback"};
+      "lu_fallback", "logdet_diag", "logdet_trsm_gemm", "logdet_syrk_gemm"};
   return (cls >= 0 && cls < K_NUM_CLASSES) ? names[cls] : "";
 }
 

@@ -1,0 +1,96 @@
+"""The energy by log-determinants against the eigenvalue methods
+(MBD_EIG_METHOD), at the edges of its kernels' blocks and over every branch:
+the first and the second guess of the spectrum's lower end, and matrices that
+have eigenvalues not above zero and must take the eigenvalue path."""
+import numpy as np
+import pytest
+
+from mbd_amd import engine, generators
+from mbd_amd.io import Geometry, Settings
+
+pytestmark = pytest.mark.gpu
+
+
+def _both(geo, st, monkeypatch, method="1"):
+    with engine.MbdEngine(0) as eng:
+        eng.set_geometry(geo, st)
+        a, _, _, c, _, _ = eng.scs("fp64")
+        monkeypatch.setenv("MBD_EIG_METHOD", method)
+        want, om, _, dw = eng.energy(a, c)
+        monkeypatch.delenv("MBD_EIG_METHOD")
+        eng.profile_enable(True)
+        got, _, _, dg = eng.energy(a, c)
+        prof = eng.profile_read()
+    cells = int(np.prod(dw["supercell"]))
+    # both sum 3 N cells square roots of eigenvalues with a backward error of
+    # about the order times eps each, divided by the number of cells
+    tol = 2.2e-16 * 3 * geo.n_atoms * cells * 1.5 * np.sum(om)
+    assert dg["n_negative"] == dw["n_negative"]
+    assert dg["supercell"] == dw["supercell"]
+    return got, want, tol, dg, prof
+
+
+def _spread(n, seed, gap=2.2):
+    """n atoms on a jittered cubic grid: physical at any n."""
+    rng = np.random.default_rng(seed)
+    m = int(np.ceil(n ** (1 / 3)))
+    g = np.stack(np.meshgrid(*[np.arange(m)] * 3, indexing="ij"), -1).reshape(-1, 3)[:n]
+    xyz = gap * g + rng.uniform(-0.2, 0.2, (n, 3))
+    return Geometry(list(rng.choice(["C", "H", "N", "O"], n)), xyz, rng.uniform(0.6, 0.95, n), None)
+
+
+# orders 3, 63, 66, 126, 129, 192, 195, 387, 771: one short of and one past the
+# bounds' 64-row and the factorisation's 128-row blocks
+@pytest.mark.parametrize("n", [1, 21, 22, 42, 43, 64, 65, 129, 257])
+def test_matches_eigenvalues(n, monkeypatch):
+    got, want, tol, _, prof = _both(_spread(n, n), Settings(), monkeypatch)
+    assert prof["logdet_diag"]["launches"] > 0 and prof["bisect"]["launches"] == 0
+    assert abs(got - want) <= tol
+
+
+def test_supercell_with_cells(monkeypatch):
+    geo, st = generators.hex_sheet(4, 3, seed=9, rc_scs=40.0)
+    got, want, tol, dg, _ = _both(geo, st, monkeypatch)
+    assert np.prod(dg["supercell"]) > 1
+    assert abs(got - want) <= tol
+
+
+def _line(n, gap):
+    return Geometry(["C"] * n, np.array([[0.0, 0.0, gap * i] for i in range(n)]), np.full(n, 0.95), None)
+
+
+def _energy(geo, alpha, monkeypatch, method=None):
+    """Energy of given polarisabilities at C6 that keep omega at 0.5."""
+    a = np.full(geo.n_atoms, alpha)
+    with engine.MbdEngine(0) as eng:
+        eng.set_geometry(geo, Settings())
+        if method:
+            monkeypatch.setenv("MBD_EIG_METHOD", method)
+        eng.profile_enable(True)
+        e, om, rf, d = eng.energy(a, 0.75 * 0.5 * a * a)
+        prof = eng.profile_read()
+        C = eng.cfdm_matrix(a, om, rf, 1)
+        if method:
+            monkeypatch.delenv("MBD_EIG_METHOD")
+    lam = np.linalg.eigvalsh(np.tril(C) + np.tril(C, -1).T)
+    return e, om, d, prof, lam
+
+
+@pytest.mark.parametrize("lo,hi,path", [(0.3, 1.0, "first"), (0.03, 0.28, "second"), (-9.0, 0.0, "eig")])
+def test_every_branch(lo, hi, path, monkeypatch):
+    """A line of atoms whose polarisability is raised until the smallest
+    eigenvalue over omega^2 falls into (lo, hi)."""
+    geo = _line(24, 0.7)
+    for alpha in np.arange(2.0, 60.0, 1.0):
+        e, om, d, prof, lam = _energy(geo, alpha, monkeypatch)
+        if lo < lam[0] / om.min() ** 2 < hi:
+            break
+    else:
+        pytest.fail("no polarisability reaches the range")
+    want = 0.5 * np.sqrt(lam[lam >= 0]).sum() - 1.5 * om.sum()
+    tol = 2.2e-16 * 72 * 1.5 * om.sum() * (1.0 if path == "first" else 30.0)
+    assert d["n_negative"] == int(np.sum(lam < 0))
+    assert (prof["bisect"]["launches"] > 0) == (path == "eig")
+    # one 72 x 72 diagonal block per attempt
+    assert prof["logdet_diag"]["launches"] == (1 if path == "first" else 2)
+    assert abs(e - want) <= tol
