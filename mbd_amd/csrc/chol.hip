@@ -96,7 +96,12 @@ __device__ __forceinline__ int wave_chol(Sub<T> &G, Sub<T> &Ri) {
     // column k of L and of L^{-T} are final
     const bool in = ih ? (j <= k) : (k <= j);
     T *p = ih ? &Ri[j][k] : &G[j][k];
-    *p = in ? x[k] * rsq_fast(dd) : T(0);
+    const T rs = rsq_fast(dd);
+    T v = x[k] * rs;
+    // the diagonal correctly rounded (one Newton step of the square root): an
+    // error of one sign in every pivot would add up in the log-determinants
+    v = (!ih && j == k) ? fma(T(0.5) * rs, fma(-v, v, dd), v) : v;
+    *p = in ? v : T(0);
     if (k == DB - 1) break;
     const T a = (ih || j > k) ? x[k] * rcp_fast(dd) : T(0);
 #pragma unroll
