@@ -67,9 +67,12 @@ __device__ inline bool in_sphere(double dx, double dy, double dz, double rc, dou
 // cutoff in a 38 A cell about 76 of 343 images per pair, scattered
 // differently over the lanes).  Each pair still sums its images in table order.
 constexpr int kImgChunk = 32;
+// NEAR: near is set if an image's r^2 is so close to rc^2 that another
+// rounding of the same displacement could decide otherwise.
+template <bool NEAR = false>
 __device__ inline unsigned sphere_mask(double d0x, double d0y, double d0z,
                                        const double *__restrict__ img, int c0, int cn, int skip,
-                                       double rc2x) {
+                                       double rc2x, bool *near = nullptr) {
   unsigned m = 0;
   for (int b = 0; b < cn; ++b) {
     double dx, dy, dz, s2;
@@ -80,6 +83,7 @@ __device__ inline unsigned sphere_mask(double d0x, double d0y, double d0z,
       s2 = s2 + dz * dz;
     }
     if (s2 <= rc2x && c0 + b != skip) m |= 1u << b;
+    if (NEAR) *near = *near || fabs(s2 - rc2x) <= 3e-14 * rc2x;
   }
   return m;
 }
@@ -420,6 +424,117 @@ __global__ __launch_bounds__(256) void k_cfdm_build(
   }
   __syncthreads();
   store_tile(S, C, ldc, n, ti, tj, full);
+}
+
+// The same matrix of a supercell by cell differences: B_a[p, q] is the block
+// of atom p in cell a and atom q in cell 0 (lower 3 x 3 blocks p >= q of N
+// atoms, matrix a of B).  near[0] is set where an image lies on the cutoff
+// sphere to rounding, so that another pair of cells with the same difference
+// could have included it or not.
+__global__ __launch_bounds__(256) void k_cfdm_cells(
+    int N, const double *__restrict__ xyz, const int *__restrict__ cell,
+    const double *__restrict__ lat, int nimg, int center, const double *__restrict__ img, double rc,
+    double beta, const double *__restrict__ alpha_eff, const double *__restrict__ omega,
+    const double *__restrict__ reff, double *__restrict__ B, int *__restrict__ near) {
+  __shared__ double S[TB][TBP];
+  const double rc2x = (rc * rc) * (1.0 + 4.0 * 2.220446049250313e-16);
+  int ti, tj;
+  tri_index(blockIdx.x, ti, tj);
+  const int a = blockIdx.y, n = 3 * N;
+  const int lx = threadIdx.x % TILE, ly = threadIdx.x / TILE;
+  const int p = TILE * ti + lx, q = TILE * tj + ly;
+  if (p < N && q < N && p >= q) {
+    double acc[6] = {0, 0, 0, 0, 0, 0};
+    const bool self = p == q && a == 0;
+    const double pref = omega[p] * omega[q] * sqrt(alpha_eff[p] * alpha_eff[q]);
+    const double R12 = reff[p] + reff[q];
+    const double di = (double)cell[3 * a], dj = (double)cell[3 * a + 1], dk = (double)cell[3 * a + 2];
+    double d0x, d0y, d0z;
+    {
+#pragma clang fp contract(off)
+      const double dcx = (di * lat[0] + dj * lat[3]) + dk * lat[6];
+      const double dcy = (di * lat[1] + dj * lat[4]) + dk * lat[7];
+      const double dcz = (di * lat[2] + dj * lat[5]) + dk * lat[8];
+      d0x = (xyz[3 * p] - xyz[3 * q]) + dcx;
+      d0y = (xyz[3 * p + 1] - xyz[3 * q + 1]) + dcy;
+      d0z = (xyz[3 * p + 2] - xyz[3 * q + 2]) + dcz;
+    }
+    bool nr = false;
+    for (int c0 = 0; c0 < nimg; c0 += kImgChunk) {
+      unsigned m = sphere_mask<true>(d0x, d0y, d0z, img, c0, min(kImgChunk, nimg - c0),
+                                     self ? center : -1, rc2x, &nr);
+      while (m) {
+        double dx, dy, dz, r;
+        if (take_marked(d0x, d0y, d0z, img, c0, m, rc, rc2x, dx, dy, dz, r))
+          lr_tensor_add64(dx, dy, dz, r, R12, beta, pref, acc);
+      }
+    }
+    if (nr) atomicOr(near, 1);
+    if (self) {
+      const double w2 = omega[p] * omega[p];
+      acc[0] += w2;
+      acc[1] += w2;
+      acc[2] += w2;
+    }
+    put_block(S, lx, ly, acc);
+  }
+  __syncthreads();
+  store_tile(S, B + (long)a * n * n, n, n, ti, tj, false);
+}
+
+void cfdm_cells(hipStream_t s, int N, int ncell, const double *xyz, const int *cell,
+                const double *lat, int nimg, int center, const double *img, double rc_bohr,
+                double beta, const double *alpha_eff, const double *omega, const double *reff,
+                double *B, int *near) {
+  const int tn = ceil_div(N, TILE);
+  ProfScope ps(K_CFDM_BUILD, s, 72.0 * 0.5 * N * (N + 1.0) * ncell, 0.0);
+  hipLaunchKernelGGL(k_cfdm_cells, dim3(tn * (tn + 1) / 2, ncell), dim3(256), 0, s, N, xyz, cell, lat,
+                     nimg, center, img, rc_bohr, beta, alpha_eff, omega, reff, B, near);
+  MBD_LAUNCH_CHECK();
+}
+
+// H_k = sum_a exp(2 pi i k.a / S) B_a for r >= c: the nreal real matrices of
+// order n (Hr), and per pair k, -k the real [Re -Im; Im Re] of order 2 n (Hp),
+// lower triangles.  phase: (nreal + npair) x ncell cosines, then the pairs'
+// sines.  Each B_a is read once from HBM; the wave vectors' further reads are
+// served by the caches.
+__global__ __launch_bounds__(256) void k_cell_dft(int n, int ncell, int nreal, int npair,
+                                                  const double *__restrict__ phase,
+                                                  const double *__restrict__ B,
+                                                  double *__restrict__ Hr, double *__restrict__ Hp) {
+  const int r = blockIdx.x * 256 + threadIdx.x, c = blockIdx.y;
+  if (r < c || r >= n) return;
+  const long nn = (long)n * n;
+  const double *b = B + r + (long)c * n;
+  for (int k = 0; k < nreal; ++k) {
+    const double *cs = phase + (long)k * ncell;
+    double v = 0.0;
+    for (int a = 0; a < ncell; ++a) v += cs[a] * b[a * nn];
+    Hr[k * nn + r + (long)c * n] = v;
+  }
+  for (int k = 0; k < npair; ++k) {
+    const double *cs = phase + (long)(nreal + k) * ncell, *sn = cs + (long)npair * ncell;
+    double re = 0.0, im = 0.0;
+    for (int a = 0; a < ncell; ++a) {
+      const double v = b[a * nn];
+      re += cs[a] * v;
+      im += sn[a] * v;
+    }
+    double *H = Hp + 4 * k * nn;
+    const long ld = 2L * n;
+    H[r + c * ld] = re;
+    H[n + r + (n + c) * ld] = re;
+    H[n + r + c * ld] = r == c ? 0.0 : im;
+    if (r != c) H[n + c + r * ld] = -im;
+  }
+}
+
+void cell_dft(hipStream_t s, int n, int ncell, int nreal, int npair, const double *phase,
+              const double *B, double *Hr, double *Hp) {
+  ProfScope ps(K_CFDM_BUILD, s, 4.0 * n * (n + 1.0) * (ncell + nreal + 4.0 * npair), 0.0);
+  hipLaunchKernelGGL(k_cell_dft, dim3(ceil_div(n, 256), n), dim3(256), 0, s, n, ncell, nreal, npair,
+                     phase, B, Hr, Hp);
+  MBD_LAUNCH_CHECK();
 }
 
 void cfdm_build(hipStream_t s, int N, int ncell, const double *xyz,

@@ -144,6 +144,37 @@ std::vector<double> image_box(const double *lat, const int *half) {
 
 double norm3(const double *v) { return std::sqrt(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]); }
 
+// Whether the image box of the coupled matrix (half images to either side of
+// each supercell vector) holds every image inside the cutoff sphere for every
+// pair of atoms and cells.  A displacement at f (in supercell vectors) plus
+// image L has |f_k + L_k| h_k <= r with h_k the distance between the lattice
+// planes, so along k only images |L_k| <= rc / h_k + max |f_k| can reach.  An
+// axis without images (vacuum) has one cell and nothing to cover.
+bool images_cover(int n_atoms, const double *xyz, const double *lat, const int *S, const int *half,
+                  const int *vac, double rc) {
+  double cr[3][3], vol = 0.0;  // cr[k] = a_i x a_j: the planes' normals
+  for (int k = 0; k < 3; ++k) {
+    const double *a = lat + 3 * ((k + 1) % 3), *b = lat + 3 * ((k + 2) % 3);
+    for (int c = 0; c < 3; ++c)
+      cr[k][c] = a[(c + 1) % 3] * b[(c + 2) % 3] - a[(c + 2) % 3] * b[(c + 1) % 3];
+  }
+  for (int c = 0; c < 3; ++c) vol += lat[c] * cr[0][c];
+  for (int k = 0; k < 3; ++k) {
+    if (vac[k]) continue;
+    double lo = 1e300, hi = -1e300;
+    for (int i = 0; i < n_atoms; ++i) {
+      double f = 0.0;
+      for (int c = 0; c < 3; ++c) f += xyz[3 * i + c] * cr[k][c];
+      lo = std::min(lo, f / vol);
+      hi = std::max(hi, f / vol);
+    }
+    const double plane = S[k] * std::fabs(vol) / norm3(cr[k]);
+    const double reach = rc / plane + (hi - lo + (S[k] - 1)) / S[k];
+    if (!(reach < half[k] + 1 - 1e-9)) return false;
+  }
+  return true;
+}
+
 }  // namespace
 
 // Scratch of mbd_batch_run_noalloc: the persistent kernel's per-workgroup
@@ -242,6 +273,10 @@ struct mbd_handle {
   // blocks share A64 / inv64; bounds and sums on the device and the host
   DevBuf<double> ldHi, ldG;
   DevBuf<int> ldInfo;
+  // supercells by cell differences: blocks, their Fourier transform, phases
+  DevBuf<double> cellB, cellH, cellPh;
+  DevBuf<int> cellNear;
+  bool cells_cover = false;  // the image box covers the cutoff sphere for every pair
   // result of the last run_energy
   double e_val = 0.0;
   int n_neg = 0;
@@ -583,25 +618,39 @@ void run_scs(mbd_handle *h, int mode, mbd_diag *d) {
 
 // The energy by log-determinants rather than eigenvalues: unless
 // MBD_EIG_METHOD asks for one of the eigenvalue methods.
-bool use_logdet(long nm) { return !getenv("MBD_EIG_METHOD") && nm <= kLdMaxOrder; }
+bool use_logdet() { return !getenv("MBD_EIG_METHOD"); }
 
-// E_MBD of the coupled matrix h->C (order nm, lower triangle) by
-// log-determinants into h->e_val.  false, with nothing decided, when C has an
-// eigenvalue below a thirtieth of the smallest omega^2 (negative ones among
-// them), a value that is not finite, or no room for one shifted matrix.
-bool energy_by_logdet(mbd_handle *h, long nm) {
+// `batch` symmetric matrices of order n (lower triangles, leading dimension
+// n, back to back) whose eigenvalues together are the coupled matrix's.
+struct LdGroup {
+  int n, batch;
+  const double *H;
+};
+
+// E_MBD of the matrices of `groups` by log-determinants into h->e_val; row r
+// belongs to atom (r % (3 N cells)) / (3 cells).  false, with nothing
+// decided, when they have an eigenvalue below 0.03 of the smallest omega^2
+// (negative ones among them), a value that is not finite, or no room for one
+// shifted matrix.
+bool energy_by_logdet(mbd_handle *h, const std::vector<LdGroup> &groups, int cells) {
   hipStream_t s = h->stream;
-  const int N = h->N, n = (int)nm;
-  const int nblk = ceil_div(nm, 64), nd_max = kLdMaxNodes + 1;
-  const long sA = nm * nm, sinv = (long)ceil_div(nm, kCholNB) * kCholNB * kCholNB;
-  const size_t one = 8 * (size_t)(sA + sinv);
-  if (mem_budget() < one) return false;
-  h->ldHi.ensure(nblk);
-  h->ldG.ensure(nd_max);
-  h->ldInfo.ensure(nd_max);
-  std::vector<double> hi(nblk), om(N);
-  ld_bounds(s, n, h->C.p, nm, sA, 1, h->ldHi.p);
-  MBD_HIP(hipMemcpyAsync(hi.data(), h->ldHi.p, 8 * nblk, hipMemcpyDeviceToHost, s));
+  const int N = h->N;
+  const size_t budget = mem_budget();
+  long nhi = 0, nmat = 0;
+  for (const LdGroup &g : groups) {
+    nhi += (long)g.batch * ceil_div(g.n, 64);
+    nmat += (long)g.batch * (kLdMaxNodes + 1);
+  }
+  h->ldHi.ensure(nhi);
+  h->ldG.ensure(nmat);
+  h->ldInfo.ensure(nmat);
+  std::vector<double> hi(nhi), om(N);
+  long at = 0;
+  for (const LdGroup &g : groups) {
+    ld_bounds(s, g.n, g.H, g.n, (long)g.n * g.n, g.batch, h->ldHi.p + at);
+    at += (long)g.batch * ceil_div(g.n, 64);
+  }
+  MBD_HIP(hipMemcpyAsync(hi.data(), h->ldHi.p, 8 * nhi, hipMemcpyDeviceToHost, s));
   MBD_HIP(hipMemcpyAsync(om.data(), h->om_at.p, 8 * N, hipMemcpyDeviceToHost, s));
   MBD_HIP(hipStreamSynchronize(s));
   double top = 0.0, w2min = 1e300;
@@ -620,48 +669,115 @@ bool energy_by_logdet(mbd_handle *h, long nm) {
     LdNodes nd;
     if (!ld_nodes(frac * w2min, top, nd)) return false;
     const int all = nd.n + 1;
-    // matrices per pass: the SCS stage's memory budget, and what is free
-    int fit = (int)std::min<size_t>(mem_budget() / one, all);
-    if (h->A64.n < (size_t)fit * sA || h->inv64.n < (size_t)fit * sinv) {
-      size_t freeb = 0, total = 0;
-      MBD_HIP(hipMemGetInfo(&freeb, &total));
-      freeb = freeb / 10 * 9 + 8 * (h->A64.n + h->inv64.n);
-      fit = (int)std::min<size_t>(fit, freeb / one);
+    batch_zero(s, h->ldInfo.p, (int)nmat);
+    std::vector<int> node;  // of each factored matrix, in order
+    for (const LdGroup &g : groups) {
+      const long sA = (long)g.n * g.n, sinv = (long)ceil_div(g.n, kCholNB) * kCholNB * kCholNB;
+      const size_t one = 8 * (size_t)(sA + sinv);
+      // shifted matrices per pass: the SCS stage's memory budget, and what is free
+      size_t fit = std::min<size_t>(budget / one, (size_t)g.batch * all);
       if (fit < 1) return false;
-      try {
-        h->A64.ensure((size_t)fit * sA);
-        h->inv64.ensure((size_t)fit * sinv);
-      } catch (const HipError &e) {
-        if (e.err != hipErrorOutOfMemory) throw;
-        (void)hipGetLastError();
-        return false;
+      if (h->A64.n < fit * sA || h->inv64.n < fit * sinv) {
+        size_t freeb = 0, total = 0;
+        MBD_HIP(hipMemGetInfo(&freeb, &total));
+        fit = std::min(fit, (freeb / 10 * 9 + 8 * (h->A64.n + h->inv64.n)) / one);
+        if (fit < 1) return false;
+        try {
+          h->A64.ensure(fit * sA);
+          h->inv64.ensure(fit * sinv);
+        } catch (const HipError &e) {
+          if (e.err != hipErrorOutOfMemory) throw;
+          (void)hipGetLastError();
+          return false;
+        }
       }
+      const int rb = std::max<int>(1, (int)(fit / all)), nbmax = std::min<int>((int)fit, all);
+      for (int r0 = 0; r0 < g.batch; r0 += rb)
+        for (int b0 = 0; b0 < all; b0 += nbmax) {
+          const int rn = std::min(rb, g.batch - r0), nb = std::min(nbmax, all - b0);
+          const size_t m0 = node.size();
+          ld_shift(s, g.n, g.H + r0 * sA, g.n, sA, rn, nd, b0, nb, h->A64.p, sA);
+          potrf_batched<double>(s, g.n, h->A64.p, g.n, sA, rn * nb, h->inv64.p, sinv,
+                                h->ldInfo.p + m0, true);
+          ld_sums(s, g.n, h->A64.p, sA, rn, nd, b0, nb, h->om_at.p, N, cells, h->ldG.p + m0);
+          for (int m = 0; m < rn * nb; ++m) node.push_back(b0 + m % nb);
+        }
     }
-    batch_zero(s, h->ldInfo.p, all);
-    // the proof's shift is in the first pass, and a failure there ends it
-    std::vector<double> g(all);
-    std::vector<int> info(all, 0);
-    bool ok = true;
-    for (int end = all; end > 0 && ok;) {
-      const int nb = std::min(fit, end), b0 = end - nb;
-      end = b0;
-      ld_shift(s, n, h->C.p, nm, sA, 1, nd, b0, nb, h->A64.p, sA);
-      potrf_batched<double>(s, n, h->A64.p, n, sA, nb, h->inv64.p, sinv, h->ldInfo.p + b0, true);
-      ld_sums(s, n, h->A64.p, sA, 1, nd, b0, nb, h->om_at.p, N, h->ncell, h->ldG.p + b0);
-      MBD_HIP(hipMemcpyAsync(g.data() + b0, h->ldG.p + b0, 8 * nb, hipMemcpyDeviceToHost, s));
-      MBD_HIP(hipMemcpyAsync(info.data() + b0, h->ldInfo.p + b0, 4 * nb, hipMemcpyDeviceToHost, s));
-      MBD_HIP(hipStreamSynchronize(s));
-      for (int b = b0; b < b0 + nb; ++b) ok = ok && info[b] == 0;
-    }
-    if (!ok) continue;
+    std::vector<double> g(node.size());
+    std::vector<int> info(node.size());
+    MBD_HIP(hipMemcpyAsync(g.data(), h->ldG.p, 8 * g.size(), hipMemcpyDeviceToHost, s));
+    MBD_HIP(hipMemcpyAsync(info.data(), h->ldInfo.p, 4 * g.size(), hipMemcpyDeviceToHost, s));
+    MBD_HIP(hipStreamSynchronize(s));
+    if (std::any_of(info.begin(), info.end(), [](int i) { return i != 0; })) continue;
     double e = 0.0;
-    for (int b = 0; b < nd.n; ++b) e += nd.w[b] * g[b];
+    for (size_t m = 0; m < g.size(); ++m)
+      if (node[m] < nd.n) e += nd.w[node[m]] * g[m];
     if (!std::isfinite(e)) return false;
     h->e_val = e / h->ncell;
     h->n_neg = 0;
     return true;
   }
   return false;
+}
+
+// The energy of a supercell from the Fourier transform of its blocks over the
+// cells: C's eigenvalues are those of one Hermitian matrix of order 3 N per
+// wave vector, (3 N cells)^3 operations fall to about cells (3 N)^3.  Taken
+// where the image box covers the cutoff sphere for every pair of atoms and
+// cells (h->cells_cover: then a block depends on the cells' difference
+// alone); false, with nothing decided, where an image lies on the sphere to
+// rounding or energy_by_logdet decides nothing.
+bool energy_by_cells(mbd_handle *h, const double *alpha_eff_d) {
+  hipStream_t s = h->stream;
+  const int N = h->N, n = h->n(), nc = h->ncell, *S = h->supercell;
+  const size_t nn = (size_t)n * n;
+  // wave vectors k = -k, then one of each pair
+  std::vector<int> real, pair;
+  auto index = [&](int i, int j, int k) { return (k * S[1] + j) * S[0] + i; };
+  std::vector<int> kv(3 * (size_t)nc);
+  for (int k = 0; k < S[2]; ++k)
+    for (int j = 0; j < S[1]; ++j)
+      for (int i = 0; i < S[0]; ++i) {
+        const int q = index(i, j, k);
+        const int m = index((S[0] - i) % S[0], (S[1] - j) % S[1], (S[2] - k) % S[2]);
+        kv[3 * q] = i;
+        kv[3 * q + 1] = j;
+        kv[3 * q + 2] = k;
+        if (m == q)
+          real.push_back(q);
+        else if (q < m)
+          pair.push_back(q);
+      }
+  const int nr = (int)real.size(), np = (int)pair.size();
+  std::vector<double> ph((size_t)(nr + 2 * np) * nc);
+  for (int w = 0; w < nr + np; ++w) {
+    const int q = w < nr ? real[w] : pair[w - nr];
+    for (int a = 0; a < nc; ++a) {
+      // the cells are numbered alike (c3 S2 S1 + c2 S1 + c1)
+      double t = 0.0;
+      for (int x = 0; x < 3; ++x) t += (double)((kv[3 * q + x] * kv[3 * a + x]) % S[x]) / S[x];
+      ph[(size_t)w * nc + a] = std::cos(2.0 * kPi * t);
+      if (w >= nr) ph[(size_t)(w + np) * nc + a] = std::sin(2.0 * kPi * t);
+    }
+  }
+  h->cellPh.ensure(ph.size());
+  h->cellB.ensure(nc * nn);
+  h->cellH.ensure((nr + 4 * (size_t)np) * nn);
+  h->cellNear.ensure(1);
+  MBD_HIP(hipMemcpyAsync(h->cellPh.p, ph.data(), 8 * ph.size(), hipMemcpyHostToDevice, s));
+  batch_zero(s, h->cellNear.p, 1);
+  cfdm_cells(s, N, nc, h->xyz.p, h->cell.p, h->lat_d.p, h->nimg_cfdm, h->nimg_cfdm / 2, h->img_cfdm.p,
+             h->rc_cfdm / kBohr, h->beta, alpha_eff_d, h->om_at.p, h->reff.p, h->cellB.p,
+             h->cellNear.p);
+  cell_dft(s, n, nc, nr, np, h->cellPh.p, h->cellB.p, h->cellH.p, h->cellH.p + nr * nn);
+  int near = 0;
+  MBD_HIP(hipMemcpyAsync(&near, h->cellNear.p, sizeof near, hipMemcpyDeviceToHost, s));
+  MBD_HIP(hipStreamSynchronize(s));
+  if (near) return false;
+  std::vector<LdGroup> groups;
+  if (nr) groups.push_back({n, nr, h->cellH.p});
+  if (np) groups.push_back({2 * n, np, h->cellH.p + nr * nn});
+  return energy_by_logdet(h, groups, 1);
 }
 
 // E_MBD from device alpha_eff / c6_eff.
@@ -673,16 +789,19 @@ void run_energy(mbd_handle *h, const double *alpha_eff_d, const double *c6_d,
   h->reff.ensure(N);
   mbd_params(s, N, alpha_eff_d, c6_d, h->a0.p, h->r0.p, h->om_at.p, h->reff.p);
   const long nm = 3L * N * h->ncell;
-  h->C.ensure((size_t)nm * nm);
-  cfdm_build(s, N, h->ncell, h->xyz.p, h->cell.p, h->lat_d.p, h->nimg_cfdm,
-             h->nimg_cfdm / 2, h->img_cfdm.p, h->rc_cfdm / kBohr, h->beta,
-             alpha_eff_d, h->om_at.p, h->reff.p, h->C.p, nm, false);
   if (d) {
     d->info_eig = 0;
     for (int k = 0; k < 3; ++k) d->supercell[k] = h->supercell[k];
   }
   h->eig_flag = 0;
-  if (use_logdet(nm) && energy_by_logdet(h, nm)) return;
+  if (h->ncell > 1 && h->cells_cover && use_logdet() && energy_by_cells(h, alpha_eff_d)) return;
+  h->C.ensure((size_t)nm * nm);
+  cfdm_build(s, N, h->ncell, h->xyz.p, h->cell.p, h->lat_d.p, h->nimg_cfdm,
+             h->nimg_cfdm / 2, h->img_cfdm.p, h->rc_cfdm / kBohr, h->beta,
+             alpha_eff_d, h->om_at.p, h->reff.p, h->C.p, nm, false);
+  if (use_logdet() && nm <= kLdMaxOrder &&
+      energy_by_logdet(h, {LdGroup{(int)nm, 1, h->C.p}}, h->ncell))
+    return;
   TrdWork wk;
   h->VW.ensure((size_t)nm * 3 * kTrdNB);
   h->tau.ensure(nm);
@@ -931,6 +1050,10 @@ int mbd_destroy(mbd_handle *h) {
   h->ldHi.release();
   h->ldG.release();
   h->ldInfo.release();
+  h->cellB.release();
+  h->cellH.release();
+  h->cellPh.release();
+  h->cellNear.release();
   batch_release(h);
   if (h->trd_exec) (void)hipGraphExecDestroy(h->trd_exec);
   if (h->stream2) (void)hipStreamSynchronize(h->stream2);
@@ -1016,6 +1139,8 @@ int mbd_set_system(mbd_handle *h, int n_atoms, const double *xyz, const double *
     for (int k = 0; k < 3; ++k)
       if (h->periodic && !vac[k])
         h->cfdm_img[k] = (int)std::ceil((rc_cfdm / kBohr) / norm3(h->latSL + 3 * k));
+    h->cells_cover = h->periodic && images_cover(n_atoms, xyz, h->lat, h->supercell, h->cfdm_img, vac,
+                                                 rc_cfdm / kBohr);
     std::vector<double> ti = image_box(h->lat, h->scs_img);
     std::vector<double> tc = image_box(h->latSL, h->cfdm_img);
     h->nimg_scs = (int)(ti.size() / 3);

@@ -94,3 +94,35 @@ def test_every_branch(lo, hi, path, monkeypatch):
     # one 72 x 72 diagonal block per attempt
     assert prof["logdet_diag"]["launches"] == (1 if path == "first" else 2)
     assert abs(e - want) <= tol
+
+
+# cells short enough for 2, 3 and 4 cells along an axis (real wave vectors,
+# conjugate pairs, both), with and without a vacuum axis; atoms outside the
+# home cell and a skewed lattice, whose image boxes do not cover the cutoff
+# sphere, and images on the cutoff sphere to rounding (2 x 30 A at 60 A) keep
+# the matrix of the whole supercell
+@pytest.mark.parametrize("edges,vac,skew,out,cells,launches", [
+    ((13.0, 14.0, 14.5), None, 0.0, 0.0, [2, 2, 2], 2),
+    ((13.0, 14.0, 15.0), None, 0.0, 0.0, [2, 2, 2], 3),
+    ((9.0, 13.0, 26.0), None, 0.0, 0.0, [3, 2, 1], 2),
+    ((8.5, 9.0, 20.0), 2, 0.0, 0.0, [3, 3, 1], 2),
+    ((7.0, 26.0, 27.0), None, 0.0, 0.0, [4, 1, 1], 2),
+    ((13.0, 14.0, 26.0), None, 0.0, 4.0, [2, 2, 1], 1),
+    ((13.0, 14.0, 26.0), None, 20.0, 0.0, [2, 2, 1], 1),
+])
+def test_supercell_by_wave_vectors(edges, vac, skew, out, cells, launches, monkeypatch):
+    rng = np.random.default_rng(int(sum(edges)))
+    geo = _spread(18, 5, gap=2.3)
+    xyz = geo.coords_ang - geo.coords_ang.min(0)
+    if out:
+        xyz[0, 0] += out * edges[0]  # an atom some cells away
+    lat = np.diag(edges).astype(float)
+    lat[1, 0] = skew
+    geo = Geometry(geo.names, xyz + rng.uniform(0, 0.1, xyz.shape), geo.hirshfeld, lat)
+    st = Settings(mbd_supercell_cutoff=25.0, mbd_cfdm_dip_cutoff=60.0, mbd_scs_dip_cutoff=30.0,
+                  mbd_scs_vacuum_axis=tuple(k == vac for k in range(3)))
+    got, want, tol, dg, prof = _both(geo, st, monkeypatch)
+    assert dg["supercell"] == cells
+    # blocks by cell difference and their transform, or the whole matrix
+    assert prof["cfdm_build"]["launches"] == launches
+    assert abs(got - want) <= tol
