@@ -20,6 +20,7 @@
 // (alpha(i w), sigma), 737-739 (R_eff, omega).
 #include "common.h"
 #include "kernels.h"
+#include "mol.h"
 #include "profile.h"
 #include "tensor.h"
 
@@ -549,6 +550,122 @@ void cfdm_build(hipStream_t s, int N, int ncell, const double *xyz,
   hipLaunchKernelGGL(k_cfdm_build, grid, dim3(256), 0, s, N, ncell, xyz, cell,
                      lat, nimg, center, img, rc_bohr, beta, alpha_eff, omega,
                      reff, C, ldc, full);
+  MBD_LAUNCH_CHECK();
+}
+
+// ---------------------------------------------------------------------------
+// The same two matrices for many non-periodic molecules (one image): molecule
+// blockIdx.x, tile blockIdx.y.  The relay matrices of all grid points are
+// formed per pair (distance, 1 / r and damping once); A both triangles, L the
+// lower one in the factorisation's type.
+template <typename T>
+__global__ __launch_bounds__(256) void k_mol_scs(int natoms, const MolInfo *__restrict__ mols,
+                                                 const double *__restrict__ xyz, double rc, double beta,
+                                                 const double *__restrict__ alpha_w,
+                                                 const double *__restrict__ sgm,
+                                                 const double *__restrict__ rvdw,
+                                                 double *__restrict__ A, T *__restrict__ L) {
+  __shared__ double S[TB][TBP];
+  const MolInfo mi = mols[blockIdx.x];
+  const int n = mi.n, N = n / 3, o = mi.atom0;
+  int ti, tj;
+  tri_index(blockIdx.y, ti, tj);
+  if (TILE * ti >= N) return;
+  const int lx = threadIdx.x % TILE, ly = threadIdx.x / TILE;
+  const int i = TILE * ti + lx, j = TILE * tj + ly;
+  const bool active = i < N && j < N && i >= j, diag = i == j;
+  const int gi = o + min(i, N - 1), gj = o + min(j, N - 1);
+  double dx = 0.0, dy = 0.0, dz = 0.0, r = 1.0, ir = 0.0, damp = 0.0;
+  bool in = false;
+  if (active && !diag) {
+    dx = xyz[3 * gi] - xyz[3 * gj];
+    dy = xyz[3 * gi + 1] - xyz[3 * gj + 1];
+    dz = xyz[3 * gi + 2] - xyz[3 * gj + 2];
+    r = exact_dist(dx, dy, dz);
+    in = r <= rc;
+    ir = 1.0 / r;
+    damp = sr_damp64(r, rvdw[gi] + rvdw[gj], beta);
+  }
+  for (int f = 0; f < kNumFreq; ++f) {
+    double acc[6] = {0, 0, 0, 0, 0, 0};
+    if (in) {
+      const double si = sgm[(long)f * natoms + gi], sj = sgm[(long)f * natoms + gj];
+      sr_tensor_add64h(dx, dy, dz, r, ir, 1.0 / sqrt(si * si + sj * sj), damp, acc);
+    }
+    if (diag) acc[0] = acc[1] = acc[2] = 1.0 / alpha_w[(long)f * natoms + gi];
+    __syncthreads();
+    if (active) {
+      put_block(S, lx, ly, acc);
+      if (ti == tj && !diag) put_block(S, ly, lx, acc);
+    }
+    __syncthreads();
+    const long at = mi.a + (long)f * n * mi.ld;
+    store_tile(S, A + at, mi.ld, n, ti, tj, true);
+    for (int e = threadIdx.x; e < TB * TB; e += 256) {
+      const int row = TB * ti + e % TB, col = TB * tj + e / TB;
+      if (row < n && col <= row) L[at + row + (long)col * mi.ld] = (T)S[e / TB][e % TB];
+    }
+  }
+}
+
+template <typename T>
+void scs_build_mols(hipStream_t s, int nmol, int nmax, int natoms, const MolInfo *mols,
+                    const double *xyz, double rc, double beta, const double *alpha_w,
+                    const double *sgm, const double *rvdw, double *A, T *L) {
+  const int tn = ceil_div(nmax / 3, TILE);
+  hipLaunchKernelGGL((k_mol_scs<T>), dim3(nmol, tn * (tn + 1) / 2), dim3(256), 0, s, natoms, mols, xyz, rc,
+                     beta, alpha_w, sgm, rvdw, A, L);
+  MBD_LAUNCH_CHECK();
+}
+template void scs_build_mols<double>(hipStream_t, int, int, int, const MolInfo *, const double *, double,
+                                     double, const double *, const double *, const double *, double *,
+                                     double *);
+template void scs_build_mols<float>(hipStream_t, int, int, int, const MolInfo *, const double *, double,
+                                    double, const double *, const double *, const double *, double *,
+                                    float *);
+
+__global__ __launch_bounds__(256) void k_mol_cfdm(const MolInfo *__restrict__ mols,
+                                                  const double *__restrict__ xyz, double rc, double beta,
+                                                  const double *__restrict__ alpha,
+                                                  const double *__restrict__ omega,
+                                                  const double *__restrict__ reff,
+                                                  double *__restrict__ C) {
+  __shared__ double S[TB][TBP];
+  const MolInfo mi = mols[blockIdx.x];
+  const int n = mi.n, N = n / 3, o = mi.atom0;
+  int ti, tj;
+  tri_index(blockIdx.y, ti, tj);
+  if (TILE * ti >= N) return;
+  const int lx = threadIdx.x % TILE, ly = threadIdx.x / TILE;
+  const int i = TILE * ti + lx, j = TILE * tj + ly;
+  if (i < N && j < N && i >= j) {
+    const int gi = o + i, gj = o + j;
+    double acc[6] = {0, 0, 0, 0, 0, 0};
+    if (i == j) {
+      acc[0] = acc[1] = acc[2] = omega[gi] * omega[gi];
+    } else {
+      const double dx = xyz[3 * gi] - xyz[3 * gj], dy = xyz[3 * gi + 1] - xyz[3 * gj + 1],
+                   dz = xyz[3 * gi + 2] - xyz[3 * gj + 2], r = exact_dist(dx, dy, dz);
+      if (r <= rc)
+        lr_tensor_add64(dx, dy, dz, r, reff[gi] + reff[gj], beta,
+                        omega[gi] * omega[gj] * sqrt(alpha[gi] * alpha[gj]), acc);
+    }
+    put_block(S, lx, ly, acc);
+  }
+  __syncthreads();
+  // lower triangle only: the upper blocks of a diagonal tile were not formed
+  for (int e = threadIdx.x; e < TB * TB; e += 256) {
+    const int row = TB * ti + e % TB, col = TB * tj + e / TB;
+    if (row < n && col <= row) C[mi.c + row + (long)col * mi.ld] = S[e / TB][e % TB];
+  }
+}
+
+void cfdm_build_mols(hipStream_t s, int nmol, int nmax, const MolInfo *mols, const double *xyz,
+                     double rc, double beta, const double *alpha, const double *omega,
+                     const double *reff, double *C) {
+  const int tn = ceil_div(nmax / 3, TILE);
+  hipLaunchKernelGGL(k_mol_cfdm, dim3(nmol, tn * (tn + 1) / 2), dim3(256), 0, s, mols, xyz, rc, beta,
+                     alpha, omega, reff, C);
   MBD_LAUNCH_CHECK();
 }
 

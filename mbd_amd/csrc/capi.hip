@@ -23,6 +23,7 @@
 #include "net.h"
 #include "batch.h"
 #include "logdet.h"
+#include "mol.h"
 #include "pcg.h"
 #include "profile.h"
 #include "refine.h"
@@ -250,6 +251,13 @@ struct mbd_handle {
     int cfg = -1;  // tuned candidate, -1 = default
     hipGraphExec_t exec[2] = {nullptr, nullptr};
     int exec_cfg[2] = {-1, -1};
+    // molecules above kMolMinOrder, the first `nlarge` of the order: solved by
+    // launches over all of them (mol.h)
+    int nlarge = 0, exec_first[2] = {0, 0};
+    std::vector<int> ord, size;  // order; matrix order of each molecule in it
+    DevBuf<double> par, wA, wC, wHi, wG, wShift, wInv;
+    DevBuf<char> wL, wInfo, wMat, again;
+    DevBuf<int> wFac, wRedo, wList;
   } bt;
   // tridiagonalisation replayed from a captured graph (36k small launches at
   // n = 12288); rebuilt when the size or any buffer address changes
@@ -317,6 +325,13 @@ void batch_release(mbd_handle *h) {
   b.stat.release();
   b.phase.release();
   b.work.release();
+  DevBuf<double> *w[] = {&b.par, &b.wA, &b.wC, &b.wHi, &b.wG, &b.wShift, &b.wInv};
+  for (auto *x : w) x->release();
+  DevBuf<char> *wc[] = {&b.wL, &b.wInfo, &b.wMat, &b.again};
+  for (auto *x : wc) x->release();
+  b.wFac.release();
+  b.wRedo.release();
+  b.wList.release();
   b.nmol = 0;
 }
 
@@ -1870,17 +1885,18 @@ int batch_default_config(int nmax) {
   return -1;
 }
 
-BatchArgs batch_args(mbd_handle *h, int mode) {
+// The persistent kernel over the molecules of b.ord[first ...].
+BatchArgs batch_args(mbd_handle *h, int mode, int first) {
   auto &b = h->bt;
   BatchArgs a;
   a.nmol = b.nmol;
-  a.ntask = b.nmol * kNumFreq;
-  a.nmax = b.nmax;
-  a.S = batch_lds_stride(b.nmax);
+  a.ntask = (b.nmol - first) * kNumFreq;
+  a.nmax = b.size[first];
+  a.S = batch_lds_stride(a.nmax);
   a.natoms = b.natoms;
   a.mode = mode == MBD_MODE_FP64 ? 0 : 1;
   a.off = b.off.p;
-  a.order = b.order.p;
+  a.order = b.order.p + first;
   a.xyz = b.xyz.p;
   a.hirsh = b.hirsh.p;
   a.a0 = b.a0.p;
@@ -1892,7 +1908,7 @@ BatchArgs batch_args(mbd_handle *h, int mode) {
   a.rc_scs = b.rc_scs;
   a.rc_cfdm = b.rc_cfdm;
   a.work = b.work.p;
-  a.slot_bytes = (long)batch_slot_bytes(b.nmax);
+  a.slot_bytes = (long)batch_slot_bytes(a.nmax);
   a.alpha = b.alpha.p;
   a.c6 = b.c6.p;
   a.energy = b.energy.p;
@@ -1904,15 +1920,231 @@ BatchArgs batch_args(mbd_handle *h, int mode) {
   return a;
 }
 
-// Zero the counters and per-molecule statistics, then the persistent kernel.
-void batch_enqueue(mbd_handle *h, int mode, int cfg) {
+// Molecules that the launches over all of them take: the large ones, unless
+// MBD_EIG_METHOD asks for eigenvalues.
+int batch_first(const mbd_handle *h) { return use_logdet() ? h->bt.nlarge : 0; }
+// The same, with room for the others in the persistent kernel's slots (a
+// change of MBD_EIG_METHOD since mbd_batch_set can ask for more; the captured
+// launches hold the old address).
+int batch_room(mbd_handle *h) {
+  auto &b = h->bt;
+  const int first = batch_first(h);
+  const size_t need = first < b.nmol ? 2 * (size_t)b.ncu * batch_slot_bytes(b.size[first]) : 0;
+  if (need > b.work.n) {
+    MBD_HIP(hipStreamSynchronize(h->stream));
+    batch_drop_graphs(h);
+    b.work.ensure(need);
+  }
+  return first;
+}
+
+// Zero the counters and per-molecule statistics, then the persistent kernel
+// over the molecules from `first` on.
+void batch_enqueue(mbd_handle *h, int mode, int cfg, int first) {
   auto &b = h->bt;
   const BatchConfig &c = kBatchConfigs[cfg];
   batch_zero(h->stream, b.counter.p, 1 + b.nmol);
   batch_zero(h->stream, b.stat.p, 4 * b.nmol);
   batch_zero(h->stream, (int *)b.resid.p, 2 * b.nmol);
   batch_zero(h->stream, b.phase.p, 2 * kBatchPhases);
-  batch_launch(h->stream, c, batch_args(h, mode), b.ncu * c.per_cu);
+  if (first < b.nmol) batch_launch(h->stream, c, batch_args(h, mode, first), b.ncu * c.per_cu);
+}
+
+// The first `count` molecules of the order by launches over all of them, in
+// chunks within the SCS stage's memory budget; energies into `e` (by
+// molecule).  Appends to `redo` those that the persistent kernel has to take:
+// a failed factor, a refinement that did not converge, eigenvalues that the
+// log-determinants do not cover, or no memory.
+template <typename T>
+void batch_large_chunk(mbd_handle *h, int m0, int m1, const std::vector<int> &offs, double *e,
+                       std::vector<int> &redo) {
+  auto &b = h->bt;
+  hipStream_t s = h->stream;
+  const int nm = m1 - m0, NA = b.natoms, nmax = b.size[m0];
+  std::vector<MolInfo> info(nm);
+  long na = 0, nc = 0, ni = 0;
+  for (int q = 0; q < nm; ++q) {
+    const int n = b.size[m0 + q], id = b.ord[m0 + q];
+    MolInfo &mi = info[q];
+    mi = MolInfo{n, mol_ld(n), offs[id], id, na, nc, ni};
+    na += (long)kNumFreq * n * mi.ld;
+    nc += (long)n * mi.ld;
+    ni += kNumFreq * mol_inv_size(n);
+  }
+  const int nmat = nm * kNumFreq, nhi = ceil_div(nmax, 64);
+  b.wA.ensure(na);
+  b.wL.ensure(sizeof(T) * na);
+  b.wC.ensure(nc);
+  b.wInv.ensure(ni);
+  b.wFac.ensure(nmat);
+  b.wRedo.ensure(b.nmol);
+  b.wHi.ensure((size_t)nm * (nhi + 2));
+  b.wG.ensure(nmat);
+  b.wShift.ensure(nmat);
+  b.wInfo.ensure(sizeof(MolInfo) * nm);
+  b.wMat.ensure(sizeof(MolMat) * nmat);
+  const MolInfo *mols = (const MolInfo *)b.wInfo.p;
+  const MolMat *mats = (const MolMat *)b.wMat.p;
+  double *aw = b.par.p, *sg = aw + (long)kNumFreq * NA, *rv = sg + (long)kNumFreq * NA, *om = rv + NA,
+         *rf = om + NA, *w2 = b.wHi.p + (size_t)nm * nhi;
+  MBD_HIP(hipMemcpyAsync(b.wInfo.p, info.data(), sizeof(MolInfo) * nm, hipMemcpyHostToDevice, s));
+  batch_zero(s, b.wFac.p, nmat);
+  batch_zero(s, b.wRedo.p, b.nmol);
+
+  // SCS at every grid point
+  auto above = [&](int k) {  // matrices of order above k
+    return kNumFreq * (int)(std::partition_point(info.begin(), info.end(),
+                                                 [&](const MolInfo &m) { return m.n > k; }) - info.begin());
+  };
+  T *L = (T *)b.wL.p, *inv = (T *)b.wInv.p;
+  scs_build_mols<T>(s, nm, nmax, NA, mols, b.xyz.p, b.rc_scs, b.beta, aw, sg, rv, b.wA.p, L);
+  potrf_mols<T>(s, nmax, mols, nullptr, above, L, inv, b.wFac.p);
+  solve_mols<T>(s, nm, nmax, NA, mols, b.wA.p, L, inv, b.wFac.p, sizeof(T) == 4 ? kBatchTol : INFINITY,
+                sizeof(T) == 4 ? kBatchMaxIter : 0, b.alpha.p, b.stat.p, b.resid.p, b.wRedo.p);
+
+  // coupled matrices and their bounds
+  params_mols(s, nm, NA, mols, h->weight.p, b.a0.p, b.r0.p, b.alpha.p, b.c6.p, om, rf, b.c6_mol.p, w2);
+  cfdm_build_mols(s, nm, nmax, mols, b.xyz.p, b.rc_cfdm, b.beta, b.alpha.p, om, rf, b.wC.p);
+  ld_bounds_mols(s, nm, nmax, mols, b.wC.p, b.wHi.p);
+  std::vector<double> hi((size_t)nm * (nhi + 2));
+  std::vector<int> bad(b.nmol);
+  MBD_HIP(hipMemcpyAsync(hi.data(), b.wHi.p, 8 * hi.size(), hipMemcpyDeviceToHost, s));
+  MBD_HIP(hipMemcpyAsync(bad.data(), b.wRedo.p, 4 * bad.size(), hipMemcpyDeviceToHost, s));
+  MBD_HIP(hipStreamSynchronize(s));
+  std::vector<int> todo;  // molecules of the chunk without an energy
+  for (int q = 0; q < nm; ++q) {
+    if (bad[info[q].id])
+      redo.push_back(info[q].id);
+    else
+      todo.push_back(q);
+  }
+  // energies, as in energy_by_logdet: two guesses of the lowest eigenvalue
+  for (double frac : {0.3, 0.03}) {
+    std::vector<MolMat> mat;
+    std::vector<double> shift, wt;
+    std::vector<int> order, left;
+    for (int q : todo) {
+      double top = hi[(size_t)nm * nhi + 2 * q + 1];
+      bool ok = std::isfinite(top);
+      for (int k = 0; k < ceil_div(info[q].n, 64); ++k) {
+        const double v = hi[(size_t)q * nhi + k];
+        ok = ok && std::isfinite(v);
+        top = std::max(top, v);
+      }
+      LdNodes nd;
+      if (!ok || !ld_nodes(frac * hi[(size_t)nm * nhi + 2 * q], top, nd)) {
+        left.push_back(q);
+        continue;
+      }
+      for (int k = 0; k <= nd.n; ++k) {
+        mat.push_back(MolMat{q, k});
+        shift.push_back(nd.t[k]);
+        wt.push_back(nd.w[k]);
+        order.push_back(info[q].n);
+      }
+    }
+    const int cnt = (int)mat.size();
+    if (cnt) {
+      MBD_HIP(hipMemcpyAsync(b.wMat.p, mat.data(), sizeof(MolMat) * cnt, hipMemcpyHostToDevice, s));
+      MBD_HIP(hipMemcpyAsync(b.wShift.p, shift.data(), 8 * cnt, hipMemcpyHostToDevice, s));
+      batch_zero(s, b.wFac.p, nmat);
+      ld_shift_mols(s, cnt, order[0], mols, mats, b.wShift.p, b.wC.p, b.wA.p);
+      potrf_mols<double>(s, order[0], mols, mats,
+                         [&](int k) {
+                           return (int)(std::partition_point(order.begin(), order.end(),
+                                                             [&](int n) { return n > k; }) - order.begin());
+                         },
+                         b.wA.p, b.wInv.p, b.wFac.p);
+      ld_sums_mols(s, cnt, mols, mats, b.wShift.p, b.wA.p, om, b.wG.p);
+      std::vector<double> g(cnt);
+      std::vector<int> fac(cnt);
+      MBD_HIP(hipMemcpyAsync(g.data(), b.wG.p, 8 * cnt, hipMemcpyDeviceToHost, s));
+      MBD_HIP(hipMemcpyAsync(fac.data(), b.wFac.p, 4 * cnt, hipMemcpyDeviceToHost, s));
+      MBD_HIP(hipStreamSynchronize(s));
+      for (int k = 0; k < cnt;) {
+        const int q = mat[k].mol;
+        double sum = 0.0;
+        bool ok = true;
+        for (; k < cnt && mat[k].mol == q; ++k) {
+          sum += wt[k] != 0.0 ? wt[k] * g[k] : 0.0;
+          ok = ok && fac[k] == 0;
+        }
+        if (ok && std::isfinite(sum))
+          e[info[q].id] = sum;
+        else
+          left.push_back(q);
+      }
+    }
+    todo.swap(left);
+    std::sort(todo.begin(), todo.end());
+    if (todo.empty()) break;
+  }
+  for (int q : todo) redo.push_back(info[q].id);
+}
+
+void batch_large(mbd_handle *h, int mode, int count, double *e, std::vector<int> &redo) {
+  auto &b = h->bt;
+  const int NA = b.natoms;
+  const size_t es = mode == MBD_MODE_FP64 ? 8 : 4, budget = mem_budget();
+  std::vector<int> offs(b.nmol + 1);
+  MBD_HIP(hipMemcpyAsync(offs.data(), b.off.p, sizeof(int) * (b.nmol + 1), hipMemcpyDeviceToHost, h->stream));
+  MBD_HIP(hipStreamSynchronize(h->stream));
+  int m0 = 0;
+  try {
+    b.par.ensure((size_t)(2 * kNumFreq + 3) * NA);
+    double *aw = b.par.p, *sg = aw + (long)kNumFreq * NA, *rv = sg + (long)kNumFreq * NA;
+    atom_params(h->stream, NA, kNumFreq, h->omega.p, b.hirsh.p, b.a0.p, b.c60.p, b.r0.p, aw, sg, rv);
+    while (m0 < count) {
+      int m1 = m0;
+      for (size_t bytes = 0; m1 < count; ++m1) {
+        const int n = b.size[m1];
+        bytes += (size_t)n * mol_ld(n) * (kNumFreq * (8 + es) + 8) + 8 * (size_t)kNumFreq * mol_inv_size(n);
+        if (bytes > budget && m1 > m0) break;
+      }
+      if (mode == MBD_MODE_FP64)
+        batch_large_chunk<double>(h, m0, m1, offs, e, redo);
+      else
+        batch_large_chunk<float>(h, m0, m1, offs, e, redo);
+      m0 = m1;
+    }
+  } catch (const HipError &x) {
+    if (x.err != hipErrorOutOfMemory) throw;
+    (void)hipGetLastError();
+    for (; m0 < count; ++m0) redo.push_back(b.ord[m0]);
+  }
+}
+
+// Molecules of `redo` by the persistent kernel, their statistics anew.
+void batch_again(mbd_handle *h, int mode, std::vector<int> &redo) {
+  auto &b = h->bt;
+  hipStream_t s = h->stream;
+  std::vector<int> rank(b.nmol);
+  for (int k = 0; k < b.nmol; ++k) rank[b.ord[k]] = k;
+  std::sort(redo.begin(), redo.end(), [&](int x, int y) { return rank[x] < rank[y]; });
+  redo.erase(std::unique(redo.begin(), redo.end()), redo.end());
+  const int first = rank[redo[0]];
+  BatchArgs a = batch_args(h, mode, first);
+  a.ntask = (int)redo.size() * kNumFreq;
+  const int cfg = batch_default_config(a.nmax), grid = std::min(b.ncu * kBatchConfigs[cfg].per_cu, a.ntask);
+  b.again.ensure((size_t)grid * a.slot_bytes);
+  b.wList.ensure(redo.size());
+  MBD_HIP(hipMemcpyAsync(b.wList.p, redo.data(), sizeof(int) * redo.size(), hipMemcpyHostToDevice, s));
+  reset_mols(s, (int)redo.size(), b.wList.p, b.counter.p, b.stat.p, b.resid.p);
+  a.work = b.again.p;
+  a.order = b.wList.p;
+  batch_prepare(kBatchConfigs[cfg], a.nmax);
+  batch_launch(s, kBatchConfigs[cfg], a, grid);
+  MBD_HIP(hipStreamSynchronize(s));  // the list is the caller's
+  std::sort(redo.begin(), redo.end());
+}
+
+// The large molecules after batch_enqueue: their energies into e, those of
+// `redo` left to the device array.
+void batch_finish(mbd_handle *h, int mode, int first, std::vector<double> &e, std::vector<int> &redo) {
+  if (!first) return;
+  e.assign(h->bt.nmol, 0.0);
+  batch_large(h, mode, first, e.data(), redo);
+  if (!redo.empty()) batch_again(h, mode, redo);
 }
 
 }  // namespace
@@ -1999,7 +2231,12 @@ int mbd_batch_set(mbd_handle *h, int nmol, const int *offsets, const double *xyz
     b.counter.ensure(1 + nmol);
     b.stat.ensure(4 * nmol);
     b.phase.ensure(2 * kBatchPhases);
-    b.work.ensure(2 * (size_t)b.ncu * batch_slot_bytes(nmax));
+    b.ord = order;
+    b.size.resize(nmol);
+    for (int k = 0; k < nmol; ++k) b.size[k] = 3 * (offsets[order[k] + 1] - offsets[order[k]]);
+    b.nlarge = (int)(std::partition_point(b.size.begin(), b.size.end(),
+                                          [](int n) { return n > kMolMinOrder; }) - b.size.begin());
+    batch_room(h);
     MBD_HIP(hipStreamSynchronize(h->stream));
     if (b.cfg >= 0 && !batch_lds_bytes(kBatchConfigs[b.cfg], nmax)) b.cfg = -1;
   } catch (const HipError &e) {
@@ -2026,14 +2263,21 @@ int mbd_batch_tune(mbd_handle *h, int mode, int reps, double *times_ms, int *bes
     MBD_HIP(hipSetDevice(h->device));
     int arg = -1;
     double tbest = 0.0;
+    const int first = batch_room(h);
     for (int c = 0; c < kBatchNumConfigs; ++c) {
       double t = -1.0;
       if (batch_lds_bytes(kBatchConfigs[c], h->bt.nmax)) {
         batch_prepare(kBatchConfigs[c], h->bt.nmax);
-        batch_enqueue(h, mode, c);  // warm-up
+        auto go = [&] {
+          std::vector<double> e;
+          std::vector<int> redo;
+          batch_enqueue(h, mode, c, first);
+          batch_finish(h, mode, first, e, redo);
+        };
+        go();  // warm-up
         Timer tm;
         tm.start(h->stream);
-        for (int r = 0; r < reps; ++r) batch_enqueue(h, mode, c);
+        for (int r = 0; r < reps; ++r) go();
         tm.stop(h->stream);
         t = tm.ms() / reps;
         if (arg < 0 || t < tbest) {
@@ -2061,15 +2305,15 @@ int mbd_batch_run(mbd_handle *h, int mode, double *energy, double *alpha_eff, do
   try {
     MBD_HIP(hipSetDevice(h->device));
     const int cfg = b.cfg >= 0 ? b.cfg : batch_default_config(b.nmax);
-    const int mi = mode == MBD_MODE_FP64 ? 0 : 1;
-    if (!b.exec[mi] || b.exec_cfg[mi] != cfg) {
+    const int mi = mode == MBD_MODE_FP64 ? 0 : 1, first = batch_room(h);
+    if (!b.exec[mi] || b.exec_cfg[mi] != cfg || b.exec_first[mi] != first) {
       if (b.exec[mi]) (void)hipGraphExecDestroy(b.exec[mi]);
       b.exec[mi] = nullptr;
       batch_prepare(kBatchConfigs[cfg], b.nmax);
       hipGraph_t g = nullptr;
       MBD_HIP(hipStreamBeginCapture(h->stream, hipStreamCaptureModeRelaxed));
       try {
-        batch_enqueue(h, mode, cfg);
+        batch_enqueue(h, mode, cfg, first);
       } catch (const HipError &) {
         (void)hipStreamEndCapture(h->stream, &g);
         if (g) (void)hipGraphDestroy(g);
@@ -2080,10 +2324,14 @@ int mbd_batch_run(mbd_handle *h, int mode, double *energy, double *alpha_eff, do
       (void)hipGraphDestroy(g);
       MBD_HIP(ie);
       b.exec_cfg[mi] = cfg;
+      b.exec_first[mi] = first;
     }
+    std::vector<double> el;
+    std::vector<int> redo;
     Timer tm;
     tm.start(h->stream);
     MBD_HIP(hipGraphLaunch(b.exec[mi], h->stream));
+    batch_finish(h, mode, first, el, redo);
     tm.stop(h->stream);
     const double ms = tm.ms();
     const int NA = b.natoms, nm = b.nmol;
@@ -2100,6 +2348,8 @@ int mbd_batch_run(mbd_handle *h, int mode, double *energy, double *alpha_eff, do
     if (c6_eff) get(c6_eff, b.c6.p, sizeof(double) * NA);
     if (c6_mol) get(c6_mol, b.c6_mol.p, sizeof(double) * nm);
     MBD_HIP(hipStreamSynchronize(h->stream));
+    for (int k = 0; k < first; ++k)
+      if (!std::binary_search(redo.begin(), redo.end(), b.ord[k])) energy[b.ord[k]] = el[b.ord[k]];
     if (stat) std::copy(st.begin(), st.end(), stat);
     if (d) {
       const BatchConfig &c = kBatchConfigs[cfg];

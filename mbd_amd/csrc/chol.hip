@@ -18,9 +18,11 @@
 #include "common.h"
 #include "kernels.h"
 #include "mfma.h"
+#include "mol.h"
 #include "profile.h"
 
 #include <algorithm>
+#include <functional>
 
 namespace mbd {
 
@@ -112,10 +114,10 @@ __device__ __forceinline__ int wave_chol(Sub<T> &G, Sub<T> &Ri) {
 
 }  // namespace
 
-// Factor the kb x kb diagonal block at (k0, k0) of every matrix in the
-// batch, write L11 back, and write inv(L11) (kb x kb, zero above the
-// diagonal) to inv + b * sinv with leading dimension NB.  info[b] records the
-// first non-positive pivot as k0 + j + 1 (LAPACK convention).
+// Factor the kb x kb diagonal block M at (k0, k0) of a matrix, write L11 back,
+// and write inv(L11) (kb x kb, zero above the diagonal) to I with leading
+// dimension NB.  info records the first non-positive pivot as k0 + j + 1
+// (LAPACK convention).
 //
 // One workgroup per matrix, so a chain of dependent steps bounds it: four
 // 32 x 32 factorisations by one wave each with the panel and trailing
@@ -123,15 +125,12 @@ __device__ __forceinline__ int wave_chol(Sub<T> &G, Sub<T> &Ri) {
 // products).  A column at a time with a barrier per step took 610 us for a
 // 128 x 128 block, FP32 and FP64 alike.
 template <typename T>
-__global__ __launch_bounds__(256) void k_potrf_diag(T *A, int lda, long sA,
-                                                    int k0, int kb, T *inv,
-                                                    long sinv, int *info) {
+__device__ __forceinline__ void potrf_diag_block(T *M, int lda, int k0, int kb, T *I, int *info) {
   extern __shared__ unsigned char smem_raw[];
   DiagLds<T> &s = *reinterpret_cast<DiagLds<T> *>(smem_raw);
   using acc_t = typename Mfma<T>::acc_t;
   const acc_t zero = {0, 0, 0, 0};
-  const int b = blockIdx.x, t = threadIdx.x;
-  T *M = A + (long)b * sA + k0 + (long)k0 * lda;
+  const int t = threadIdx.x;
 
   // lower triangle into the sub-blocks, 16 columns in flight per thread
   // (clamped addresses); the identity past kb
@@ -153,7 +152,7 @@ __global__ __launch_bounds__(256) void k_potrf_diag(T *A, int lda, long sA,
   for (int k = 0; k < nb; ++k) {
     if (t < 64) {
       const int bad = wave_chol<T>(s.l[sub_index(k, k)], s.ri[k]);
-      if (t == 0 && bad < DB && info[b] == 0) info[b] = k0 + k * DB + bad + 1;
+      if (t == 0 && bad < DB && *info == 0) *info = k0 + k * DB + bad + 1;
     }
     __syncthreads();
     if (k + 1 == nb) break;
@@ -238,7 +237,6 @@ __global__ __launch_bounds__(256) void k_potrf_diag(T *A, int lda, long sA,
     }
     __syncthreads();
   }
-  T *I = inv + (long)b * sinv;
   for (int c0 = 0; c0 < kCholNB; c0 += 2) {
     const int c = c0 + ch;
     if (r < kb && c < kb)
@@ -247,6 +245,26 @@ __global__ __launch_bounds__(256) void k_potrf_diag(T *A, int lda, long sA,
                 : (r / DB == c / DB ? s.ri[r / DB][c % DB][r % DB]
                                     : s.l[sub_index(r / DB, c / DB)][r % DB][c % DB]);
   }
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void k_potrf_diag(T *A, int lda, long sA, int k0, int kb, T *inv,
+                                                    long sinv, int *info) {
+  const int b = blockIdx.x;
+  potrf_diag_block(A + (long)b * sA + k0 + (long)k0 * lda, lda, k0, kb, inv + (long)b * sinv, info + b);
+}
+
+// The same for matrix blockIdx.x of matrices of different orders.
+template <typename T>
+__global__ __launch_bounds__(256) void k_potrf_diag_mols(int k0, const MolInfo *__restrict__ mols,
+                                                         const MolMat *__restrict__ mats, T *L, T *inv,
+                                                         int *info) {
+  const MolMat z = mol_mat(mats, blockIdx.x);
+  const MolInfo mi = mols[z.mol];
+  if (k0 >= mi.n) return;
+  potrf_diag_block(L + mi.a + (long)z.slot * mi.n * mi.ld + k0 + (long)k0 * mi.ld, mi.ld, k0,
+                   min(kCholNB, mi.n - k0),
+                   inv + mi.inv + z.slot * mol_inv_size(mi.n) + (long)k0 * kCholNB, info + blockIdx.x);
 }
 
 template <typename T>
@@ -302,6 +320,31 @@ void potrf_batched(hipStream_t s, int n, T *A, int lda, long sA, int batch,
             A + o1 + (long)o1 * lda, lda, sA, batch);
   }
 }
+
+// Left-looking: block column k0 of every matrix that reaches it is updated by
+// all columns before it at once, so each element is written twice and the
+// update's K grows with k0 (orders up to about 1000: the outer blocks of the
+// right-looking form would be the whole matrix).  atleast(k) matrices, the
+// first of the list, have an order above k.
+template <typename T>
+void potrf_mols(hipStream_t s, int nmax, const MolInfo *mols, const MolMat *mats,
+                const std::function<int(int)> &atleast, T *L, T *inv, int *info) {
+  const size_t smem = sizeof(DiagLds<T>);
+  MBD_HIP(hipFuncSetAttribute((const void *)k_potrf_diag_mols<T>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
+  for (int k0 = 0; k0 < nmax; k0 += kCholNB) {
+    const int cnt = atleast(k0);
+    if (k0) gemm_mols<T>(s, true, k0, nmax, cnt, mols, mats, L, inv);
+    hipLaunchKernelGGL((k_potrf_diag_mols<T>), dim3(cnt), dim3(256), smem, s, k0, mols, mats, L, inv, info);
+    MBD_LAUNCH_CHECK();
+    gemm_mols<T>(s, false, k0, nmax, atleast(k0 + kCholNB), mols, mats, L, inv);
+  }
+}
+template void potrf_mols<double>(hipStream_t, int, const MolInfo *, const MolMat *,
+                                 const std::function<int(int)> &, double *, double *, int *);
+template void potrf_mols<float>(hipStream_t, int, const MolInfo *, const MolMat *,
+                                const std::function<int(int)> &, float *, float *, int *);
+
 template void potrf_batched<double>(hipStream_t, int, double *, int, long,
                                     int, double *, long, int *, bool);
 template void potrf_batched<float>(hipStream_t, int, float *, int, long, int,

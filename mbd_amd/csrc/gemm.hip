@@ -20,7 +20,9 @@
 // accesses, branches between the loads and K = 128 updates), against 77 and
 // 155 of the MFMAs alone.
 #include "common.h"
+#include "kernels.h"
 #include "mfma.h"
+#include "mol.h"
 
 namespace mbd {
 
@@ -52,31 +54,17 @@ struct Vec16<float> {
 // addresses are clamped and the values put right (uniform branch, edge tiles
 // only) before they go to LDS; branches between the loads had made the
 // compiler wait for each one.
+// ml, nl: rows of A and of B that may be read (m, n or more).  A wave whose
+// 64 x 64 sub-tile lies past m or n computes nothing.
 template <typename T, bool LOWER, bool GEN>
-__global__ __launch_bounds__(NT, 2) void k_gemm_nt(
-    int m, int n, int k, T alpha, const T *__restrict__ A, int lda, long sA,
-    const T *__restrict__ B, int ldb, long sB, T beta, T *__restrict__ C,
-    int ldc, long sC, int tiles_n, int ta, int tb) {
+__device__ __forceinline__ void gemm_tile(int m, int n, int ml, int nl, int k, T alpha,
+                                          const T *__restrict__ A, int lda, const T *__restrict__ B,
+                                          int ldb, T beta, T *__restrict__ C, int ldc, int tm, int tn,
+                                          int ta, int tb) {
   using vec = typename Vec16<T>::t;
   constexpr int V = Vec16<T>::n, G = 4 / V;  // row groups of a wave
   constexpr int NV = BM * BK / V / NT;       // operand vectors per thread
   constexpr int KS = NT / (BM / V);          // their distance in k
-  int tm, tn;
-  const int idx = blockIdx.x;
-  if (LOWER && idx < tiles_n * (tiles_n + 1) / 2) {
-    tm = (int)((sqrt(8.0 * idx + 1.0) - 1.0) * 0.5);
-    while ((tm + 1) * (tm + 2) / 2 <= idx) ++tm;
-    while (tm * (tm + 1) / 2 > idx) --tm;
-    tn = idx - tm * (tm + 1) / 2;
-  } else {
-    const int rest = LOWER ? idx - tiles_n * (tiles_n + 1) / 2 : idx;
-    tm = rest / tiles_n + (LOWER ? tiles_n : 0);
-    tn = rest % tiles_n;
-  }
-  const long bz = blockIdx.z;
-  A += bz * sA;
-  B += bz * sB;
-  C += bz * sC;
   const int row0 = tm * BM, col0 = tn * BN;
 
   __shared__ __align__(16) T As[2][BK][BM];
@@ -95,7 +83,7 @@ __global__ __launch_bounds__(NT, 2) void k_gemm_nt(
   // this thread's vectors: rows sr ... sr + V - 1 of the tiles, columns
   // sk + KS i; at the edges the last V rows, shifted back into place below
   const int sr = (t % (BM / V)) * V, sk = t / (BM / V);
-  const int ar = min(row0 + sr, m - V), br = min(col0 + sr, n - V);
+  const int ar = min(row0 + sr, ml - V), br = min(col0 + sr, nl - V);
   const bool edge = row0 + BM > m || col0 + BN > n;
   vec ra[NV], rb[NV];
   auto gload = [&](int k0) {
@@ -105,7 +93,7 @@ __global__ __launch_bounds__(NT, 2) void k_gemm_nt(
       if (GEN) {
 #pragma unroll
         for (int q = 0; q < V; ++q) {
-          const int r = min(row0 + sr + q, m - 1), c = min(col0 + sr + q, n - 1);
+          const int r = min(row0 + sr + q, ml - 1), c = min(col0 + sr + q, nl - 1);
           ra[i][q] = A[ta ? kc + (long)r * lda : r + (long)kc * lda];
           rb[i][q] = B[tb ? kc + (long)c * ldb : c + (long)kc * ldb];
         }
@@ -167,13 +155,14 @@ __global__ __launch_bounds__(NT, 2) void k_gemm_nt(
     }
   };
 
+  const bool idle = row0 + wm * 64 >= m || col0 + wn * 64 >= n;
   const int nk = (k + BK - 1) / BK;
   gload(0);
   sstore(0, 0);
   __syncthreads();
   for (int kt = 0; kt < nk; ++kt) {
     if (kt + 1 < nk) gload((kt + 1) * BK);
-    compute(kt & 1);
+    if (!idle) compute(kt & 1);
     if (kt + 1 < nk) sstore((kt & 1) ^ 1, (kt + 1) * BK);
     __syncthreads();
   }
@@ -244,6 +233,53 @@ __global__ __launch_bounds__(NT, 2) void k_gemm_nt(
           if (r < m && c < n && (!LOWER || r >= c)) C[r + (long)c * ldc] = x[v][q];
         }
     }
+}
+
+// One uniform batch: matrix blockIdx.z of each operand, tile blockIdx.x.
+template <typename T, bool LOWER, bool GEN>
+__global__ __launch_bounds__(NT, 2) void k_gemm_nt(
+    int m, int n, int k, T alpha, const T *__restrict__ A, int lda, long sA,
+    const T *__restrict__ B, int ldb, long sB, T beta, T *__restrict__ C,
+    int ldc, long sC, int tiles_n, int ta, int tb) {
+  int tm, tn;
+  const int idx = blockIdx.x;
+  if (LOWER && idx < tiles_n * (tiles_n + 1) / 2) {
+    tm = (int)((sqrt(8.0 * idx + 1.0) - 1.0) * 0.5);
+    while ((tm + 1) * (tm + 2) / 2 <= idx) ++tm;
+    while (tm * (tm + 1) / 2 > idx) --tm;
+    tn = idx - tm * (tm + 1) / 2;
+  } else {
+    const int rest = LOWER ? idx - tiles_n * (tiles_n + 1) / 2 : idx;
+    tm = rest / tiles_n + (LOWER ? tiles_n : 0);
+    tn = rest % tiles_n;
+  }
+  const long bz = blockIdx.z;
+  gemm_tile<T, LOWER, GEN>(m, n, m, n, k, alpha, A + bz * sA, lda, B + bz * sB, ldb, beta, C + bz * sC,
+                           ldc, tm, tn, ta, tb);
+}
+
+// The two products of a left-looking Cholesky's block column k0 over matrices
+// of different orders, matrix blockIdx.x, row tile blockIdx.y:
+// UPD:  L[k0:, k0:k0+NB] -= L[k0:, 0:k0] L[k0:k0+NB, 0:k0]^T on and below the diagonal;
+// else: L[k0+NB:, k0:k0+NB] <- itself times inv(L11)^T.
+// Rows between the order and the leading dimension may be read (they reach
+// only elements that are not stored).
+template <typename T, bool UPD>
+__global__ __launch_bounds__(NT, 2) void k_gemm_mols(int k0, const MolInfo *__restrict__ mols,
+                                                     const MolMat *__restrict__ mats, T *L,
+                                                     const T *inv) {
+  const MolMat z = mol_mat(mats, blockIdx.x);
+  const MolInfo mi = mols[z.mol];
+  const int r0 = UPD ? k0 : k0 + kCholNB, m = mi.n - r0, tm = blockIdx.y;
+  if (tm * BM >= m) return;
+  T *M = L + mi.a + (long)z.slot * mi.n * mi.ld;
+  if (UPD)
+    gemm_tile<T, true, false>(m, min(m, kCholNB), mi.ld - r0, mi.ld - r0, k0, T(-1), M + r0, mi.ld,
+                              M + r0, mi.ld, T(1), M + r0 + (long)k0 * mi.ld, mi.ld, tm, 0, 0, 0);
+  else
+    gemm_tile<T, false, false>(m, kCholNB, mi.ld - r0, kCholNB, kCholNB, T(1), M + r0 + (long)k0 * mi.ld,
+                               mi.ld, inv + mi.inv + z.slot * mol_inv_size(mi.n) + (long)k0 * kCholNB,
+                               kCholNB, T(0), M + r0 + (long)k0 * mi.ld, mi.ld, tm, 0, 0, 0);
 }
 
 // Tall-skinny FP64 update C = alpha (A1 B1^T + A2 B2^T) + beta C for at most
@@ -364,6 +400,20 @@ void gemm_ts2(hipStream_t s, int m, int n, int k, double alpha, const double *A1
                      B2, lda, ldb, beta, C, ldc);
   MBD_LAUNCH_CHECK();
 }
+
+template <typename T>
+void gemm_mols(hipStream_t s, bool upd, int k0, int nmax, int nmat, const MolInfo *mols,
+               const MolMat *mats, T *L, const T *inv) {
+  const int m = nmax - (upd ? k0 : k0 + kCholNB);
+  if (m <= 0 || nmat <= 0) return;
+  hipLaunchKernelGGL((upd ? k_gemm_mols<T, true> : k_gemm_mols<T, false>), dim3(nmat, ceil_div(m, BM)),
+                     dim3(NT), 0, s, k0, mols, mats, L, inv);
+  MBD_LAUNCH_CHECK();
+}
+template void gemm_mols<double>(hipStream_t, bool, int, int, int, const MolInfo *, const MolMat *,
+                                double *, const double *);
+template void gemm_mols<float>(hipStream_t, bool, int, int, int, const MolInfo *, const MolMat *, float *,
+                               const float *);
 
 void gemm_nt(hipStream_t s, bool lower, int m, int n, int k, double alpha,
              const double *A, int lda, long sA, const double *B, int ldb,

@@ -23,6 +23,7 @@
 
 #include "common.h"
 #include "logdet.h"
+#include "mol.h"
 
 namespace mbd {
 
@@ -93,12 +94,10 @@ bool ld_nodes(double lo, double hi, LdNodes &nd) {
 // of the diagonal) with lanes down a column; every partial has one owner and
 // a fixed order.  Each element off the diagonal blocks is read twice; HBM
 // bound (0.4 ms at n = 12288).
-__global__ __launch_bounds__(64 * GW) void k_ld_bounds(int n, const double *__restrict__ H, long ld,
-                                                       long sH, double *__restrict__ hi) {
+__device__ void bounds_block(int n, const double *__restrict__ M, long ld, int r0, double *hi) {
   __shared__ double part[GW][GB], diag[GB], below[GB];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int r0 = blockIdx.x * GB, nr = min(GB, n - r0);
-  const double *M = H + (long)blockIdx.y * sH;
+  const int nr = min(GB, n - r0);
   const int row = r0 + min(lane, nr - 1);
   double s = 0.0;
   for (int c = w; c < r0; c += 8 * GW) {
@@ -139,8 +138,28 @@ __global__ __launch_bounds__(64 * GW) void k_ld_bounds(int n, const double *__re
     double m = lane < nr ? t : -1e300;
     for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o, 64));
     if (__any(bad)) m = INFINITY;
-    if (lane == 0) hi[(long)blockIdx.y * gridDim.x + blockIdx.x] = m;
+    if (lane == 0) *hi = m;
   }
+}
+
+__global__ __launch_bounds__(64 * GW) void k_ld_bounds(int n, const double *__restrict__ H, long ld,
+                                                       long sH, double *__restrict__ hi) {
+  bounds_block(n, H + (long)blockIdx.y * sH, ld, blockIdx.x * GB,
+               hi + (long)blockIdx.y * gridDim.x + blockIdx.x);
+}
+
+// Molecule blockIdx.x, rows of blockIdx.y.
+__global__ __launch_bounds__(64 * GW) void k_ld_bounds_mols(const MolInfo *__restrict__ mols,
+                                                            const double *__restrict__ C,
+                                                            double *__restrict__ hi) {
+  const MolInfo mi = mols[blockIdx.x];
+  if ((int)blockIdx.y * GB < mi.n)
+    bounds_block(mi.n, C + mi.c, mi.ld, blockIdx.y * GB, hi + (long)blockIdx.x * gridDim.y + blockIdx.y);
+}
+
+void ld_bounds_mols(hipStream_t s, int nmol, int nmax, const MolInfo *mols, const double *C, double *hi) {
+  hipLaunchKernelGGL(k_ld_bounds_mols, dim3(nmol, ceil_div(nmax, GB)), dim3(64 * GW), 0, s, mols, C, hi);
+  MBD_LAUNCH_CHECK();
 }
 
 void ld_bounds(hipStream_t s, int n, const double *H, long ld, long sH, int batch, double *hi) {
@@ -173,6 +192,67 @@ void ld_shift(hipStream_t s, int n, const double *H, long ld, long sH, int batch
               int b0, int nb, double *A, long sA) {
   hipLaunchKernelGGL(k_ld_shift, dim3(ceil_div(n, 256), ceil_div(n, SC), batch), dim3(256), 0, s, n, H,
                      ld, sH, nd, b0, nb, A, sA);
+  MBD_LAUNCH_CHECK();
+}
+
+// Matrix blockIdx.x of a list, 256 rows by SCM columns per workgroup.
+constexpr int SCM = 32;
+__global__ __launch_bounds__(256) void k_ld_shift_mols(const MolInfo *__restrict__ mols,
+                                                       const MolMat *__restrict__ mats,
+                                                       const double *__restrict__ shift,
+                                                       const double *__restrict__ C,
+                                                       double *__restrict__ A) {
+  const MolMat z = mats[blockIdx.x];
+  const MolInfo mi = mols[z.mol];
+  const int r = blockIdx.y * 256 + threadIdx.x, n = mi.n;
+  const double t = shift[blockIdx.x];
+  const int c1 = min(n, (int)(blockIdx.z + 1) * SCM);
+  const double *M = C + mi.c;
+  double *out = A + mi.a + (long)z.slot * n * mi.ld;
+  if (r >= n) return;
+  for (int c0 = blockIdx.z * SCM; c0 < c1 && c0 <= r; c0 += SC) {
+    double v[SC];
+#pragma unroll
+    for (int i = 0; i < SC; ++i) v[i] = M[r + (long)min(c0 + i, n - 1) * mi.ld];
+#pragma unroll
+    for (int i = 0; i < SC; ++i)
+      if (c0 + i <= r) out[r + (long)(c0 + i) * mi.ld] = r == c0 + i ? v[i] + t : v[i];
+  }
+}
+
+void ld_shift_mols(hipStream_t s, int nmat, int nmax, const MolInfo *mols, const MolMat *mats,
+                   const double *shift, const double *C, double *A) {
+  hipLaunchKernelGGL(k_ld_shift_mols, dim3(nmat, ceil_div(nmax, 256), ceil_div(nmax, SCM)), dim3(256), 0, s,
+                     mols, mats, shift, C, A);
+  MBD_LAUNCH_CHECK();
+}
+
+// Matrix blockIdx.x of a list: as k_ld_sums.
+__global__ __launch_bounds__(256) void k_ld_sums_mols(const MolInfo *__restrict__ mols,
+                                                      const MolMat *__restrict__ mats,
+                                                      const double *__restrict__ shift,
+                                                      const double *__restrict__ A,
+                                                      const double *__restrict__ omega,
+                                                      double *__restrict__ g) {
+  __shared__ double red[4];
+  const MolMat z = mats[blockIdx.x];
+  const MolInfo mi = mols[z.mol];
+  const int t = threadIdx.x;
+  const double *M = A + mi.a + (long)z.slot * mi.n * mi.ld;
+  double s = 0.0;
+  for (int j = t; j < mi.n; j += 256) {
+    const double l = M[j + (long)j * mi.ld], w = omega[mi.atom0 + j / 3];
+    s += log(l * l / (w * w + shift[blockIdx.x]));
+  }
+  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+  if ((t & 63) == 0) red[t >> 6] = s;
+  __syncthreads();
+  if (t == 0) g[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
+}
+
+void ld_sums_mols(hipStream_t s, int nmat, const MolInfo *mols, const MolMat *mats, const double *shift,
+                  const double *A, const double *omega, double *g) {
+  hipLaunchKernelGGL(k_ld_sums_mols, dim3(nmat), dim3(256), 0, s, mols, mats, shift, A, omega, g);
   MBD_LAUNCH_CHECK();
 }
 
