@@ -4,6 +4,7 @@
 #include <vector>
 
 #include "common.h"
+#include "refine.h"
 
 namespace mbd {
 
@@ -23,6 +24,14 @@ bool ld_nodes(double lo, double hi, LdNodes &nd);
 // Gershgorin discs of `batch` symmetric n x n matrices (lower triangle read): hi[b nblk + i] is the
 // largest right end over rows 64 i ... 64 i + 63 of matrix b, nblk = ceil(n / 64).
 void ld_bounds(hipStream_t s, int n, const double *H, long ld, long sH, int batch, double *hi);
+// kLzSteps Lanczos steps on each matrix from three start vectors at once (V, P, Q: batch x 3 n; sv,
+// part as symv3_lower takes them, ceil(n / 256) partials per matrix); ab[((3 b + k) kLzSteps + j) 2]:
+// the tridiagonal matrices' diagonals and off-diagonals.
+constexpr int kLzSteps = 16;
+void ld_lanczos(hipStream_t s, int n, const double *H, long ld, long sH, int batch, double *V, double *P,
+                double *Q, const Symv3Work &sv, double *part, double *ab);
+// Smallest and largest Ritz value of the `count` tridiagonal matrices; false if one is not finite.
+bool ld_ritz(const double *ab, int count, double &lo, double &hi);
 // Lower triangle of H_r + t[b0 + b] I as matrix r nb + b of A (leading dimension n), r < batch, b < nb.
 void ld_shift(hipStream_t s, int n, const double *H, long ld, long sH, int batch, const LdNodes &nd,
               int b0, int nb, double *A, long sA);

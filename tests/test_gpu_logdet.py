@@ -48,6 +48,31 @@ def test_matches_eigenvalues(n, monkeypatch):
     assert abs(got - want) <= tol
 
 
+# orders from 7000 on: the interval from Ritz values (order 7002 and, one short
+# of whole 128-row blocks, 7167), and one that shows an eigenvalue below zero
+@pytest.mark.parametrize("n", [2334, 2389])
+def test_interval_from_ritz_values(n, monkeypatch):
+    got, want, tol, _, prof = _both(_spread(n, n), Settings(), monkeypatch, "2")
+    assert prof["logdet_diag"]["launches"] == -(-3 * n // 128)  # the first guess holds
+    assert abs(got - want) <= tol
+
+
+def test_ritz_value_below_zero(monkeypatch):
+    geo = _spread(2334, 7)
+    a = np.full(2334, 60.0)
+    with engine.MbdEngine(0) as eng:
+        eng.set_geometry(geo, Settings())
+        monkeypatch.setenv("MBD_EIG_METHOD", "2")
+        want, om, _, dw = eng.energy(a, 0.75 * 0.5 * a * a)
+        monkeypatch.delenv("MBD_EIG_METHOD")
+        eng.profile_enable(True)
+        got, _, _, dg = eng.energy(a, 0.75 * 0.5 * a * a)
+        prof = eng.profile_read()
+    assert dw["n_negative"] > 0 and dg["n_negative"] == dw["n_negative"]
+    assert prof["logdet_diag"]["launches"] == 0 and prof["bisect"]["launches"] > 0
+    assert got == want
+
+
 def test_supercell_with_cells(monkeypatch):
     geo, st = generators.hex_sheet(4, 3, seed=9, rc_scs=40.0)
     got, want, tol, dg, _ = _both(geo, st, monkeypatch)
