@@ -32,12 +32,12 @@ void ld_lanczos(hipStream_t s, int n, const double *H, long ld, long sH, int bat
                 double *Q, const Symv3Work &sv, double *part, double *ab);
 // Smallest and largest Ritz value of the `count` tridiagonal matrices; false if one is not finite.
 bool ld_ritz(const double *ab, int count, double &lo, double &hi);
-// Lower triangle of H_r + t[b0 + b] I as matrix r nb + b of A (leading dimension n), r < batch, b < nb.
+// Lower triangle of H_r + t[b0 + b] I as matrix r nb + b of A (leading dimension lda), r < batch, b < nb.
 void ld_shift(hipStream_t s, int n, const double *H, long ld, long sH, int batch, const LdNodes &nd,
-              int b0, int nb, double *A, long sA);
+              int b0, int nb, double *A, long lda, long sA);
 // g[m] = ln det(A_m) - ln det(D + t) from the factor's diagonal, for m < batch nb; row r of a matrix
 // belongs to atom (r % (3 N cells)) / (3 cells).
-void ld_sums(hipStream_t s, int n, const double *L, long sA, int batch, const LdNodes &nd, int b0,
+void ld_sums(hipStream_t s, int n, const double *L, long lda, long sA, int batch, const LdNodes &nd, int b0,
              int nb, const double *omega, int N, int cells, double *g);
 
 }  // namespace mbd

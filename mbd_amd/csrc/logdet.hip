@@ -289,7 +289,7 @@ void ld_bounds(hipStream_t s, int n, const double *H, long ld, long sH, int batc
 // Each element of the lower triangle read once and written once per node.
 __global__ __launch_bounds__(256) void k_ld_shift(int n, const double *__restrict__ H, long ld,
                                                   long sH, LdNodes nd, int b0, int nb,
-                                                  double *__restrict__ A, long sA) {
+                                                  double *__restrict__ A, long lda, long sA) {
   const int r = blockIdx.x * 256 + threadIdx.x, c0 = blockIdx.y * SC;
   if (blockIdx.x * 256 + 255 < c0 || r >= n) return;
   const double *M = H + (long)blockIdx.z * sH;
@@ -302,15 +302,15 @@ __global__ __launch_bounds__(256) void k_ld_shift(int n, const double *__restric
 #pragma unroll
     for (int i = 0; i < SC; ++i) {
       const int c = c0 + i;
-      if (c <= r) out[(long)c * n] = r == c ? v[i] + t : v[i];
+      if (c <= r) out[(long)c * lda] = r == c ? v[i] + t : v[i];
     }
   }
 }
 
 void ld_shift(hipStream_t s, int n, const double *H, long ld, long sH, int batch, const LdNodes &nd,
-              int b0, int nb, double *A, long sA) {
+              int b0, int nb, double *A, long lda, long sA) {
   hipLaunchKernelGGL(k_ld_shift, dim3(ceil_div(n, 256), ceil_div(n, SC), batch), dim3(256), 0, s, n, H,
-                     ld, sH, nd, b0, nb, A, sA);
+                     ld, sH, nd, b0, nb, A, lda, sA);
   MBD_LAUNCH_CHECK();
 }
 
@@ -377,7 +377,7 @@ void ld_sums_mols(hipStream_t s, int nmat, const MolInfo *mols, const MolMat *ma
 
 // One workgroup per matrix: sum over the rows of ln(L_jj^2 / (omega_j^2 + t)),
 // terms near zero, in a fixed order.
-__global__ __launch_bounds__(1024) void k_ld_sums(int n, const double *__restrict__ L, long sA,
+__global__ __launch_bounds__(1024) void k_ld_sums(int n, const double *__restrict__ L, long lda, long sA,
                                                   LdNodes nd, int b0, int nb,
                                                   const double *__restrict__ omega, int N, int cells,
                                                   double *__restrict__ g) {
@@ -387,7 +387,7 @@ __global__ __launch_bounds__(1024) void k_ld_sums(int n, const double *__restric
   const double *M = L + (long)m * sA;
   double s = 0.0;
   for (int j = t; j < n; j += 1024) {
-    const double l = M[j + (long)j * n], w = omega[(j % (3 * N * cells)) / (3 * cells)];
+    const double l = M[j + (long)j * lda], w = omega[(j % (3 * N * cells)) / (3 * cells)];
     s += log(l * l / (w * w + shift));
   }
   for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
@@ -400,9 +400,9 @@ __global__ __launch_bounds__(1024) void k_ld_sums(int n, const double *__restric
   }
 }
 
-void ld_sums(hipStream_t s, int n, const double *L, long sA, int batch, const LdNodes &nd, int b0,
+void ld_sums(hipStream_t s, int n, const double *L, long lda, long sA, int batch, const LdNodes &nd, int b0,
              int nb, const double *omega, int N, int cells, double *g) {
-  hipLaunchKernelGGL(k_ld_sums, dim3(batch * nb), dim3(1024), 0, s, n, L, sA, nd, b0, nb, omega, N,
+  hipLaunchKernelGGL(k_ld_sums, dim3(batch * nb), dim3(1024), 0, s, n, L, lda, sA, nd, b0, nb, omega, N,
                      cells, g);
   MBD_LAUNCH_CHECK();
 }
