@@ -20,6 +20,7 @@
 #include "mfma.h"
 #include "mol.h"
 #include "profile.h"
+#include "tri3.h"
 
 #include <algorithm>
 #include <functional>
@@ -354,91 +355,68 @@ template void potrf_batched<float>(hipStream_t, int, float *, int, long, int,
 // Triangular solves with NRHS = 3, X column-major n x 3 (ldx) per matrix,
 // accumulated in double (X is double; L may be float).
 
-template <typename T>
-__global__ __launch_bounds__(256) void k_trsv_diag(const T *inv, long sinv,
-                                                   int k0, int kb, double *X,
-                                                   int ldx, long sX,
-                                                   int transposed) {
-  __shared__ double xs[3][kCholNB];
-  const int b = blockIdx.x, t = threadIdx.x;
-  const T *I = inv + (long)b * sinv;
-  double *Xb = X + (long)b * sX + k0;
-  for (int e = t; e < 3 * kb; e += blockDim.x) xs[e / kb][e % kb] = Xb[(e % kb) + (long)(e / kb) * ldx];
-  __syncthreads();
-  for (int r = t; r < kb; r += blockDim.x) {
-    double s0 = 0, s1 = 0, s2 = 0;
-    if (!transposed) {
-      for (int p = 0; p <= r; ++p) {
-        const double l = (double)I[r + (long)p * kCholNB];
-        s0 += l * xs[0][p];
-        s1 += l * xs[1][p];
-        s2 += l * xs[2][p];
-      }
-    } else {
-      for (int p = r; p < kb; ++p) {
-        const double l = (double)I[p + (long)r * kCholNB];
-        s0 += l * xs[0][p];
-        s1 += l * xs[1][p];
-        s2 += l * xs[2][p];
-      }
-    }
-    Xb[r] = s0;
-    Xb[r + ldx] = s1;
-    Xb[r + 2L * ldx] = s2;
+// HBM bound: 16 coalesced loads in flight per thread on both sides (a column
+// per thread and one load at a time moved 1.8 TB/s, now 2.7; the SCS stage of a
+// 4096-atom mixed solve 158.5 -> 147 ms, of a sheet of 2048 32.3 -> 27.6).
+__device__ inline void load_rhs(const double *X, int ldx, int kb, double (*xs)[kCholNB]) {
+  for (int e = threadIdx.x; e < 3 * kCholNB; e += kTriNT) {
+    const int b = e / kCholNB, r = e % kCholNB;
+    xs[b][r] = r < kb ? X[r + (long)b * ldx] : 0.0;
   }
+  __syncthreads();
 }
 
-// forward update: X[r] -= L[r, k0:k1] X[k0:k1] for r >= k1
 template <typename T>
-__global__ __launch_bounds__(256) void k_trsv_upd_fwd(int n, const T *A, int lda,
-                                                      long sA, int k0, int kb,
-                                                      double *X, int ldx,
-                                                      long sX) {
-  __shared__ double xs[3][kCholNB];
-  const int b = blockIdx.y, t = threadIdx.x;
-  const T *M = A + (long)b * sA;
-  double *Xb = X + (long)b * sX;
-  for (int e = t; e < 3 * kb; e += blockDim.x) xs[e / kb][e % kb] = Xb[k0 + (e % kb) + (long)(e / kb) * ldx];
-  __syncthreads();
-  const int r = k0 + kb + blockIdx.x * blockDim.x + t;
-  if (r >= n) return;
-  double s0 = 0, s1 = 0, s2 = 0;
-  for (int p = 0; p < kb; ++p) {
-    const double l = (double)M[r + (long)(k0 + p) * lda];
-    s0 += l * xs[0][p];
-    s1 += l * xs[1][p];
-    s2 += l * xs[2][p];
-  }
-  Xb[r] -= s0;
-  Xb[r + ldx] -= s1;
-  Xb[r + 2L * ldx] -= s2;
+__global__ __launch_bounds__(kTriNT) void k_trsv_diag(const T *inv, long sinv, int k0, int kb, double *X,
+                                                      int ldx, long sX, int transposed) {
+  __shared__ double xs[3][kCholNB], P[3 * kTriPW];
+  const T *I = inv + (long)blockIdx.x * sinv;
+  double *Xb = X + (long)blockIdx.x * sX + k0;
+  load_rhs(Xb, ldx, kb, xs);
+  auto put = [&](int r, double a, double b, double c) {
+    Xb[r] = a;
+    Xb[r + ldx] = b;
+    Xb[r + 2L * ldx] = c;
+  };
+  if (transposed)
+    dot3(I, kCholNB, kb, kb, xs[0], kCholNB, put);
+  else
+    mv3(I, kCholNB, kb, kb, xs[0], kCholNB, P, put);
 }
 
-// backward update: X[j] -= L[k0:k1, j]^T X[k0:k1] for j < k0
+// forward update: X[r] -= L[r, k0:k1] X[k0:k1] for r >= k1, kTriNT rows per
+// workgroup
 template <typename T>
-__global__ __launch_bounds__(256) void k_trsv_upd_bwd(const T *A, int lda,
-                                                      long sA, int k0, int kb,
-                                                      double *X, int ldx,
-                                                      long sX) {
+__global__ __launch_bounds__(kTriNT) void k_trsv_upd_fwd(int n, const T *A, int lda, long sA, int k0,
+                                                         int kb, double *X, int ldx, long sX) {
+  __shared__ double xs[3][kCholNB], P[3 * kTriPW];
+  double *Xb = X + (long)blockIdx.y * sX;
+  load_rhs(Xb + k0, ldx, kb, xs);
+  const int r0 = k0 + kb + blockIdx.x * kTriNT;
+  mv3(A + (long)blockIdx.y * sA + r0 + (long)k0 * lda, lda, min(kTriNT, n - r0), kb, xs[0], kCholNB, P,
+      [&](int r, double a, double b, double c) {
+        Xb[r0 + r] -= a;
+        Xb[r0 + r + ldx] -= b;
+        Xb[r0 + r + 2L * ldx] -= c;
+      });
+}
+
+// backward update: X[j] -= L[k0:k1, j]^T X[k0:k1] for j < k0, kTrsvCols
+// columns per workgroup
+constexpr int kTrsvCols = kTriNT / 64 * kTriU;
+template <typename T>
+__global__ __launch_bounds__(kTriNT) void k_trsv_upd_bwd(const T *A, int lda, long sA, int k0, int kb,
+                                                         double *X, int ldx, long sX) {
   __shared__ double xs[3][kCholNB];
-  const int b = blockIdx.y, t = threadIdx.x;
-  const T *M = A + (long)b * sA;
-  double *Xb = X + (long)b * sX;
-  for (int e = t; e < 3 * kb; e += blockDim.x) xs[e / kb][e % kb] = Xb[k0 + (e % kb) + (long)(e / kb) * ldx];
-  __syncthreads();
-  const int j = blockIdx.x * blockDim.x + t;
-  if (j >= k0) return;
-  const T *col = M + k0 + (long)j * lda;
-  double s0 = 0, s1 = 0, s2 = 0;
-  for (int p = 0; p < kb; ++p) {
-    const double l = (double)col[p];
-    s0 += l * xs[0][p];
-    s1 += l * xs[1][p];
-    s2 += l * xs[2][p];
-  }
-  Xb[j] -= s0;
-  Xb[j + ldx] -= s1;
-  Xb[j + 2L * ldx] -= s2;
+  double *Xb = X + (long)blockIdx.y * sX;
+  load_rhs(Xb + k0, ldx, kb, xs);
+  const int j0 = blockIdx.x * kTrsvCols;
+  dot3(A + (long)blockIdx.y * sA + k0 + (long)j0 * lda, lda, kb, min(kTrsvCols, k0 - j0), xs[0], kCholNB,
+       [&](int c, double a, double b, double d) {
+         Xb[j0 + c] -= a;
+         Xb[j0 + c + ldx] -= b;
+         Xb[j0 + c + 2L * ldx] -= d;
+       });
 }
 
 template <typename T>
@@ -467,7 +445,7 @@ void potrs3_batched(hipStream_t s, int n, const T *L, int lda, long sA,
     MBD_LAUNCH_CHECK();
     if (k0 > 0) {
       ProfScope ps(K_TRSV, s, batch * (double)k0 * kb * sizeof(T), 2.0 * 3 * batch * k0 * kb);
-      hipLaunchKernelGGL((k_trsv_upd_bwd<T>), dim3(ceil_div(k0, 256), batch),
+      hipLaunchKernelGGL((k_trsv_upd_bwd<T>), dim3(ceil_div(k0, kTrsvCols), batch),
                          dim3(256), 0, s, L, lda, sA, k0, kb, X, ldx, sX);
       MBD_LAUNCH_CHECK();
     }
