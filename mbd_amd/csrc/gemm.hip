@@ -162,7 +162,9 @@ __device__ __forceinline__ void gemm_tile(int m, int n, int ml, int nl, int k, T
   __syncthreads();
   for (int kt = 0; kt < nk; ++kt) {
     if (kt + 1 < nk) gload((kt + 1) * BK);
+    __builtin_amdgcn_s_setprio(1);  // its MFMAs before the other waves' loads
     if (!idle) compute(kt & 1);
+    __builtin_amdgcn_s_setprio(0);
     if (kt + 1 < nk) sstore((kt & 1) ^ 1, (kt + 1) * BK);
     __syncthreads();
   }
