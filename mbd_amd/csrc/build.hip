@@ -28,6 +28,7 @@ namespace mbd {
 
 namespace {
 
+constexpr int kFullTiles = 512;  // tiles that fill the 256 CUs with one workgroup each
 constexpr int kFreqGroup = 7;   // grid points per image scan of the SCS builder
 constexpr int TILE = 16;        // atoms (sites) per tile edge
 constexpr int TB = 3 * TILE;    // matrix rows per tile edge
@@ -172,19 +173,20 @@ void atom_params(hipStream_t s, int N, int nf, const double *omega,
 // kFreqGroup grid points.  Off-diagonal block (i, j): sum over images n of
 // T_sr(r_i - r_j + L_n; sqrt(s_i^2 + s_j^2), R_i + R_j); diagonal block:
 // (1/alpha_i) I + sum over n != 0 of T_sr(L_n; s_i, 2 R_i).
-template <typename T>
-__global__ __launch_bounds__(256) void k_scs_build(
+template <typename T, int F, int IS>
+__global__ __launch_bounds__(256 * IS) void k_scs_build(
     int N, const double *__restrict__ xyz, int nimg, int center,
     const double *__restrict__ img, double rc, double beta,
     const double *__restrict__ alpha_w, const double *__restrict__ sgm,
     const double *__restrict__ rvdw, T *__restrict__ A, int lda,
     long stride, int nf, bool full) {
-  constexpr int F = kFreqGroup;
   __shared__ T S[TB][TBP];
+  __shared__ double part[IS > 1 ? IS - 1 : 1][6][IS > 1 ? 256 : 1];
   int ti, tj;
   tri_index(blockIdx.x, ti, tj);
   const int n = 3 * N;
-  const int lx = threadIdx.x % TILE, ly = threadIdx.x / TILE;
+  const int pair = threadIdx.x % 256, slice = IS > 1 ? threadIdx.x / 256 : 0;
+  const int lx = pair % TILE, ly = pair / TILE;
   const int i = TILE * ti + lx, j = TILE * tj + ly;
   const bool active = (i < N && j < N && (ti != tj || i >= j));
   const bool diag = (i == j);
@@ -200,9 +202,13 @@ __global__ __launch_bounds__(256) void k_scs_build(
       R12 = rvdw[i] + rvdw[j];
     }
   }
-  for (int f0 = 0; f0 < nf; f0 += F) {
+  for (int f0 = blockIdx.y * F; f0 < nf; f0 += gridDim.y * F) {
     const int nfg = min(F, nf - f0);
-    T out[F][6];
+    double acc[F][6];
+#pragma unroll
+    for (int g = 0; g < F; ++g)
+#pragma unroll
+      for (int e = 0; e < 6; ++e) acc[g][e] = 0.0;
     if (active) {
       // sigma of the pair at each grid point of the group
       double sg12[F];
@@ -213,14 +219,10 @@ __global__ __launch_bounds__(256) void k_scs_build(
         sg12[g] = diag ? si : sqrt(si * si + sj * sj);
       }
       if (sizeof(T) == 8) {
-        double acc[F][6], isg[F];
+        double isg[F];
 #pragma unroll
-        for (int g = 0; g < F; ++g) {
-          isg[g] = 1.0 / sg12[g];
-#pragma unroll
-          for (int e = 0; e < 6; ++e) acc[g][e] = 0.0;
-        }
-        for (int c0 = 0; c0 < nimg; c0 += kImgChunk) {
+        for (int g = 0; g < F; ++g) isg[g] = 1.0 / sg12[g];
+        for (int c0 = kImgChunk * slice; c0 < nimg; c0 += kImgChunk * IS) {
           unsigned m = sphere_mask(d0x, d0y, d0z, img, c0, min(kImgChunk, nimg - c0),
                                    diag ? center : -1, rc2x);
           while (m) {
@@ -232,21 +234,10 @@ __global__ __launch_bounds__(256) void k_scs_build(
               if (g < nfg) sr_tensor_add64h(dx, dy, dz, r, ir, isg[g], damp, acc[g]);
           }
         }
-#pragma unroll
-        for (int g = 0; g < F; ++g) {
-          const double inv = diag ? 1.0 / alpha_w[(long)(f0 + min(g, nfg - 1)) * N + i] : 0.0;
-#pragma unroll
-          for (int e = 0; e < 6; ++e) out[g][e] = (T)(acc[g][e] + (e < 3 ? inv : 0.0));
-        }
       } else {
         // FP32 terms summed in FP64: a conversion and an add per term
         // against the eight operations of a compensated FP32 sum, with the
         // same registers and a smaller error (FP64 adds run at the FP32 rate)
-        double acc[F][6];
-#pragma unroll
-        for (int g = 0; g < F; ++g)
-#pragma unroll
-          for (int e = 0; e < 6; ++e) acc[g][e] = 0.0;
         const float fb = (float)beta, fR = (float)R12;
         const float ibR = 1.0f / (fb * fR);
         // per grid point 1 / sigma and 2/sqrt(pi) / sigma^3, per image the
@@ -259,7 +250,7 @@ __global__ __launch_bounds__(256) void k_scs_build(
           isg[g] = 1.0f / (float)sg12[g];
           zc[g] = 2.25675833f * isg[g] * isg[g] * isg[g];
         }
-        for (int c0 = 0; c0 < nimg; c0 += kImgChunk) {
+        for (int c0 = kImgChunk * slice; c0 < nimg; c0 += kImgChunk * IS) {
           unsigned m = sphere_mask(d0x, d0y, d0z, img, c0, min(kImgChunk, nimg - c0),
                                    diag ? center : -1, rc2x);
           while (m) {
@@ -288,21 +279,29 @@ __global__ __launch_bounds__(256) void k_scs_build(
             }
           }
         }
-#pragma unroll
-        for (int g = 0; g < F; ++g) {
-          const double inv = diag ? 1.0 / alpha_w[(long)(f0 + min(g, nfg - 1)) * N + i] : 0.0;
-#pragma unroll
-          for (int e = 0; e < 6; ++e) out[g][e] = (T)(acc[g][e] + (e < 3 ? inv : 0.0));
-        }
       }
     }
 #pragma unroll
     for (int g = 0; g < F; ++g) {
       if (g < nfg) {
         __syncthreads();
-        if (active) {
-          put_block(S, lx, ly, out[g]);
-          if (ti == tj && !diag) put_block(S, ly, lx, out[g]);
+        if (IS > 1) {  // the slices' sums, in their order
+          if (slice > 0)
+#pragma unroll
+            for (int e = 0; e < 6; ++e) part[slice - 1][e][pair] = acc[g][e];
+          __syncthreads();
+          if (slice == 0)
+            for (int q = 0; q < IS - 1; ++q)
+#pragma unroll
+              for (int e = 0; e < 6; ++e) acc[g][e] += part[q][e][pair];
+        }
+        if (active && slice == 0) {
+          const double inv = diag ? 1.0 / alpha_w[(long)(f0 + g) * N + i] : 0.0;
+          T out[6];
+#pragma unroll
+          for (int e = 0; e < 6; ++e) out[e] = (T)(acc[g][e] + (e < 3 ? inv : 0.0));
+          put_block(S, lx, ly, out);
+          if (ti == tj && !diag) put_block(S, ly, lx, out);
         }
         __syncthreads();
         store_tile(S, A + (long)(f0 + g) * stride, lda, n, ti, tj, full);
@@ -316,13 +315,28 @@ void scs_build(hipStream_t s, int N, const double *xyz, int nimg, int center,
                const double *img, double rc_bohr, double beta,
                const double *alpha_w, const double *sgm, const double *rvdw,
                T *A, int lda, long stride, int nf, bool full) {
-  const int tn = ceil_div(N, TILE);
-  dim3 grid(tn * (tn + 1) / 2);
+  const int tn = ceil_div(N, TILE), nt = tn * (tn + 1) / 2;
   // algorithmic output: the lower 3x3 blocks of each matrix
   ProfScope ps(K_SCS_BUILD, s, 9.0 * sizeof(T) * 0.5 * N * (N + 1.0) * nf, 0.0);
-  hipLaunchKernelGGL((k_scs_build<T>), grid, dim3(256), 0, s, N, xyz, nimg,
-                     center, img, rc_bohr, beta, alpha_w, sgm, rvdw, A, lda,
-                     stride, nf, full);
+  auto go = [&](auto *kern, int f, int is) {
+    hipLaunchKernelGGL(kern, dim3(nt, ceil_div(nf, f)), dim3(256 * is), 0, s, N, xyz, nimg, center, img,
+                       rc_bohr, beta, alpha_w, sgm, rvdw, A, lda, stride, nf, full);
+  };
+  // Few tiles leave the chip idle: the grid points go to workgroups of their
+  // own (a tile's distances are formed again for each group of them), and a
+  // long image list to two or four slices of a workgroup (FP64: a sheet of 60
+  // atoms 2.23 -> 0.18 ms, a cell of 60 3.9 -> 0.31, of 150 1.9 -> 0.56, of
+  // 400 1.28 -> 1.06; with the chip full the shared distances win).
+  const bool split = nimg >= 4 * kImgChunk;
+  if (nt >= kFullTiles)
+    hipLaunchKernelGGL((k_scs_build<T, kFreqGroup, 1>), dim3(nt), dim3(256), 0, s, N, xyz, nimg, center,
+                       img, rc_bohr, beta, alpha_w, sgm, rvdw, A, lda, stride, nf, full);
+  else if (!split)
+    go(k_scs_build<T, 1, 1>, 1, 1);
+  else if (nt >= kFullTiles / 14)
+    go(k_scs_build<T, 3, 2>, 3, 2);
+  else
+    go(k_scs_build<T, 1, 4>, 1, 4);
   MBD_LAUNCH_CHECK();
 }
 template void scs_build<double>(hipStream_t, int, const double *, int, int,
