@@ -280,6 +280,7 @@ def main():
     bound = {"trd_symv": "hbm", "scs_build": "hbm", "cfdm_build": "hbm", "trsv": "hbm",
              "refine_residual": "hbm", "pcg_symv": "hbm", "chol_syrk_gemm": "fp32_tflops",
              "chol_trsm_gemm": "fp32_tflops", "trd_syr2k_gemm": "fp64_tflops",
+             "logdet_syrk_gemm": "fp64_tflops", "logdet_trsm_gemm": "fp64_tflops",
              "sbr_symm": "fp64_tflops", "sbr_panel_qr": "hbm", "sbr_chase": "hbm"}.get(dom, "hbm")
     out["roofline"] = roofline_entry(prof_m, dom, bound)
     ratio = measured_traffic_ratio(dom)
@@ -290,10 +291,11 @@ def main():
             f"the same workload) times the algorithmic bytes per launch of this run")
     others = {}
     for k in ("scs_build", "cfdm_build", "pcg_symv", "refine_residual", "trd_symv", "chol_syrk_gemm",
-              "sbr_symm", "trd_syr2k_gemm", "sbr_chase"):
+              "sbr_symm", "trd_syr2k_gemm", "sbr_chase", "logdet_syrk_gemm"):
         if k in prof_m and prof_m[k]["launches"] and k != dom:
             others[k] = roofline_entry(prof_m, k, {"chol_syrk_gemm": "fp32_tflops",
                                                    "sbr_symm": "fp64_tflops",
+                                                   "logdet_syrk_gemm": "fp64_tflops",
                                                    "trd_syr2k_gemm": "fp64_tflops"}.get(k, "hbm"))
             r = measured_traffic_ratio(k)
             if r is not None and prof_m[k]["bytes"] > 0:
