@@ -254,7 +254,10 @@ struct mbd_handle {
     // molecules above kMolMinOrder, the first `nlarge` of the order: solved by
     // launches over all of them (mol.h)
     int nlarge = 0, exec_first[2] = {0, 0};
+    hipStream_t side = nullptr;  // the persistent kernel beside them
+    hipEvent_t fork = nullptr, join = nullptr;
     std::vector<int> ord, size;  // order; matrix order of each molecule in it
+    std::vector<int> first;      // first atom of each molecule
     DevBuf<double> par, wA, wC, wHi, wG, wShift, wInv;
     DevBuf<char> wL, wInfo, wMat, again;
     DevBuf<int> wFac, wRedo, wList;
@@ -329,6 +332,13 @@ void batch_release(mbd_handle *h) {
   for (auto *x : w) x->release();
   DevBuf<char> *wc[] = {&b.wL, &b.wInfo, &b.wMat, &b.again};
   for (auto *x : wc) x->release();
+  if (b.side) {
+    (void)hipStreamSynchronize(b.side);
+    (void)hipEventDestroy(b.fork);
+    (void)hipEventDestroy(b.join);
+    (void)hipStreamDestroy(b.side);
+    b.side = nullptr;
+  }
   b.wFac.release();
   b.wRedo.release();
   b.wList.release();
@@ -1997,16 +2007,19 @@ int batch_room(mbd_handle *h) {
   return first;
 }
 
-// Zero the counters and per-molecule statistics, then the persistent kernel
-// over the molecules from `first` on.
-void batch_enqueue(mbd_handle *h, int mode, int cfg, int first) {
+// Counters and per-molecule statistics to zero.
+void batch_clear(mbd_handle *h) {
   auto &b = h->bt;
-  const BatchConfig &c = kBatchConfigs[cfg];
   batch_zero(h->stream, b.counter.p, 1 + b.nmol);
   batch_zero(h->stream, b.stat.p, 4 * b.nmol);
   batch_zero(h->stream, (int *)b.resid.p, 2 * b.nmol);
   batch_zero(h->stream, b.phase.p, 2 * kBatchPhases);
-  if (first < b.nmol) batch_launch(h->stream, c, batch_args(h, mode, first), b.ncu * c.per_cu);
+}
+
+// The persistent kernel over the molecules from `first` on.
+void batch_small(mbd_handle *h, hipStream_t s, int mode, int cfg, int first) {
+  const BatchConfig &c = kBatchConfigs[cfg];
+  if (first < h->bt.nmol) batch_launch(s, c, batch_args(h, mode, first), h->bt.ncu * c.per_cu);
 }
 
 // The first `count` molecules of the order by launches over all of them, in
@@ -2015,8 +2028,7 @@ void batch_enqueue(mbd_handle *h, int mode, int cfg, int first) {
 // a failed factor, a refinement that did not converge, eigenvalues that the
 // log-determinants do not cover, or no memory.
 template <typename T>
-void batch_large_chunk(mbd_handle *h, int m0, int m1, const std::vector<int> &offs, double *e,
-                       std::vector<int> &redo) {
+void batch_large_chunk(mbd_handle *h, int m0, int m1, double *e, std::vector<int> &redo) {
   auto &b = h->bt;
   hipStream_t s = h->stream;
   const int nm = m1 - m0, NA = b.natoms, nmax = b.size[m0];
@@ -2025,7 +2037,7 @@ void batch_large_chunk(mbd_handle *h, int m0, int m1, const std::vector<int> &of
   for (int q = 0; q < nm; ++q) {
     const int n = b.size[m0 + q], id = b.ord[m0 + q];
     MolInfo &mi = info[q];
-    mi = MolInfo{n, mol_ld(n), offs[id], id, na, nc, ni};
+    mi = MolInfo{n, mol_ld(n), b.first[id], id, na, nc, ni};
     na += (long)kNumFreq * n * mi.ld;
     nc += (long)n * mi.ld;
     ni += kNumFreq * mol_inv_size(n);
@@ -2145,9 +2157,6 @@ void batch_large(mbd_handle *h, int mode, int count, double *e, std::vector<int>
   auto &b = h->bt;
   const int NA = b.natoms;
   const size_t es = mode == MBD_MODE_FP64 ? 8 : 4, budget = mem_budget();
-  std::vector<int> offs(b.nmol + 1);
-  MBD_HIP(hipMemcpyAsync(offs.data(), b.off.p, sizeof(int) * (b.nmol + 1), hipMemcpyDeviceToHost, h->stream));
-  MBD_HIP(hipStreamSynchronize(h->stream));
   int m0 = 0;
   try {
     b.par.ensure((size_t)(2 * kNumFreq + 3) * NA);
@@ -2161,9 +2170,9 @@ void batch_large(mbd_handle *h, int mode, int count, double *e, std::vector<int>
         if (bytes > budget && m1 > m0) break;
       }
       if (mode == MBD_MODE_FP64)
-        batch_large_chunk<double>(h, m0, m1, offs, e, redo);
+        batch_large_chunk<double>(h, m0, m1, e, redo);
       else
-        batch_large_chunk<float>(h, m0, m1, offs, e, redo);
+        batch_large_chunk<float>(h, m0, m1, e, redo);
       m0 = m1;
     }
   } catch (const HipError &x) {
@@ -2197,12 +2206,37 @@ void batch_again(mbd_handle *h, int mode, std::vector<int> &redo) {
   std::sort(redo.begin(), redo.end());
 }
 
-// The large molecules after batch_enqueue: their energies into e, those of
-// `redo` left to the device array.
-void batch_finish(mbd_handle *h, int mode, int first, std::vector<double> &e, std::vector<int> &redo) {
+// One pass over the batch, `small(stream)` launching the persistent kernel:
+// energies of the first `first` molecules into e, those of `redo` (sorted)
+// and of the others left to the device array.  With molecules of both kinds
+// the persistent kernel runs on a stream of its own beside the launches for
+// the large ones: they share no results, and it leaves half of each CU idle.
+template <typename F>
+void batch_pass(mbd_handle *h, int mode, int first, F small, std::vector<double> &e, std::vector<int> &redo) {
+  auto &b = h->bt;
+  batch_clear(h);
+  if (!first || first == b.nmol) {
+    if (!first) small(h->stream);
+  } else {
+    if (!b.side) {
+      MBD_HIP(hipStreamCreateWithFlags(&b.side, hipStreamNonBlocking));
+      MBD_HIP(hipEventCreateWithFlags(&b.fork, hipEventDisableTiming));
+      MBD_HIP(hipEventCreateWithFlags(&b.join, hipEventDisableTiming));
+    }
+    MBD_HIP(hipEventRecord(b.fork, h->stream));
+    MBD_HIP(hipStreamWaitEvent(b.side, b.fork, 0));
+    small(b.side);
+    MBD_HIP(hipEventRecord(b.join, b.side));
+  }
   if (!first) return;
-  e.assign(h->bt.nmol, 0.0);
-  batch_large(h, mode, first, e.data(), redo);
+  e.assign(b.nmol, 0.0);
+  try {
+    batch_large(h, mode, first, e.data(), redo);
+  } catch (...) {
+    if (b.side) (void)hipStreamSynchronize(b.side);
+    throw;
+  }
+  if (first < b.nmol) MBD_HIP(hipStreamWaitEvent(h->stream, b.join, 0));
   if (!redo.empty()) batch_again(h, mode, redo);
 }
 
@@ -2291,6 +2325,7 @@ int mbd_batch_set(mbd_handle *h, int nmol, const int *offsets, const double *xyz
     b.stat.ensure(4 * nmol);
     b.phase.ensure(2 * kBatchPhases);
     b.ord = order;
+    b.first.assign(offsets, offsets + nmol);
     b.size.resize(nmol);
     for (int k = 0; k < nmol; ++k) b.size[k] = 3 * (offsets[order[k] + 1] - offsets[order[k]]);
     b.nlarge = (int)(std::partition_point(b.size.begin(), b.size.end(),
@@ -2330,8 +2365,7 @@ int mbd_batch_tune(mbd_handle *h, int mode, int reps, double *times_ms, int *bes
         auto go = [&] {
           std::vector<double> e;
           std::vector<int> redo;
-          batch_enqueue(h, mode, c, first);
-          batch_finish(h, mode, first, e, redo);
+          batch_pass(h, mode, first, [&](hipStream_t s) { batch_small(h, s, mode, c, first); }, e, redo);
         };
         go();  // warm-up
         Timer tm;
@@ -2365,14 +2399,14 @@ int mbd_batch_run(mbd_handle *h, int mode, double *energy, double *alpha_eff, do
     MBD_HIP(hipSetDevice(h->device));
     const int cfg = b.cfg >= 0 ? b.cfg : batch_default_config(b.nmax);
     const int mi = mode == MBD_MODE_FP64 ? 0 : 1, first = batch_room(h);
-    if (!b.exec[mi] || b.exec_cfg[mi] != cfg || b.exec_first[mi] != first) {
+    if (first < b.nmol && (!b.exec[mi] || b.exec_cfg[mi] != cfg || b.exec_first[mi] != first)) {
       if (b.exec[mi]) (void)hipGraphExecDestroy(b.exec[mi]);
       b.exec[mi] = nullptr;
       batch_prepare(kBatchConfigs[cfg], b.nmax);
       hipGraph_t g = nullptr;
       MBD_HIP(hipStreamBeginCapture(h->stream, hipStreamCaptureModeRelaxed));
       try {
-        batch_enqueue(h, mode, cfg, first);
+        batch_small(h, h->stream, mode, cfg, first);
       } catch (const HipError &) {
         (void)hipStreamEndCapture(h->stream, &g);
         if (g) (void)hipGraphDestroy(g);
@@ -2389,8 +2423,7 @@ int mbd_batch_run(mbd_handle *h, int mode, double *energy, double *alpha_eff, do
     std::vector<int> redo;
     Timer tm;
     tm.start(h->stream);
-    MBD_HIP(hipGraphLaunch(b.exec[mi], h->stream));
-    batch_finish(h, mode, first, el, redo);
+    batch_pass(h, mode, first, [&](hipStream_t s) { MBD_HIP(hipGraphLaunch(b.exec[mi], s)); }, el, redo);
     tm.stop(h->stream);
     const double ms = tm.ms();
     const int NA = b.natoms, nm = b.nmol;

@@ -79,3 +79,24 @@ def test_memory_chunks(monkeypatch):
     got = _batch(mols, "mixed", monkeypatch)
     assert np.array_equal(got["energy"], want["energy"])
     assert np.array_equal(got["alpha_all"], want["alpha_all"])
+
+
+# molecules with close contacts, some of them with an atom of negative alpha
+# (a coupled matrix that is not finite) or with omega^2 over four decades and
+# more, which the log-determinants do not cover
+@pytest.mark.parametrize("mode", ["fp64", "mixed"])
+def test_close_contacts(mode, monkeypatch):
+    mols = generators.chain_molecules()[0][::11]
+    got, want = _batch(mols, mode, monkeypatch), _batch(mols, mode, monkeypatch, "1")
+    off = got["offsets"]
+    low = np.array([want["alpha_eff"][a:b].min() for a, b in zip(off[:-1], off[1:])])
+    assert (low < 0).any() and ((low > 0) & (low < 0.5)).any()
+    # as above, alpha relative to its molecule's largest: a small one is a difference
+    for a, b in zip(off[:-1], off[1:]):
+        w = want["alpha_all"][:, a:b]
+        assert np.all(np.abs(got["alpha_all"][:, a:b] - w) <= 2e-9 * np.abs(w).max(1, keepdims=True))
+    assert np.array_equal(got["stat"][:, [0, 1, 3]], want["stat"][:, [0, 1, 3]])
+    ok = low > 2.0  # omega = 4 C6 / (3 alpha^2) of a difference carries its error
+    assert ok.sum() > 20
+    assert np.allclose(got["energy"][ok], want["energy"][ok], rtol=4e-9, atol=1e-11)
+    assert np.allclose(got["energy"], want["energy"], rtol=1e-6, atol=0, equal_nan=True)
