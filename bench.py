@@ -2,7 +2,7 @@
 
 One step = one full E_MBD evaluation (the span pmbd.x times around
 MBD_at_rsSCS, MBD_rsSCS.f90:220-222): SCS at 21 imaginary frequencies, C6 and
-omega sums, coupled-QHO matrix, all eigenvalues, energy.  The workload is the
+omega sums, coupled-QHO matrix and energy.  The workload is the
 4096-atom random periodic cell (38 A cube, C:H:N:O = 40:40:10:10, seeded; SCS
 cutoff 40 A, supercell 25 A, CFDM 100 A), so n_SCS = n_MBD = 12288.  The
 geometry is resident on the device before the timed region.
@@ -11,7 +11,7 @@ Forms timed in the same run: plain FP64 (FP64 tensors, FP64 MFMA Cholesky);
 mixed (FP32 tensors, FP32 MFMA Cholesky with FP64 refinement); learned
 (FP32 tensors, batched block-PCG over all 21 frequencies with the network's
 warm start when weights are loaded, gated on the FP64 residual with Cholesky
-fallback).  The eigen stage is FP64 in every form.  The headline value is the
+fallback).  The energy stage is FP64 in every form.  The headline value is the
 learned form; each form's errors against the FP64 form are reported.
 
 Prints one JSON line on stdout; progress goes to stderr.
@@ -84,7 +84,7 @@ def traffic_probe(args):
     """Workload of the hardware-counter runs: one 1 GiB copy with the plain
     copy kernel (the known-size reference), then one learned-form solve of the
     benchmark cell with every kernel launched eagerly (no graph replay), its
-    SCS stage, CFDM build and two-stage eigen reduction at n = 12288.  Meant to
+    SCS stage, CFDM build and energy stage at n = 12288.  Meant to
     run under rocprofv3 --pmc; prints progress and, per profiler class, the
     launches and algorithmic bytes of the solve (stderr) for the summary."""
     os.environ["MBD_TRD_GRAPH"] = "0"  # eager launches: one counter record per dispatch

@@ -108,9 +108,10 @@ int mbd_scs(mbd_handle *h, int mode, double *alpha_eff, double *coupled_pol,
             double *molpol_eig, double *c6_eff, double *c6_mol, mbd_diag *d);
 
 /* E_MBD from alpha_eff[n] and c6_eff[n] (UTILS.f90:700-879): builds the
- * coupled-QHO matrix over the supercell, all its eigenvalues in FP64, and
- * E = 1/2 sum_{l>=0} sqrt(l) / Ncell - 3/2 sum w.  omega[n], reff[n] may be
- * NULL.  Returns 0 or MBD_ERR_*; d->info_eig and d->n_negative report. */
+ * coupled-QHO matrix over the supercell and, in FP64,
+ * E = 1/2 sum_{l>=0} sqrt(l) / Ncell - 3/2 sum w, from log-determinants of
+ * shifted matrices where all eigenvalues l are proved positive, from the
+ * eigenvalues otherwise.  omega[n], reff[n] may be NULL.  Returns 0 or MBD_ERR_*; d->info_eig and d->n_negative report. */
 int mbd_energy(mbd_handle *h, const double *alpha_eff, const double *c6_eff,
                double *e_mbd, double *omega, double *reff, mbd_diag *d);
 
@@ -202,10 +203,12 @@ int mbd_debug_gemm_nt(int device, int fp32, int m, int n, int k,
                       double beta, double *C);
 
 /* ---- Batched molecules ----------------------------------------------------
- * Many independent non-periodic molecules solved together: every
- * (molecule, grid point) SCS problem and every molecule's coupled-QHO
+ * Many independent non-periodic molecules solved together.  Up to 32 atoms,
+ * every (molecule, grid point) SCS problem and every molecule's coupled-QHO
  * eigenproblem run in ONE persistent kernel launch, replayed from a captured
- * hipGraph.  Per molecule the results are what mbd_run returns for that
+ * hipGraph; for larger molecules every step is one launch over all of them,
+ * and those whose factor, refinement or lower spectrum fails there go through
+ * the persistent kernel.  Per molecule the results are what mbd_run returns for that
  * molecule alone (the reference runs one system per pmbd.x invocation:
  * MBD_rsSCS.f90:220-222 around MBD_at_rsSCS, UTILS.f90:153-349).
  * Modes: MBD_MODE_FP64, or MBD_MODE_MIXED (FP32 Cholesky, FP64 refinement
@@ -219,8 +222,8 @@ typedef struct {
   int n_failed;        /* molecules with a non-positive FP64 pivot */
   int n_negative;      /* negative coupled-QHO eigenvalues, all molecules */
   double max_residual; /* largest final max|B - A X| */
-  double t_ms;         /* device time of the replayed graph */
-  double phase_ms[6];  /* workgroup time summed over workgroups: relay build,
+  double t_ms;         /* device time of the pass */
+  double phase_ms[6];  /* persistent kernel, workgroup time summed over workgroups: relay build,
                           factorisation, solves + refinement, C6 + coupled-QHO
                           build, tridiagonalisation, bisection + energy */
 } mbd_batch_diag;

@@ -1,6 +1,6 @@
-// Batched MBD@rsSCS for many small non-periodic molecules: one persistent
-// launch solves every (molecule, frequency) SCS problem and then each
-// molecule's coupled-QHO eigenvalue problem and energy.
+// Batched MBD@rsSCS for small non-periodic molecules (mol.h has the larger
+// ones): one persistent launch solves every (molecule, frequency) SCS problem
+// and then each molecule's coupled-QHO eigenvalue problem and energy.
 #pragma once
 
 #include "common.h"

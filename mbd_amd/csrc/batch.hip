@@ -1,4 +1,5 @@
-// Batched MBD@rsSCS over many small non-periodic molecules in ONE persistent
+// Batched MBD@rsSCS over many small non-periodic molecules (larger ones reach
+// it only when mol.hip cannot finish them) in ONE persistent
 // launch (the reference handles one system per pmbd.x run; its per-system
 // steps are UTILS.f90:239-315 for SCS and C6 and UTILS.f90:700-879 for the
 // coupled-QHO energy).

@@ -241,7 +241,7 @@ struct mbd_handle {
   DevBuf<double> C, om_at, reff, lam, e2, bounds, E, VW, tau, dd, ee, alph, pa, pb, py, qred, ps;
   DevBuf<double> ext_alpha, ext_c6;
   DevBuf<int> nneg;
-  // batched molecules (one persistent launch, replayed from a hipGraph)
+  // batched molecules (small ones: one persistent launch, replayed from a hipGraph)
   struct Batch {
     int nmol = 0, natoms = 0, nmax = 0, ncu = 0;
     double beta = 1.0, rc_scs = 0.0, rc_cfdm = 0.0;  // bohr
