@@ -226,7 +226,9 @@ struct mbd_handle {
   DevBuf<int> info1, luPiv;
   // device: iterative (learned) form; preconditioner clusters of the system
   DevBuf<double> pMinv, pR, pZ, pP, pQ, pscal, ppart, alpha_pred;
-  Clusters cl;
+  Clusters cl;  // formed by the system's first iterative solve
+  bool cl_ready = false;
+  std::vector<double> xyz_h, hirsh_h;
   DevBuf<int> clOff, clAtoms;
   DevBuf<long> clMoff;
   // partials of the lower-triangle products (refinement residuals, block-PCG)
@@ -480,6 +482,26 @@ int solve_point_fp64(mbd_handle *h, int k, double *Xk) {
   return info;
 }
 
+// Atom clusters of the iterative solve's block preconditioner, formed on the
+// host while the device builds the relay matrices (formed with the system they
+// cost a 4096-atom learned solve 8 of 184 ms before its first launch, and the
+// other forms, which do not use them, as much).
+void system_clusters(mbd_handle *h) {
+  if (h->cl_ready) return;
+  h->cl = build_clusters(h->N, h->xyz_h.data(), h->lat, h->periodic != 0, h->hirsh_h.data(),
+                         h->a0_h.data(), h->r0_h.data(), h->beta);
+  h->clOff.ensure(h->cl.off.size());
+  h->clAtoms.ensure(h->cl.atoms.size());
+  h->clMoff.ensure(h->cl.moff.size());
+  MBD_HIP(hipMemcpyAsync(h->clOff.p, h->cl.off.data(), sizeof(int) * h->cl.off.size(),
+                         hipMemcpyHostToDevice, h->stream));
+  MBD_HIP(hipMemcpyAsync(h->clAtoms.p, h->cl.atoms.data(), sizeof(int) * h->cl.atoms.size(),
+                         hipMemcpyHostToDevice, h->stream));
+  MBD_HIP(hipMemcpyAsync(h->clMoff.p, h->cl.moff.data(), sizeof(long) * h->cl.moff.size(),
+                         hipMemcpyHostToDevice, h->stream));
+  h->cl_ready = true;
+}
+
 // SCS at all 21 points into h->alpha (21 x N), h->P (21 x 9), then C6.
 void run_scs(mbd_handle *h, int mode, mbd_diag *d) {
   const int N = h->N, n = h->n();
@@ -541,15 +563,12 @@ void run_scs(mbd_handle *h, int mode, mbd_diag *d) {
     const Symv3Sizes svz = symv3_sizes(n);
     h->svU.ensure((size_t)nb * svz.upart);
     h->svV.ensure((size_t)nb * svz.vpart);
-    const int npart = std::max(h->cl.n, ceil_div(n, 256));
     if (mode == MBD_MODE_LEARNED) {
-      h->pMinv.ensure((size_t)nb * h->cl.mtot);
       h->pR.ensure((size_t)nb * sX);
       h->pZ.ensure((size_t)nb * sX);
       h->pP.ensure((size_t)nb * sX);
       h->pQ.ensure((size_t)nb * sX);
       h->pscal.ensure((size_t)nb * kPcgScal);
-      h->ppart.ensure((size_t)nb * npart * 4);
     }
     if (mode == MBD_MODE_LEARNED && h->have_net) {
       // network warm start: descriptors and forward pass for every atom and
@@ -589,6 +608,10 @@ void run_scs(mbd_handle *h, int mode, mbd_diag *d) {
             redo.push_back(b);
         }
       } else {
+        system_clusters(h);
+        const int npart = std::max(h->cl.n, ceil_div(n, 256));
+        h->pMinv.ensure((size_t)nb * h->cl.mtot);
+        h->ppart.ensure((size_t)nb * npart * 4);
         PcgWork wk;
         wk.cl_off = h->clOff.p;
         wk.cl_atoms = h->clAtoms.p;
@@ -1291,17 +1314,11 @@ int mbd_set_system(mbd_handle *h, int n_atoms, const double *xyz, const double *
     }
     up(h->img_cfdm, tc.data(), tc.size());
     up(h->lat_d, h->lat, 9);
-    // atom clusters of the iterative solve's block preconditioner
-    h->cl = build_clusters(n_atoms, xyz, h->lat, h->periodic != 0, hirshfeld, alpha0, r0, beta);
-    h->clOff.ensure(h->cl.off.size());
-    h->clAtoms.ensure(h->cl.atoms.size());
-    h->clMoff.ensure(h->cl.moff.size());
-    MBD_HIP(hipMemcpyAsync(h->clOff.p, h->cl.off.data(), sizeof(int) * h->cl.off.size(),
-                           hipMemcpyHostToDevice, h->stream));
-    MBD_HIP(hipMemcpyAsync(h->clAtoms.p, h->cl.atoms.data(), sizeof(int) * h->cl.atoms.size(),
-                           hipMemcpyHostToDevice, h->stream));
-    MBD_HIP(hipMemcpyAsync(h->clMoff.p, h->cl.moff.data(), sizeof(long) * h->cl.moff.size(),
-                           hipMemcpyHostToDevice, h->stream));
+    h->xyz_h.assign(xyz, xyz + 3L * n_atoms);
+    h->hirsh_h.assign(hirshfeld, hirshfeld + n_atoms);
+    h->a0_h.assign(alpha0, alpha0 + n_atoms);
+    h->r0_h.assign(r0, r0 + n_atoms);
+    h->cl_ready = false;
     h->cell.ensure(cells.size());
     MBD_HIP(hipMemcpyAsync(h->cell.p, cells.data(), sizeof(int) * cells.size(),
                            hipMemcpyHostToDevice, h->stream));
