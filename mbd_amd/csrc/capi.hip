@@ -725,8 +725,8 @@ bool ritz_values(mbd_handle *h, const std::vector<LdGroup> &groups, double &lo, 
 // E_MBD of the matrices of `groups` by log-determinants into h->e_val; row r
 // belongs to atom (r % (3 N cells)) / (3 cells).  false, with nothing
 // decided, when they have an eigenvalue below 0.03 of the smallest omega^2
-// (negative ones among them), a value that is not finite, or no room for one
-// shifted matrix.
+// (negative ones among them), an omega that is not positive, a value that is
+// not finite, or no room for one shifted matrix.
 bool energy_by_logdet(mbd_handle *h, const std::vector<LdGroup> &groups, int cells) {
   hipStream_t s = h->stream;
   const int N = h->N;
@@ -754,7 +754,9 @@ bool energy_by_logdet(mbd_handle *h, const std::vector<LdGroup> &groups, int cel
     top = std::max(top, v);
   }
   for (double w : om) {
-    if (!std::isfinite(w)) return false;
+    // the log-determinants know omega^2 only: a negative omega (of a negative
+    // C6) would enter the sum of -3/2 omega with the wrong sign
+    if (!(w > 0.0) || !std::isfinite(w)) return false;
     w2min = std::min(w2min, w * w);
     w2max = std::max(w2max, w * w);
   }

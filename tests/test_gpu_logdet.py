@@ -151,3 +151,33 @@ def test_supercell_by_wave_vectors(edges, vac, skew, out, cells, launches, monke
     # blocks by cell difference and their transform, or the whole matrix
     assert prof["cfdm_build"]["launches"] == launches
     assert abs(got - want) <= tol
+
+
+# atoms whose C6, and with it omega = 4 C6 / (3 alpha^2), is negative or zero:
+# the energy's -3/2 sum omega takes it with its sign, in a molecule and in a
+# supercell
+@pytest.mark.parametrize("w", [-0.4, 0.0])
+@pytest.mark.parametrize("edge", [None, 13.0])
+def test_omega_not_positive(w, edge, monkeypatch):
+    geo = _spread(5, 3)
+    xyz = geo.coords_ang - geo.coords_ang.min(0)
+    geo = Geometry(geo.names, xyz, geo.hirshfeld, None if edge is None else np.diag([edge, 26.0, 27.0]))
+    st = Settings(mbd_supercell_cutoff=25.0, mbd_cfdm_dip_cutoff=30.0, mbd_scs_dip_cutoff=20.0)
+    cells = 1 if edge is None else 2
+    a = np.full(5, 3.0)
+    omega = np.array([0.5, 0.6, w, 0.55, 0.45])
+    with engine.MbdEngine(0) as eng:
+        eng.set_geometry(geo, st)
+        got, om, rf, d = eng.energy(a, 0.75 * omega * a * a)
+        monkeypatch.setenv("MBD_EIG_METHOD", "1")
+        by_eig = eng.energy(a, 0.75 * omega * a * a)[0]
+        monkeypatch.delenv("MBD_EIG_METHOD")
+        C = eng.cfdm_matrix(a, om, rf, cells)
+    lam = np.linalg.eigvalsh(np.tril(C) + np.tril(C, -1).T)
+    # a row of zeros (omega = 0) has eigenvalue 0 to rounding: either sign, no energy
+    want = 0.5 * np.sqrt(lam[lam >= 0]).sum() / cells - 1.5 * omega.sum()
+    assert np.allclose(om, omega, rtol=1e-15, atol=0)
+    # 15 cells square roots of eigenvalues good to 15 cells eps; sqrt(15 cells eps) at a zero one
+    tol = 2.2e-16 * 15 * cells * 1.5 * np.abs(om).sum() if w else 3.0 * np.sqrt(2.2e-16 * 15 * cells)
+    assert abs(got - want) <= tol
+    assert got == by_eig
