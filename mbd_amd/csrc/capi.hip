@@ -832,9 +832,14 @@ bool energy_by_logdet(mbd_handle *h, const std::vector<LdGroup> &groups, int cel
 // wave vector, (3 N cells)^3 operations fall to about cells (3 N)^3.  Taken
 // where the image box covers the cutoff sphere for every pair of atoms and
 // cells (h->cells_cover: then a block depends on the cells' difference
-// alone); false, with nothing decided, where an image lies on the sphere to
-// rounding or energy_by_logdet decides nothing.
-bool energy_by_cells(mbd_handle *h, const double *alpha_eff_d) {
+// alone).  kBlocks: an image lies on the sphere to rounding, the blocks cannot
+// be used; kSpectrum: energy_by_logdet decided nothing on them, and would not
+// on the whole matrix, which has the same eigenvalues (tried there too, a 2 x
+// 2 x 2 supercell of 64 atoms with negative eigenvalues took 22.0 ms instead
+// of 18.6, against 17.9 by eigenvalues alone; 3 x 3 x 3 cells of 27 atoms
+// 34.0, 27.3 and 26.5).
+enum class ByCells { kDone, kBlocks, kSpectrum };
+ByCells energy_by_cells(mbd_handle *h, const double *alpha_eff_d) {
   hipStream_t s = h->stream;
   const int N = h->N, n = h->n(), nc = h->ncell, *S = h->supercell;
   const size_t nn = (size_t)n * n;
@@ -880,11 +885,11 @@ bool energy_by_cells(mbd_handle *h, const double *alpha_eff_d) {
   int near = 0;
   MBD_HIP(hipMemcpyAsync(&near, h->cellNear.p, sizeof near, hipMemcpyDeviceToHost, s));
   MBD_HIP(hipStreamSynchronize(s));
-  if (near) return false;
+  if (near) return ByCells::kBlocks;
   std::vector<LdGroup> groups;
   if (nr) groups.push_back({n, nr, h->cellH.p});
   if (np) groups.push_back({2 * n, np, h->cellH.p + nr * nn});
-  return energy_by_logdet(h, groups, 1);
+  return energy_by_logdet(h, groups, 1) ? ByCells::kDone : ByCells::kSpectrum;
 }
 
 // E_MBD from device alpha_eff / c6_eff.
@@ -901,12 +906,17 @@ void run_energy(mbd_handle *h, const double *alpha_eff_d, const double *c6_d,
     for (int k = 0; k < 3; ++k) d->supercell[k] = h->supercell[k];
   }
   h->eig_flag = 0;
-  if (h->ncell > 1 && h->cells_cover && use_logdet() && energy_by_cells(h, alpha_eff_d)) return;
+  bool logdet = use_logdet();
+  if (h->ncell > 1 && h->cells_cover && logdet) {
+    const ByCells r = energy_by_cells(h, alpha_eff_d);
+    if (r == ByCells::kDone) return;
+    logdet = r == ByCells::kBlocks;
+  }
   h->C.ensure((size_t)nm * nm);
   cfdm_build(s, N, h->ncell, h->xyz.p, h->cell.p, h->lat_d.p, h->nimg_cfdm,
              h->nimg_cfdm / 2, h->img_cfdm.p, h->rc_cfdm / kBohr, h->beta,
              alpha_eff_d, h->om_at.p, h->reff.p, h->C.p, nm, false);
-  if (use_logdet() && nm <= kLdMaxOrder &&
+  if (logdet && nm <= kLdMaxOrder &&
       energy_by_logdet(h, {LdGroup{(int)nm, 1, h->C.p}}, h->ncell))
     return;
   TrdWork wk;

@@ -181,3 +181,26 @@ def test_omega_not_positive(w, edge, monkeypatch):
     tol = 2.2e-16 * 15 * cells * 1.5 * np.abs(om).sum() if w else 3.0 * np.sqrt(2.2e-16 * 15 * cells)
     assert abs(got - want) <= tol
     assert got == by_eig
+
+
+def test_supercell_with_negative_eigenvalues(monkeypatch):
+    """The wave vectors' matrices have the supercell's eigenvalues: what they
+    decline goes to the eigenvalues at once."""
+    rng = np.random.default_rng(2)
+    g = 3.25 * np.stack(np.meshgrid(*[np.arange(4)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    geo = Geometry(["C"] * 64, g + rng.uniform(0, 0.1, g.shape), np.full(64, 0.8), np.diag([13.0, 13.2, 13.3]))
+    st = Settings(mbd_supercell_cutoff=25.0, mbd_cfdm_dip_cutoff=60.0, mbd_scs_dip_cutoff=30.0)
+    a = np.full(64, 150.0)
+    with engine.MbdEngine(0) as eng:
+        eng.set_geometry(geo, st)
+        monkeypatch.setenv("MBD_EIG_METHOD", "2")  # the default method of order 1536
+        want, _, _, dw = eng.energy(a, 0.75 * 0.5 * a * a)
+        monkeypatch.delenv("MBD_EIG_METHOD")
+        eng.profile_enable(True)
+        got, _, _, dg = eng.energy(a, 0.75 * 0.5 * a * a)
+        prof = eng.profile_read()
+    assert dw["supercell"] == [2, 2, 2] and dg["n_negative"] == dw["n_negative"] > 0
+    # the wave vectors' matrices of order 192, two diagonal blocks in each of
+    # two attempts; the whole matrix of order 1536 would add twelve in each
+    assert 0 < prof["logdet_diag"]["launches"] <= 4 and prof["bisect"]["launches"] > 0
+    assert got == want
