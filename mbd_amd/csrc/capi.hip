@@ -679,6 +679,13 @@ void run_scs(mbd_handle *h, int mode, mbd_diag *d) {
 bool use_logdet() { return !getenv("MBD_EIG_METHOD"); }
 
 constexpr int kLzMinOrder = 7000;
+// From this n^3 (summed over the matrices) on, a guess of the lower end after
+// one that failed is proved before its nodes are factored: the matrix most
+// likely has an eigenvalue that is not positive.  Energies of matrices with
+// negative eigenvalues, nodes with their proof / proof first: order 2100 31.3 /
+// 30.3 ms, 3000 47.8 / 44.5, 6000 130 / 107, 6900 168 / 134; below, one matrix
+// takes about as long as all of them (order 900: 31.5 / 31.3).
+constexpr double kLdProofWork = 2048.0 * 2048.0 * 2048.0;
 void fetch(mbd_handle *h, double *dst, const double *src, size_t count);
 
 // `batch` symmetric matrices of order n (lower triangles, leading dimension
@@ -722,6 +729,65 @@ bool ritz_values(mbd_handle *h, const std::vector<LdGroup> &groups, double &lo, 
   return ld_ritz(v.data(), (int)(nab / (2 * kLzSteps)), lo, hi);
 }
 
+// Factors entries b0 ... b1 - 1 of `nd` for every matrix of `groups` and adds
+// the nodes' terms to e.  1: done; 0: a matrix is not positive definite; -1:
+// no room for one shifted matrix.
+int ld_factor(mbd_handle *h, const std::vector<LdGroup> &groups, int cells, const LdNodes &nd, int b0,
+              int b1, double &e) {
+  hipStream_t s = h->stream;
+  const size_t budget = mem_budget();
+  const int all = b1 - b0;
+  size_t nmat = 0;
+  for (const LdGroup &g : groups) nmat += (size_t)g.batch * all;
+  h->ldG.ensure(nmat);
+  h->ldInfo.ensure(nmat);
+  batch_zero(s, h->ldInfo.p, (int)nmat);
+  std::vector<int> node;  // of each factored matrix, in order
+  for (const LdGroup &g : groups) {
+    const int lda = lead_dim(g.n);
+    const long sH = (long)g.n * g.n, sA = (long)g.n * lda,
+               sinv = (long)ceil_div(g.n, kCholNB) * kCholNB * kCholNB;
+    const size_t one = 8 * (size_t)(sA + sinv);
+    // shifted matrices per pass: the SCS stage's memory budget, and what is free
+    size_t fit = std::min<size_t>(budget / one, (size_t)g.batch * all);
+    if (fit < 1) return -1;
+    if (h->A64.n < fit * sA || h->inv64.n < fit * sinv) {
+      size_t freeb = 0, total = 0;
+      MBD_HIP(hipMemGetInfo(&freeb, &total));
+      fit = std::min(fit, (freeb / 10 * 9 + 8 * (h->A64.n + h->inv64.n)) / one);
+      if (fit < 1) return -1;
+      try {
+        h->A64.ensure(fit * sA);
+        h->inv64.ensure(fit * sinv);
+      } catch (const HipError &x) {
+        if (x.err != hipErrorOutOfMemory) throw;
+        (void)hipGetLastError();
+        return -1;
+      }
+    }
+    const int rb = std::max<int>(1, (int)(fit / all)), nbmax = std::min<int>((int)fit, all);
+    for (int r0 = 0; r0 < g.batch; r0 += rb)
+      for (int q0 = b0; q0 < b1; q0 += nbmax) {
+        const int rn = std::min(rb, g.batch - r0), nb = std::min(nbmax, b1 - q0);
+        const size_t m0 = node.size();
+        ld_shift(s, g.n, g.H + r0 * sH, g.n, sH, rn, nd, q0, nb, h->A64.p, lda, sA);
+        potrf_batched<double>(s, g.n, h->A64.p, lda, sA, rn * nb, h->inv64.p, sinv,
+                              h->ldInfo.p + m0, true);
+        ld_sums(s, g.n, h->A64.p, lda, sA, rn, nd, q0, nb, h->om_at.p, h->N, cells, h->ldG.p + m0);
+        for (int m = 0; m < rn * nb; ++m) node.push_back(q0 + m % nb);
+      }
+  }
+  std::vector<double> g(node.size());
+  std::vector<int> info(node.size());
+  MBD_HIP(hipMemcpyAsync(g.data(), h->ldG.p, 8 * g.size(), hipMemcpyDeviceToHost, s));
+  MBD_HIP(hipMemcpyAsync(info.data(), h->ldInfo.p, 4 * g.size(), hipMemcpyDeviceToHost, s));
+  MBD_HIP(hipStreamSynchronize(s));
+  if (std::any_of(info.begin(), info.end(), [](int i) { return i != 0; })) return 0;
+  for (size_t m = 0; m < g.size(); ++m)
+    if (node[m] < nd.n) e += nd.w[node[m]] * g[m];
+  return 1;
+}
+
 // E_MBD of the matrices of `groups` by log-determinants into h->e_val; row r
 // belongs to atom (r % (3 N cells)) / (3 cells).  false, with nothing
 // decided, when they have an eigenvalue below 0.03 of the smallest omega^2
@@ -730,15 +796,13 @@ bool ritz_values(mbd_handle *h, const std::vector<LdGroup> &groups, double &lo, 
 bool energy_by_logdet(mbd_handle *h, const std::vector<LdGroup> &groups, int cells) {
   hipStream_t s = h->stream;
   const int N = h->N;
-  const size_t budget = mem_budget();
-  long nhi = 0, nmat = 0;
+  long nhi = 0;
+  double work = 0.0;  // n^3 over the matrices
   for (const LdGroup &g : groups) {
     nhi += (long)g.batch * ceil_div(g.n, 64);
-    nmat += (long)g.batch * (kLdMaxNodes + 1);
+    work += g.batch * (double)g.n * g.n * g.n;
   }
   h->ldHi.ensure(nhi);
-  h->ldG.ensure(nmat);
-  h->ldInfo.ensure(nmat);
   std::vector<double> hi(nhi), om(N);
   long at = 0;
   for (const LdGroup &g : groups) {
@@ -764,65 +828,34 @@ bool energy_by_logdet(mbd_handle *h, const std::vector<LdGroup> &groups, int cel
   // the smallest eigenvalue is 0.38 (graphene) to 0.97 (water) of the
   // smallest omega^2 on the reference's examples and the benchmark's systems
   std::vector<std::pair<double, double>> guess = {{0.3 * w2min, top}, {0.03 * w2min, top}};
-  double rlo, rhi;
+  double rlo, rhi, above = INFINITY;  // the smallest eigenvalue is not above this
   if (ritz_values(h, groups, rlo, rhi)) {
     if (rlo <= 0.0) return false;  // an eigenvalue is not positive
+    above = rlo;
     const double up = std::max(w2max, std::min(top, rhi + 0.2 * (rhi - rlo)));
     guess.insert(guess.begin(), {0.65 * std::min(rlo, w2min), up});
   }
+  bool failed = false;
   for (const auto &[lo, up] : guess) {
+    if (lo >= above) continue;  // its proof cannot hold
     LdNodes nd;
     if (!ld_nodes(lo, up, nd)) return false;
-    const int all = nd.n + 1;
-    batch_zero(s, h->ldInfo.p, (int)nmat);
-    std::vector<int> node;  // of each factored matrix, in order
-    for (const LdGroup &g : groups) {
-      const int lda = lead_dim(g.n);
-      const long sH = (long)g.n * g.n, sA = (long)g.n * lda,
-                 sinv = (long)ceil_div(g.n, kCholNB) * kCholNB * kCholNB;
-      const size_t one = 8 * (size_t)(sA + sinv);
-      // shifted matrices per pass: the SCS stage's memory budget, and what is free
-      size_t fit = std::min<size_t>(budget / one, (size_t)g.batch * all);
-      if (fit < 1) return false;
-      if (h->A64.n < fit * sA || h->inv64.n < fit * sinv) {
-        size_t freeb = 0, total = 0;
-        MBD_HIP(hipMemGetInfo(&freeb, &total));
-        fit = std::min(fit, (freeb / 10 * 9 + 8 * (h->A64.n + h->inv64.n)) / one);
-        if (fit < 1) return false;
-        try {
-          h->A64.ensure(fit * sA);
-          h->inv64.ensure(fit * sinv);
-        } catch (const HipError &e) {
-          if (e.err != hipErrorOutOfMemory) throw;
-          (void)hipGetLastError();
-          return false;
-        }
-      }
-      const int rb = std::max<int>(1, (int)(fit / all)), nbmax = std::min<int>((int)fit, all);
-      for (int r0 = 0; r0 < g.batch; r0 += rb)
-        for (int b0 = 0; b0 < all; b0 += nbmax) {
-          const int rn = std::min(rb, g.batch - r0), nb = std::min(nbmax, all - b0);
-          const size_t m0 = node.size();
-          ld_shift(s, g.n, g.H + r0 * sH, g.n, sH, rn, nd, b0, nb, h->A64.p, lda, sA);
-          potrf_batched<double>(s, g.n, h->A64.p, lda, sA, rn * nb, h->inv64.p, sinv,
-                                h->ldInfo.p + m0, true);
-          ld_sums(s, g.n, h->A64.p, lda, sA, rn, nd, b0, nb, h->om_at.p, N, cells, h->ldG.p + m0);
-          for (int m = 0; m < rn * nb; ++m) node.push_back(b0 + m % nb);
-        }
-    }
-    std::vector<double> g(node.size());
-    std::vector<int> info(node.size());
-    MBD_HIP(hipMemcpyAsync(g.data(), h->ldG.p, 8 * g.size(), hipMemcpyDeviceToHost, s));
-    MBD_HIP(hipMemcpyAsync(info.data(), h->ldInfo.p, 4 * g.size(), hipMemcpyDeviceToHost, s));
-    MBD_HIP(hipStreamSynchronize(s));
-    if (std::any_of(info.begin(), info.end(), [](int i) { return i != 0; })) continue;
     double e = 0.0;
-    for (size_t m = 0; m < g.size(); ++m)
-      if (node[m] < nd.n) e += nd.w[node[m]] * g[m];
-    if (!std::isfinite(e)) return false;
-    h->e_val = e / h->ncell;
-    h->n_neg = 0;
-    return true;
+    int pd = 1;
+    if (failed && work >= kLdProofWork) {
+      pd = ld_factor(h, groups, cells, nd, nd.n, nd.n + 1, e);
+      if (pd > 0) pd = ld_factor(h, groups, cells, nd, 0, nd.n, e);
+    } else {
+      pd = ld_factor(h, groups, cells, nd, 0, nd.n + 1, e);
+    }
+    if (pd < 0 || !std::isfinite(e)) return false;
+    if (pd) {
+      h->e_val = e / h->ncell;
+      h->n_neg = 0;
+      return true;
+    }
+    above = lo;
+    failed = true;
   }
   return false;
 }

@@ -204,3 +204,25 @@ def test_supercell_with_negative_eigenvalues(monkeypatch):
     # two attempts; the whole matrix of order 1536 would add twelve in each
     assert 0 < prof["logdet_diag"]["launches"] <= 4 and prof["bisect"]["launches"] > 0
     assert got == want
+
+
+def test_second_guess_proved_first(monkeypatch):
+    """A matrix of order 3000 with negative eigenvalues: the nodes of the first
+    guess are factored, of the second only its proof."""
+    geo = _spread(1000, 7)
+    a = np.full(1000, 60.0)
+    with engine.MbdEngine(0) as eng:
+        eng.set_geometry(geo, Settings())
+        monkeypatch.setenv("MBD_EIG_METHOD", "2")
+        want, _, _, dw = eng.energy(a, 0.75 * 0.5 * a * a)
+        monkeypatch.delenv("MBD_EIG_METHOD")
+        eng.profile_enable(True)
+        got, _, _, dg = eng.energy(a, 0.75 * 0.5 * a * a)
+        prof = eng.profile_read()
+    assert dg["n_negative"] == dw["n_negative"] > 0
+    assert got == want
+    # trailing updates are n^3 / 3 operations less the blocks' own per matrix;
+    # the nodes of one set are at most 13 (interval ends up to 0.3 : 12) and
+    # those of the second at least 12 (0.03 : 1)
+    mats = prof["logdet_syrk_gemm"]["flops"] / (3000.0 ** 3 / 3.0)
+    assert 8 < mats <= 15
