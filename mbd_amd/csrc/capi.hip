@@ -680,11 +680,15 @@ bool use_logdet() { return !getenv("MBD_EIG_METHOD"); }
 
 constexpr int kLzMinOrder = 7000;
 // From this n^3 (summed over the matrices) on, a guess of the lower end after
-// one that failed is proved before its nodes are factored: the matrix most
-// likely has an eigenvalue that is not positive.  Energies of matrices with
-// negative eigenvalues, nodes with their proof / proof first: order 2100 31.3 /
-// 30.3 ms, 3000 47.8 / 44.5, 6000 130 / 107, 6900 168 / 134; below, one matrix
-// takes about as long as all of them (order 900: 31.5 / 31.3).
+// one that failed is proved before its nodes are factored (the matrix most
+// likely has an eigenvalue that is not positive), and a set's products end
+// once its proof has failed.  Energies of matrices with negative eigenvalues
+// (a factorisation of order 3000 fails at row 231), without either / proof
+// first / both / by eigenvalues alone: order 2100 31.3 / 30.3 / 27.8 / 25.1
+// ms, 3000 47.8 / 44.5 / 40.1 / 36.3, 6000 130 / 107 / 85 / 77, 6900 168 / 134
+// / 101 / 92.  Below, one matrix takes about as long as a set (order 900: 31.5
+// / 31.3 / 30.7 / 29.2), and the products' look at the proof 1 % of a
+// molecule of order 1584.
 constexpr double kLdProofWork = 2048.0 * 2048.0 * 2048.0;
 void fetch(mbd_handle *h, double *dst, const double *src, size_t count);
 
@@ -729,6 +733,13 @@ bool ritz_values(mbd_handle *h, const std::vector<LdGroup> &groups, double &lo, 
   return ld_ritz(v.data(), (int)(nab / (2 * kLzSteps)), lo, hi);
 }
 
+// n^3 over the matrices.
+double ld_work(const std::vector<LdGroup> &groups) {
+  double w = 0.0;
+  for (const LdGroup &g : groups) w += g.batch * (double)g.n * g.n * g.n;
+  return w;
+}
+
 // Factors entries b0 ... b1 - 1 of `nd` for every matrix of `groups` and adds
 // the nodes' terms to e.  1: done; 0: a matrix is not positive definite; -1:
 // no room for one shifted matrix.
@@ -739,6 +750,7 @@ int ld_factor(mbd_handle *h, const std::vector<LdGroup> &groups, int cells, cons
   const int all = b1 - b0;
   size_t nmat = 0;
   for (const LdGroup &g : groups) nmat += (size_t)g.batch * all;
+  const double work = ld_work(groups);
   h->ldG.ensure(nmat);
   h->ldInfo.ensure(nmat);
   batch_zero(s, h->ldInfo.p, (int)nmat);
@@ -772,7 +784,7 @@ int ld_factor(mbd_handle *h, const std::vector<LdGroup> &groups, int cells, cons
         const size_t m0 = node.size();
         ld_shift(s, g.n, g.H + r0 * sH, g.n, sH, rn, nd, q0, nb, h->A64.p, lda, sA);
         potrf_batched<double>(s, g.n, h->A64.p, lda, sA, rn * nb, h->inv64.p, sinv,
-                              h->ldInfo.p + m0, true);
+                              h->ldInfo.p + m0, true, work >= kLdProofWork && q0 + nb == nd.n + 1 ? nb : 0);
         ld_sums(s, g.n, h->A64.p, lda, sA, rn, nd, q0, nb, h->om_at.p, h->N, cells, h->ldG.p + m0);
         for (int m = 0; m < rn * nb; ++m) node.push_back(q0 + m % nb);
       }
@@ -797,11 +809,7 @@ bool energy_by_logdet(mbd_handle *h, const std::vector<LdGroup> &groups, int cel
   hipStream_t s = h->stream;
   const int N = h->N;
   long nhi = 0;
-  double work = 0.0;  // n^3 over the matrices
-  for (const LdGroup &g : groups) {
-    nhi += (long)g.batch * ceil_div(g.n, 64);
-    work += g.batch * (double)g.n * g.n * g.n;
-  }
+  for (const LdGroup &g : groups) nhi += (long)g.batch * ceil_div(g.n, 64);
   h->ldHi.ensure(nhi);
   std::vector<double> hi(nhi), om(N);
   long at = 0;
@@ -842,7 +850,7 @@ bool energy_by_logdet(mbd_handle *h, const std::vector<LdGroup> &groups, int cel
     if (!ld_nodes(lo, up, nd)) return false;
     double e = 0.0;
     int pd = 1;
-    if (failed && work >= kLdProofWork) {
+    if (failed && ld_work(groups) >= kLdProofWork) {
       pd = ld_factor(h, groups, cells, nd, nd.n, nd.n + 1, e);
       if (pd > 0) pd = ld_factor(h, groups, cells, nd, 0, nd.n, e);
     } else {

@@ -268,10 +268,14 @@ __global__ __launch_bounds__(256) void k_potrf_diag_mols(int k0, const MolInfo *
                    inv + mi.inv + z.slot * mol_inv_size(mi.n) + (long)k0 * kCholNB, info + blockIdx.x);
 }
 
+// energy: matrices of log-determinants.  proof > 0: of every `proof`
+// consecutive ones the others are useless if the last is not positive definite,
+// and their products are left out once it has shown that.
 template <typename T>
 void potrf_batched(hipStream_t s, int n, T *A, int lda, long sA, int batch,
-                   T *inv, long sinv_blk, int *info, bool energy) {
-  const int NB = kCholNB;
+                   T *inv, long sinv_blk, int *info, bool energy, int proof) {
+  const int NB = kCholNB, per = std::max(1, proof);
+  const int *stop = proof ? info : nullptr;
   const size_t smem = sizeof(DiagLds<T>);
   static bool attr_set = false;
   if (!attr_set) {
@@ -301,14 +305,14 @@ void potrf_batched(hipStream_t s, int n, T *A, int lda, long sA, int batch,
       {
         ProfScope ps(energy ? K_LD_TRSM : K_CHOL_TRSM, s, 0.0, batch * (double)m2 * kb * kb);
         gemm_nt(s, false, m2, kb, kb, T(1), A21, lda, sA, invk, NB, sinv_blk,
-                T(0), A21, lda, sA, batch);
+                T(0), A21, lda, sA, batch, stop, per);
       }
       // the rest of the outer block's columns, on and below the diagonal
       const int w2 = o1 - k1;
       if (w2 > 0) {
         ProfScope ps(energy ? K_LD_SYRK : K_CHOL_SYRK, s, 0.0, batch * (double)kb * w2 * (2.0 * m2 - w2 + 1.0));
         gemm_nt(s, true, m2, w2, kb, T(-1), A21, lda, sA, A21, lda, sA, T(1),
-                A + k1 + (long)k1 * lda, lda, sA, batch);
+                A + k1 + (long)k1 * lda, lda, sA, batch, stop, per);
       }
     }
     // trailing A22 -= A21 A21^T on the lower triangle, A21 the outer block's
@@ -318,7 +322,7 @@ void potrf_batched(hipStream_t s, int n, T *A, int lda, long sA, int batch,
     const T *A21 = A + o1 + (long)o0 * lda;
     ProfScope ps(energy ? K_LD_SYRK : K_CHOL_SYRK, s, 0.0, batch * (double)m2 * (m2 + 1.0) * (o1 - o0));
     gemm_nt(s, true, m2, m2, o1 - o0, T(-1), A21, lda, sA, A21, lda, sA, T(1),
-            A + o1 + (long)o1 * lda, lda, sA, batch);
+            A + o1 + (long)o1 * lda, lda, sA, batch, stop, per);
   }
 }
 
@@ -347,9 +351,9 @@ template void potrf_mols<float>(hipStream_t, int, const MolInfo *, const MolMat 
                                 const std::function<int(int)> &, float *, float *, int *);
 
 template void potrf_batched<double>(hipStream_t, int, double *, int, long,
-                                    int, double *, long, int *, bool);
+                                    int, double *, long, int *, bool, int);
 template void potrf_batched<float>(hipStream_t, int, float *, int, long, int,
-                                   float *, long, int *, bool);
+                                   float *, long, int *, bool, int);
 
 // ---------------------------------------------------------------------------
 // Triangular solves with NRHS = 3, X column-major n x 3 (ldx) per matrix,

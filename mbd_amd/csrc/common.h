@@ -47,13 +47,17 @@ struct MatBatch {
 
 // C[m x n] = alpha * A[m x k] * B[n x k]^T + beta * C, batched over
 // blockIdx.z; lower != 0 restricts to tiles that touch the lower triangle
-// (row tile >= column tile), for symmetric rank-k updates.
+// (row tile >= column tile), for symmetric rank-k updates.  With stop (device,
+// one entry per matrix; tall-skinny single products do not look at it), `per`
+// consecutive matrices are left as they are where the last one's entry is set.
 void gemm_nt(hipStream_t s, bool lower, int m, int n, int k, double alpha,
              const double *A, int lda, long sA, const double *B, int ldb,
-             long sB, double beta, double *C, int ldc, long sC, int batch);
+             long sB, double beta, double *C, int ldc, long sC, int batch,
+             const int *stop = nullptr, int per = 1);
 void gemm_nt(hipStream_t s, bool lower, int m, int n, int k, float alpha,
              const float *A, int lda, long sA, const float *B, int ldb,
-             long sB, float beta, float *C, int ldc, long sC, int batch);
+             long sB, float beta, float *C, int ldc, long sC, int batch,
+             const int *stop = nullptr, int per = 1);
 // C = alpha (A1 B1^T + A2 B2^T) + beta C for n <= 32 columns and k <= 128
 // (A2, B2 may be null); column-major, A1 and A2 with lda, B1 and B2 with ldb.
 void gemm_ts2(hipStream_t s, int m, int n, int k, double alpha, const double *A1, const double *B1,

@@ -242,7 +242,8 @@ template <typename T, bool LOWER, bool GEN>
 __global__ __launch_bounds__(NT, 2) void k_gemm_nt(
     int m, int n, int k, T alpha, const T *__restrict__ A, int lda, long sA,
     const T *__restrict__ B, int ldb, long sB, T beta, T *__restrict__ C,
-    int ldc, long sC, int tiles_n, int ta, int tb) {
+    int ldc, long sC, int tiles_n, int ta, int tb, const int *stop, int per) {
+  if (stop && stop[(blockIdx.z / per + 1) * per - 1]) return;
   int tm, tn;
   const int idx = blockIdx.x;
   if (LOWER && idx < tiles_n * (tiles_n + 1) / 2) {
@@ -376,7 +377,8 @@ __global__ __launch_bounds__(256) void k_gemm_ts(int m, int n, int k, double alp
 template <typename T>
 void launch(hipStream_t s, bool lower, int m, int n, int k, T alpha,
             const T *A, int lda, long sA, const T *B, int ldb, long sB,
-            T beta, T *C, int ldc, long sC, int batch, int ta = 0, int tb = 0) {
+            T beta, T *C, int ldc, long sC, int batch, int ta = 0, int tb = 0,
+            const int *stop = nullptr, int per = 1) {
   if (m <= 0 || n <= 0 || batch <= 0) return;
   const int tmn = ceil_div(m, BM), tnn = ceil_div(n, BN);
   const bool gen = ta || tb || m < Vec16<T>::n || n < Vec16<T>::n;
@@ -384,7 +386,7 @@ void launch(hipStream_t s, bool lower, int m, int n, int k, T alpha,
   auto *f = lower ? (gen ? k_gemm_nt<T, true, true> : k_gemm_nt<T, true, false>)
                   : (gen ? k_gemm_nt<T, false, true> : k_gemm_nt<T, false, false>);
   hipLaunchKernelGGL(f, grid, dim3(NT), 0, s, m, n, k, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc,
-                     sC, tnn, ta, tb);
+                     sC, tnn, ta, tb, stop, per);
   MBD_LAUNCH_CHECK();
 }
 
@@ -419,20 +421,20 @@ template void gemm_mols<float>(hipStream_t, bool, int, int, int, const MolInfo *
 
 void gemm_nt(hipStream_t s, bool lower, int m, int n, int k, double alpha,
              const double *A, int lda, long sA, const double *B, int ldb,
-             long sB, double beta, double *C, int ldc, long sC, int batch) {
+             long sB, double beta, double *C, int ldc, long sC, int batch, const int *stop, int per) {
   if (!lower && batch == 1 && n <= TS_N && k >= 1 && k <= TS_K) {
     gemm_ts2(s, m, n, k, alpha, A, B, nullptr, nullptr, lda, ldb, beta, C, ldc);
     return;
   }
   launch<double>(s, lower, m, n, k, alpha, A, lda, sA, B, ldb, sB, beta, C,
-                 ldc, sC, batch);
+                 ldc, sC, batch, 0, 0, stop, per);
 }
 
 void gemm_nt(hipStream_t s, bool lower, int m, int n, int k, float alpha,
              const float *A, int lda, long sA, const float *B, int ldb,
-             long sB, float beta, float *C, int ldc, long sC, int batch) {
+             long sB, float beta, float *C, int ldc, long sC, int batch, const int *stop, int per) {
   launch<float>(s, lower, m, n, k, alpha, A, lda, sA, B, ldb, sB, beta, C,
-                ldc, sC, batch);
+                ldc, sC, batch, 0, 0, stop, per);
 }
 
 }  // namespace mbd

@@ -38,7 +38,7 @@ void cell_dft(hipStream_t s, int n, int ncell, int nreal, int npair, const doubl
 // chol.hip
 template <typename T>
 void potrf_batched(hipStream_t s, int n, T *A, int lda, long sA, int batch,
-                   T *inv, long sinv_blk, int *info, bool energy = false);
+                   T *inv, long sinv_blk, int *info, bool energy = false, int proof = 0);
 template <typename T>
 void potrs3_batched(hipStream_t s, int n, const T *L, int lda, long sA,
                     int batch, const T *inv, long sinv_blk, double *X, int ldx,

@@ -226,3 +226,35 @@ def test_second_guess_proved_first(monkeypatch):
     # those of the second at least 12 (0.03 : 1)
     mats = prof["logdet_syrk_gemm"]["flops"] / (3000.0 ** 3 / 3.0)
     assert 8 < mats <= 15
+
+
+# a set of shifted matrices is left at the first pivot that is not positive: at
+# row 231 of 3000 (by numpy's factorisation), and at row 778 of 780, where
+# everything before it is factored; the handle's next energy is whole again
+@pytest.mark.parametrize("case", ["early", "last"])
+def test_set_left_at_first_bad_pivot(case, monkeypatch):
+    if case == "early":
+        n, alpha, method, geo = 1000, 60.0, "2", _spread(1000, 7)
+    else:
+        n, alpha, method, geo = 260, 30.0, "1", _spread(260, 4, gap=4.0)
+        xyz = geo.coords_ang
+        xyz[-1] = xyz[-2] + [0.3, 0.0, 0.0]
+        geo = Geometry(["C"] * n, xyz, np.full(n, 0.95), None)
+    low, a = np.full(n, 4.0), np.full(n, alpha)
+    with engine.MbdEngine(0) as eng:
+        eng.set_geometry(geo, Settings())
+        eng.profile_enable(True)
+        good = eng.energy(low, 0.75 * 0.5 * low * low)[0]
+        whole = eng.profile_read()
+        monkeypatch.setenv("MBD_EIG_METHOD", method)
+        want, om, rf, dw = eng.energy(a, 0.75 * 0.5 * a * a)
+        monkeypatch.delenv("MBD_EIG_METHOD")
+        eng.profile_enable(True)
+        got, _, _, dg = eng.energy(a, 0.75 * 0.5 * a * a)
+        prof = eng.profile_read()
+        again = eng.energy(low, 0.75 * 0.5 * low * low)[0]
+    assert dg["n_negative"] == dw["n_negative"] > 0
+    assert got == want and again == good
+    assert whole["bisect"]["launches"] == 0 and prof["bisect"]["launches"] > 0
+    if case == "early":  # both guesses together take less than half of one whole set
+        assert prof["logdet_syrk_gemm"]["ms"] < 0.5 * whole["logdet_syrk_gemm"]["ms"]
