@@ -14,6 +14,7 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <numeric>
 #include <string>
 #include <vector>
 
@@ -288,7 +289,7 @@ struct mbd_handle {
   DevBuf<int> ldInfo;
   // supercells by cell differences: blocks, their Fourier transform, phases
   DevBuf<double> cellB, cellH, cellPh;
-  DevBuf<int> cellNear;
+  DevBuf<int> cellNear, cellK;
   bool cells_cover = false;  // the image box covers the cutoff sphere for every pair
   // result of the last run_energy
   double e_val = 0.0;
@@ -885,44 +886,39 @@ ByCells energy_by_cells(mbd_handle *h, const double *alpha_eff_d) {
   const int N = h->N, n = h->n(), nc = h->ncell, *S = h->supercell;
   const size_t nn = (size_t)n * n;
   // wave vectors k = -k, then one of each pair
-  std::vector<int> real, pair;
+  std::vector<int> kv, pair;
   auto index = [&](int i, int j, int k) { return (k * S[1] + j) * S[0] + i; };
-  std::vector<int> kv(3 * (size_t)nc);
   for (int k = 0; k < S[2]; ++k)
     for (int j = 0; j < S[1]; ++j)
       for (int i = 0; i < S[0]; ++i) {
         const int q = index(i, j, k);
         const int m = index((S[0] - i) % S[0], (S[1] - j) % S[1], (S[2] - k) % S[2]);
-        kv[3 * q] = i;
-        kv[3 * q + 1] = j;
-        kv[3 * q + 2] = k;
         if (m == q)
-          real.push_back(q);
+          kv.insert(kv.end(), {i, j, k});
         else if (q < m)
-          pair.push_back(q);
+          pair.insert(pair.end(), {i, j, k});
       }
-  const int nr = (int)real.size(), np = (int)pair.size();
-  std::vector<double> ph((size_t)(nr + 2 * np) * nc);
-  for (int w = 0; w < nr + np; ++w) {
-    const int q = w < nr ? real[w] : pair[w - nr];
-    for (int a = 0; a < nc; ++a) {
-      // the cells are numbered alike (c3 S2 S1 + c2 S1 + c1)
-      double t = 0.0;
-      for (int x = 0; x < 3; ++x) t += (double)((kv[3 * q + x] * kv[3 * a + x]) % S[x]) / S[x];
-      ph[(size_t)w * nc + a] = std::cos(2.0 * kPi * t);
-      if (w >= nr) ph[(size_t)(w + np) * nc + a] = std::sin(2.0 * kPi * t);
-    }
+  const int nr = (int)kv.size() / 3, np = (int)pair.size() / 3;
+  kv.insert(kv.end(), pair.begin(), pair.end());
+  const int L = std::lcm(S[0], std::lcm(S[1], S[2]));
+  std::vector<double> cs(2 * (size_t)L);
+  for (int m = 0; m < L; ++m) {
+    cs[m] = std::cos(2.0 * kPi * m / L);
+    cs[L + m] = std::sin(2.0 * kPi * m / L);
   }
-  h->cellPh.ensure(ph.size());
+  h->cellPh.ensure(cs.size() + (size_t)(nr + 2 * np) * nc);
+  h->cellK.ensure(kv.size());
   h->cellB.ensure(nc * nn);
   h->cellH.ensure((nr + 4 * (size_t)np) * nn);
   h->cellNear.ensure(1);
-  MBD_HIP(hipMemcpyAsync(h->cellPh.p, ph.data(), 8 * ph.size(), hipMemcpyHostToDevice, s));
+  MBD_HIP(hipMemcpyAsync(h->cellPh.p, cs.data(), 8 * cs.size(), hipMemcpyHostToDevice, s));
+  MBD_HIP(hipMemcpyAsync(h->cellK.p, kv.data(), sizeof(int) * kv.size(), hipMemcpyHostToDevice, s));
   batch_zero(s, h->cellNear.p, 1);
   cfdm_cells(s, N, nc, h->xyz.p, h->cell.p, h->lat_d.p, h->nimg_cfdm, h->nimg_cfdm / 2, h->img_cfdm.p,
              h->rc_cfdm / kBohr, h->beta, alpha_eff_d, h->om_at.p, h->reff.p, h->cellB.p,
              h->cellNear.p);
-  cell_dft(s, n, nc, nr, np, h->cellPh.p, h->cellB.p, h->cellH.p, h->cellH.p + nr * nn);
+  cell_dft(s, n, S, L, nr, np, h->cellK.p, h->cellPh.p, h->cellPh.p + 2 * L, h->cellB.p, h->cellH.p,
+           h->cellH.p + nr * nn);
   int near = 0;
   MBD_HIP(hipMemcpyAsync(&near, h->cellNear.p, sizeof near, hipMemcpyDeviceToHost, s));
   MBD_HIP(hipStreamSynchronize(s));
@@ -1214,6 +1210,7 @@ int mbd_destroy(mbd_handle *h) {
   h->cellH.release();
   h->cellPh.release();
   h->cellNear.release();
+  h->cellK.release();
   batch_release(h);
   if (h->trd_exec) (void)hipGraphExecDestroy(h->trd_exec);
   if (h->stream2) (void)hipStreamSynchronize(h->stream2);

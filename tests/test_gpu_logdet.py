@@ -258,3 +258,31 @@ def test_set_left_at_first_bad_pivot(case, monkeypatch):
     assert whole["bisect"]["launches"] == 0 and prof["bisect"]["launches"] > 0
     if case == "early":  # both guesses together take less than half of one whole set
         assert prof["logdet_syrk_gemm"]["ms"] < 0.5 * whole["logdet_syrk_gemm"]["ms"]
+
+
+# primitive cells, many short axes with different numbers of cells: tens to
+# over a thousand wave vectors of order 3, 6 and 60
+@pytest.mark.parametrize("n,edge,cells", [(1, 2.5, [11, 10, 11]), (2, 4.6, [6, 6, 6]), (20, 7.6, [4, 4, 4])])
+def test_primitive_cells(n, edge, cells, monkeypatch):
+    rng = np.random.default_rng(n)
+    m = int(np.ceil(n ** (1 / 3)))
+    g = np.stack(np.meshgrid(*[np.arange(m)] * 3, indexing="ij"), -1).reshape(-1, 3)[:n] * edge / m
+    lat = np.diag([0.998 * edge, 1.003 * edge, 0.997 * edge])
+    geo = Geometry(["H" if n == 1 else "Ar"] * n, g + rng.uniform(0, 0.1, g.shape), np.full(n, 0.8), lat)
+    st = Settings(mbd_supercell_cutoff=25.0, mbd_cfdm_dip_cutoff=60.0, mbd_scs_dip_cutoff=20.0)
+    a = np.full(n, 2.0)
+    with engine.MbdEngine(0) as eng:
+        eng.set_geometry(geo, st)
+        times = {}
+        for method in ("2" if 3 * n * np.prod(cells) >= 1024 else "1", None):
+            if method:
+                monkeypatch.setenv("MBD_EIG_METHOD", method)
+            for _ in range(2):  # the first pass allocates
+                e, om, _, d = eng.energy(a, 0.75 * 0.5 * a * a)
+            times[method] = (e, d["t_mbd_ms"])
+            if method:
+                monkeypatch.delenv("MBD_EIG_METHOD")
+    (want, t_eig), (got, t_cells) = times.values()
+    assert d["supercell"] == cells
+    assert abs(got - want) <= 2.2e-16 * 3 * n * np.prod(cells) * 1.5 * np.sum(om)
+    assert t_cells < t_eig
