@@ -137,6 +137,14 @@ def test_tuner_mixed_over_every_shape():
         assert float(np.abs(got["energy"] - ref["energy"]).max()) <= 1e-6
 
 
+# molecules above 32 atoms take a launch shape only where eigenvalues are asked
+# for: the two tests above once more with every molecule in the persistent kernel
+@pytest.mark.parametrize("test", [test_every_launch_shape_matches_default, test_tuner_mixed_over_every_shape])
+def test_launch_shapes_with_large_molecules(test, monkeypatch):
+    monkeypatch.setenv("MBD_EIG_METHOD", "1")
+    test()
+
+
 def test_batch_rejects_bad_input():
     with engine.MbdEngine(0) as eng:
         big = io.Geometry(["C"] * 600, np.arange(1800, dtype=float).reshape(600, 3) * 0.5,

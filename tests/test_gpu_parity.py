@@ -214,6 +214,37 @@ def test_tridiagonalisation_forms_agree(monkeypatch):
             assert r.diag["n_negative"] == eager.diag["n_negative"]
 
 
+@pytest.mark.parametrize("positive", [True, False])
+def test_one_stage_graph_replays_agree(positive, monkeypatch):
+    """The same two forms where the eigenvalues are computed: asked for
+    (MBD_EIG_METHOD) for a positive definite matrix of order 768, and by default
+    for one of order 300 with negative eigenvalues."""
+    from mbd_amd import engine, generators
+    from mbd_amd.io import Geometry, Settings
+    if positive:
+        monkeypatch.setenv("MBD_EIG_METHOD", "1")
+        geo, st = generators.random_periodic(256, 15.1, seed=77, rc_scs=20.0, rc_sc=12.0, rc_cfdm=30.0)
+    else:
+        geo, st = Geometry(["Na"] * 100, np.array([[0.0, 0.0, 3.0 * i] for i in range(100)]), np.ones(100)), Settings()
+    with engine.MbdEngine(0) as g, engine.MbdEngine(0) as other:
+        g.set_geometry(geo, st)
+        other.set_geometry(*CASES["C6H6"]())
+        monkeypatch.setenv("MBD_TRD_GRAPH", "0")
+        eager = g.run("fp64")
+        g.profile_enable(True)
+        assert g.run("fp64").e_mbd == eager.e_mbd
+        prof = g.profile_read()
+        g.profile_enable(False)
+        assert prof["trd_symv"]["launches"] > 0 and prof["bisect"]["launches"] > 0
+        assert (eager.diag["n_negative"] == 0) == positive
+        monkeypatch.delenv("MBD_TRD_GRAPH")
+        for _ in range(3):
+            r = g.run("fp64")
+            other.run("mixed")  # eager work on another stream between replays
+            assert r.e_mbd == eager.e_mbd
+            assert r.diag["n_negative"] == eager.diag["n_negative"]
+
+
 @pytest.mark.parametrize("case", ["C6H6", "graphene_111", "random64_periodic",
                                   "sheet48_vacuum_z"])
 def test_full_run_iterative(eng, case):
