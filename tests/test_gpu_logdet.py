@@ -286,3 +286,55 @@ def test_primitive_cells(n, edge, cells, monkeypatch):
     assert d["supercell"] == cells
     assert abs(got - want) <= 2.2e-16 * 3 * n * np.prod(cells) * 1.5 * np.sum(om)
     assert t_cells < t_eig
+
+
+def _budget(geo, st, gb, monkeypatch):
+    """Energy with room for all shifted matrices and within a memory budget; the
+    launches of the diagonal blocks of both; the eigenvalues' energy."""
+    with engine.MbdEngine(0) as eng:
+        eng.set_geometry(geo, st)
+        a, _, _, c, _, _ = eng.scs("fp64")
+        out = []
+        for env in ({}, {"MBD_SCS_MEM_GB": gb}, {"MBD_EIG_METHOD": "1"}):
+            for k, v in env.items():
+                monkeypatch.setenv(k, v)
+            eng.profile_enable(True)
+            e, om, _, d = eng.energy(a, c)
+            out.append((e, eng.profile_read()))
+            for k in env:
+                monkeypatch.delenv(k)
+    tol = 2.2e-16 * 3 * geo.n_atoms * np.prod(d["supercell"]) * 1.5 * np.sum(om)
+    assert abs(out[0][0] - out[2][0]) <= tol
+    return out, d["supercell"]
+
+
+# a few shifted matrices at a time: of one matrix its nodes in parts (order 771:
+# 5.8 MB each, 3 at a time), of several matrices a part of them with all their
+# nodes (order 54: 158 KB, order 108 of the paired wave vectors 228 KB; 9 to 13
+# shifts each, so 5.5 MB hold two or three of eight, and one or two of four)
+@pytest.mark.parametrize("edges,cells,gb", [(None, [1, 1, 1], "0.02"),
+                                            ((13.0, 14.0, 14.5), [2, 2, 2], "0.0055"),
+                                            ((9.0, 9.1, 26.0), [3, 3, 1], "0.0055")])
+def test_shifted_matrices_in_parts(edges, cells, gb, monkeypatch):
+    if edges is None:
+        geo, st = _spread(257, 257), Settings()
+    else:
+        geo = _spread(18, 5, gap=2.3)
+        geo = Geometry(geo.names, geo.coords_ang - geo.coords_ang.min(0), geo.hirshfeld, np.diag(edges))
+        st = Settings(mbd_supercell_cutoff=25.0, mbd_cfdm_dip_cutoff=60.0, mbd_scs_dip_cutoff=30.0)
+    out, supercell = _budget(geo, st, gb, monkeypatch)
+    assert supercell == cells
+    assert out[1][1]["logdet_diag"]["launches"] > out[0][1]["logdet_diag"]["launches"] > 0
+    assert out[1][1]["bisect"]["launches"] == 0
+    assert out[1][0] == out[0][0]
+
+
+@pytest.mark.parametrize("edges", [None, (13.0, 14.0, 14.5)])
+def test_no_room_for_a_shifted_matrix(edges, monkeypatch):
+    geo = _spread(18, 5, gap=2.3)
+    lat = None if edges is None else np.diag(edges)
+    geo = Geometry(geo.names, geo.coords_ang - geo.coords_ang.min(0), geo.hirshfeld, lat)
+    st = Settings(mbd_supercell_cutoff=25.0, mbd_cfdm_dip_cutoff=60.0, mbd_scs_dip_cutoff=30.0)
+    out, _ = _budget(geo, st, "0.0001", monkeypatch)
+    assert out[1][1]["logdet_diag"]["launches"] == 0 and out[1][1]["bisect"]["launches"] > 0
+    assert out[1][0] == out[2][0]
