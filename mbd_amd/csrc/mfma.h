@@ -29,14 +29,15 @@ struct Mfma<float> {
 };
 
 // 1 / sqrt(x) and 1 / x for x > 0 from the hardware estimates refined by
-// Newton steps (a few ulp; the correctly rounded square root and division are
-// long dependent chains on the factorisations' critical path)
+// Newton steps (the correctly rounded square root and division are long
+// dependent chains on the factorisations' critical path).  The last step adds
+// a correction formed from the residual, an error of 1.5 units of 2^-53 (FP32:
+// 2^-24) against 2 of 1 / sqrt(x) from the two rounded operations; the form
+// y (3/2 - x y^2 / 2) of the same length has 2.5.
 __device__ inline double rsq_fast(double x) {
   double y = __builtin_amdgcn_rsq(x);
-  const double h = 0.5 * x;
-  y = y * fma(-h, y * y, 1.5);
-  y = y * fma(-h, y * y, 1.5);
-  return y;
+  y = y * fma(-0.5 * x, y * y, 1.5);
+  return fma(0.5 * y, fma(-(x * y), y, 1.0), y);
 }
 __device__ inline double rcp_fast(double x) {
   double r = __builtin_amdgcn_rcp(x);
@@ -45,8 +46,8 @@ __device__ inline double rcp_fast(double x) {
   return r;
 }
 __device__ inline float rsq_fast(float x) {
-  float y = __builtin_amdgcn_rsqf(x);
-  return y * fmaf(-0.5f * x, y * y, 1.5f);
+  const float y = __builtin_amdgcn_rsqf(x);
+  return fmaf(0.5f * y, fmaf(-(x * y), y, 1.0f), y);
 }
 __device__ inline float rcp_fast(float x) {
   float r = __builtin_amdgcn_rcpf(x);

@@ -45,3 +45,23 @@ def test_gemm_edges(m, n, k, fp32):
     # k + 1 roundings of sums no larger than |A| |B|^T + |C|
     eps = 6e-8 if fp32 else 1.2e-16
     assert np.all(np.abs(got - (C - A @ B.T)) <= 2 * (k + 2) * eps * (np.abs(A) @ np.abs(B).T + np.abs(C)))
+
+
+def test_cholesky_pivot_rounding():
+    """Column 0 of the factor is a_i / sqrt(d): no further from it than the
+    reciprocal square root's 1.5 and the product's 1 unit of 2^-53 (d and a_i
+    from 31 of 640 arrow matrices; the two rounded operations and the product
+    reach 3 units)."""
+    from mbd_amd import engine
+    rng = np.random.default_rng(0)
+    b, n = 640, 32
+    A = np.zeros((b, n, n))
+    A[:, np.arange(n), np.arange(n)] = 1e6
+    A[:, 0, 0] = np.exp(rng.uniform(-4, 4, b))
+    A[:, 1:, 0] = rng.uniform(-1, 1, (b, n - 1))
+    A[:, 0, 1:] = A[:, 1:, 0]
+    L, info = engine.device_cholesky(A)
+    assert not info.any()
+    want = A[:, 1:, 0].astype(np.longdouble) / np.sqrt(A[:, 0, 0].astype(np.longdouble))[:, None]
+    err = np.abs(L[:, 1:, 0] - want) / np.abs(want)
+    assert err.max() <= 2.5 * 2.0 ** -53 * (1 + 1e-6)
