@@ -749,13 +749,17 @@ int ld_factor(mbd_handle *h, const std::vector<LdGroup> &groups, int cells, cons
   hipStream_t s = h->stream;
   const size_t budget = mem_budget();
   const int all = b1 - b0;
-  size_t nmat = 0;
-  for (const LdGroup &g : groups) nmat += (size_t)g.batch * all;
+  size_t nmat = 0, npart = 0;
+  for (const LdGroup &g : groups) {
+    nmat += (size_t)g.batch * all;
+    npart += (size_t)g.batch * all * ceil_div(g.n, 64);
+  }
   const double work = ld_work(groups);
-  h->ldG.ensure(nmat);
+  h->ldG.ensure(npart);
   h->ldInfo.ensure(nmat);
   batch_zero(s, h->ldInfo.p, (int)nmat);
   std::vector<int> node;  // of each factored matrix, in order
+  size_t p0 = 0;          // their sums' parts
   for (const LdGroup &g : groups) {
     const int lda = lead_dim(g.n);
     const long sH = (long)g.n * g.n, sA = (long)g.n * lda,
@@ -786,18 +790,25 @@ int ld_factor(mbd_handle *h, const std::vector<LdGroup> &groups, int cells, cons
         ld_shift(s, g.n, g.H + r0 * sH, g.n, sH, rn, nd, q0, nb, h->A64.p, lda, sA);
         potrf_batched<double>(s, g.n, h->A64.p, lda, sA, rn * nb, h->inv64.p, sinv,
                               h->ldInfo.p + m0, true, work >= kLdProofWork && q0 + nb == nd.n + 1 ? nb : 0);
-        ld_sums(s, g.n, h->A64.p, lda, sA, rn, nd, q0, nb, h->om_at.p, h->N, cells, h->ldG.p + m0);
+        ld_sums(s, g.n, g.H + r0 * sH, g.n, sH, h->A64.p, lda, sA, rn, nd, q0, nb, h->om_at.p, h->N, cells,
+                h->ldG.p + p0);
         for (int m = 0; m < rn * nb; ++m) node.push_back(q0 + m % nb);
+        p0 += (size_t)rn * nb * ceil_div(g.n, 64);
       }
   }
-  std::vector<double> g(node.size());
+  std::vector<double> part(p0);
   std::vector<int> info(node.size());
-  MBD_HIP(hipMemcpyAsync(g.data(), h->ldG.p, 8 * g.size(), hipMemcpyDeviceToHost, s));
-  MBD_HIP(hipMemcpyAsync(info.data(), h->ldInfo.p, 4 * g.size(), hipMemcpyDeviceToHost, s));
+  MBD_HIP(hipMemcpyAsync(part.data(), h->ldG.p, 8 * p0, hipMemcpyDeviceToHost, s));
+  MBD_HIP(hipMemcpyAsync(info.data(), h->ldInfo.p, 4 * info.size(), hipMemcpyDeviceToHost, s));
   MBD_HIP(hipStreamSynchronize(s));
   if (std::any_of(info.begin(), info.end(), [](int i) { return i != 0; })) return 0;
-  for (size_t m = 0; m < g.size(); ++m)
-    if (node[m] < nd.n) e += nd.w[node[m]] * g[m];
+  size_t m = 0, at = 0;
+  for (const LdGroup &g : groups)
+    for (int q = 0; q < g.batch * all; ++q, ++m) {
+      double sum = 0.0;
+      for (int i = 0; i < ceil_div(g.n, 64); ++i) sum += part[at++];
+      if (node[m] < nd.n) e += nd.w[node[m]] * sum;
+    }
   return 1;
 }
 

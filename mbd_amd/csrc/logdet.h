@@ -35,9 +35,10 @@ bool ld_ritz(const double *ab, int count, double &lo, double &hi);
 // Lower triangle of H_r + t[b0 + b] I as matrix r nb + b of A (leading dimension lda), r < batch, b < nb.
 void ld_shift(hipStream_t s, int n, const double *H, long ld, long sH, int batch, const LdNodes &nd,
               int b0, int nb, double *A, long lda, long sA);
-// g[m] = ln det(A_m) - ln det(D + t) from the factor's diagonal, for m < batch nb; row r of a matrix
-// belongs to atom (r % (3 N cells)) / (3 cells).
-void ld_sums(hipStream_t s, int n, const double *L, long lda, long sA, int batch, const LdNodes &nd, int b0,
-             int nb, const double *omega, int N, int cells, double *g);
+// g[m nblk + i], nblk = ceil(n / 64): the part of rows 64 i ... 64 i + 63 in ln det(H_r + t) - ln det(D +
+// t) from the factor L_m of m < batch nb; row r of a matrix belongs to atom (r % (3 N cells)) / (3 cells).
+// Nothing for the entry without a weight.
+void ld_sums(hipStream_t s, int n, const double *H, long ld, long sH, const double *L, long lda, long sA,
+             int batch, const LdNodes &nd, int b0, int nb, const double *omega, int N, int cells, double *g);
 
 }  // namespace mbd

@@ -63,9 +63,9 @@ void jacobi(double u, double kc, double &sn, double &cn, double &dn) {
   dn = std::sqrt(cn * cn + kc * kc * sn * sn);
 }
 
-// The midpoint rule's relative error.  Energies against the same sums in 80-bit
-// arithmetic (order 900 / 1020; the eigenvalue path is off by 1.3e-14 / 7e-15
-// Ha): 1e-12 1.0e-12 / 3.3e-13, 1e-13 7e-15 / 3.3e-13, 1e-14 7e-15 / 4e-15.
+// The midpoint rule's relative error.  Its error alone, of energies of order 36
+// to 1800 (rings, chains, cells): 1e-13 up to 8e-13 of the energy, 1e-14 up to
+// 2e-14, 1e-15 up to 1e-15 (for one node more).
 constexpr double kLdEps = 1e-14;
 constexpr int GB = 64;            // rows of a bounds workgroup
 constexpr int GW = 8;             // its waves
@@ -375,35 +375,61 @@ void ld_sums_mols(hipStream_t s, int nmat, const MolInfo *mols, const MolMat *ma
   MBD_LAUNCH_CHECK();
 }
 
-// One workgroup per matrix: sum over the rows of ln(L_jj^2 / (omega_j^2 + t)),
-// terms near zero, in a fixed order.
-__global__ __launch_bounds__(1024) void k_ld_sums(int n, const double *__restrict__ L, long lda, long sA,
-                                                  LdNodes nd, int b0, int nb,
-                                                  const double *__restrict__ omega, int N, int cells,
-                                                  double *__restrict__ g) {
-  __shared__ double red[16];
-  const int m = blockIdx.x, t = threadIdx.x;
-  const double shift = nd.t[b0 + m % nb];
-  const double *M = L + (long)m * sA;
+// Sum over the rows of ln(L_jj^2 / (omega_j^2 + t)) in a fixed order, 64 rows
+// per workgroup.  In exact arithmetic L_jj^2 = C_jj + t - d_j with d_j the sum
+// of the squares left of the diagonal, and the term is log1p((C_jj - omega_j^2
+// - d_j) / (omega_j^2 + t)): it has no rounding of the diagonal's size, which
+// at a large shift is far above the term (d_j / t is 1e-5 and 1e-7 at the last
+// two nodes) and has the largest weights (the last node's 1 to 3, the third
+// last's 0.08).  So the last kLdRowNodes nodes' rows are read, the others'
+// diagonal only.  Relative errors against 80-bit energies, of the eigenvalue
+// path / all nodes by the diagonal / the last two by rows / all by rows: ring
+// of 12 (order 36) 1.7e-13 / 3.6e-13 / 1.3e-14 / 1.0e-14, order 42 1.1e-13 /
+// 1.5e-13 / 1.5e-14 / 6.5e-15, 1584 2.5e-14 / 1.8e-14 / 5.6e-15 / 4.6e-15,
+// periodic of order 3993 2.6e-14 / 8.8e-14 / 7e-16 / 1.4e-15; 88 matrices of
+// order 3072 16 us / 176 us / 0.8 ms of a pass of 34 ms.
+constexpr int kLdRowNodes = 2;
+__global__ __launch_bounds__(64 * GW) void k_ld_sums(int n, const double *__restrict__ H, long ld, long sH,
+                                                     const double *__restrict__ L, long lda, long sA,
+                                                     LdNodes nd, int b0, int nb,
+                                                     const double *__restrict__ omega, int N, int cells,
+                                                     double *__restrict__ g) {
+  __shared__ double part[GW][GB];
+  const int m = blockIdx.y, b = b0 + m % nb, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  if (b == nd.n) return;  // the proof has no weight
+  const int r0 = blockIdx.x * GB, row = min(r0 + lane, n - 1), end = min(r0 + GB - 1, n - 1);
+  const double *M = L + (long)m * sA + row;
+  const bool rows = b >= nd.n - kLdRowNodes;
   double s = 0.0;
-  for (int j = t; j < n; j += 1024) {
-    const double l = M[j + (long)j * lda], w = omega[(j % (3 * N * cells)) / (3 * cells)];
-    s += log(l * l / (w * w + shift));
+  if (rows) {
+    for (int c = w; c < end; c += 8 * GW) {
+      double v[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) v[q] = M[(long)min(c + q * GW, end) * lda];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) s = c + q * GW < row ? fma(v[q], v[q], s) : s;
+    }
+    part[w][lane] = s;
+    __syncthreads();
   }
+  if (w) return;
+  const double om = omega[(row % (3 * N * cells)) / (3 * cells)], w2 = om * om, d = w2 + nd.t[b];
+  if (rows) {
+    for (int i = 1; i < GW; ++i) s += part[i][lane];
+    s = log1p(((H[(long)(m / nb) * sH + row + row * ld] - w2) - s) / d);
+  } else {
+    const double l = M[row * lda];
+    s = log(l * l / d);
+  }
+  s = r0 + lane < n ? s : 0.0;
   for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-  if ((t & 63) == 0) red[t >> 6] = s;
-  __syncthreads();
-  if (t == 0) {
-    double a = 0.0;
-    for (int i = 0; i < 16; ++i) a += red[i];
-    g[m] = a;
-  }
+  if (lane == 0) g[(long)m * gridDim.x + blockIdx.x] = s;
 }
 
-void ld_sums(hipStream_t s, int n, const double *L, long lda, long sA, int batch, const LdNodes &nd, int b0,
-             int nb, const double *omega, int N, int cells, double *g) {
-  hipLaunchKernelGGL(k_ld_sums, dim3(batch * nb), dim3(1024), 0, s, n, L, lda, sA, nd, b0, nb, omega, N,
-                     cells, g);
+void ld_sums(hipStream_t s, int n, const double *H, long ld, long sH, const double *L, long lda, long sA,
+             int batch, const LdNodes &nd, int b0, int nb, const double *omega, int N, int cells, double *g) {
+  hipLaunchKernelGGL(k_ld_sums, dim3(ceil_div(n, GB), batch * nb), dim3(64 * GW), 0, s, n, H, ld, sH, L, lda,
+                     sA, nd, b0, nb, omega, N, cells, g);
   MBD_LAUNCH_CHECK();
 }
 

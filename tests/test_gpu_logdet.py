@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 from mbd_amd import engine, generators
-from mbd_amd.io import Geometry, Settings
+from mbd_amd.io import BOHR, Geometry, Settings
 
 pytestmark = pytest.mark.gpu
 
@@ -338,3 +338,54 @@ def test_no_room_for_a_shifted_matrix(edges, monkeypatch):
     out, _ = _budget(geo, st, "0.0001", monkeypatch)
     assert out[1][1]["logdet_diag"]["launches"] == 0 and out[1][1]["bisect"]["launches"] > 0
     assert out[1][0] == out[2][0]
+
+
+def _energy80(geo, alpha, omega, reff, beta):
+    """Energy of a molecule in 80-bit arithmetic by Jacobi's method."""
+    L = np.longdouble
+    x = (np.asarray(geo.coords_ang) / BOHR).astype(L)
+    a, w, R = (np.asarray(v).astype(L) for v in (alpha, omega, reff))
+    n = len(x)
+    d = x[:, None] - x[None]
+    r = np.sqrt((d ** 2).sum(-1)) + np.eye(n, dtype=L)
+    damp = 1 + np.exp(-6 * (r / (L(beta) * (R[:, None] + R[None])) - 1))
+    c = w[:, None] * w[None] * np.sqrt(a[:, None] * a[None]) / (damp * r ** 5) * (1 - np.eye(n, dtype=L))
+    A = np.zeros((n, 3, n, 3), L)
+    for i in range(3):
+        for j in range(3):
+            A[:, i, :, j] = ((r * r if i == j else 0) - 3 * d[..., i] * d[..., j]) * c
+    A = A.reshape(3 * n, 3 * n) + np.diag(np.repeat(w * w, 3))
+    while np.abs(np.tril(A, -1)).max() > 1e-17:
+        for p in range(3 * n - 1):
+            for q in range(p + 1, 3 * n):
+                if abs(A[p, q]) < 1e-22:
+                    continue
+                th = (A[q, q] - A[p, p]) / (2 * A[p, q])
+                t = (1 if th >= 0 else -1) / (abs(th) + np.sqrt(th * th + 1))
+                cs = 1 / np.sqrt(t * t + 1)
+                sn = t * cs
+                A[p], A[q] = cs * A[p] - sn * A[q], sn * A[p] + cs * A[q]
+                A[:, p], A[:, q] = cs * A[:, p] - sn * A[:, q], sn * A[:, p] + cs * A[:, q]
+    return np.sqrt(np.diag(A)).sum() / 2 - 1.5 * w.sum()
+
+
+def test_small_energies_against_80_bits():
+    """Eight rings of 12 atoms, energies of 0.007 Ha between sums of 8 Ha: the
+    quadrature's 2e-14 of the energy, the matrix elements' (16 eps each, the
+    energy is quadratic in them), and eps of every row in the nodes whose
+    logarithms come from the diagonal (weights below 0.25 in all)."""
+    worst = 0.0
+    for seed in range(8):
+        rng = np.random.default_rng(seed)
+        geo, st = generators.ring()
+        geo.coords_ang = geo.coords_ang + rng.normal(0.0, 0.02, geo.coords_ang.shape)
+        free = np.array([engine.free_atom_params(s) for s in geo.names])
+        a = free[:, 1] * rng.uniform(0.5, 0.8, 12)
+        with engine.MbdEngine(0) as eng:
+            eng.set_geometry(geo, st)
+            got, om, rf, _ = eng.energy(a, free[:, 0] * rng.uniform(0.4, 0.6, 12))
+        want = _energy80(geo, a, om, rf, engine.beta(st.flag_xc))
+        eps = 2.2e-16
+        tol = (2e-14 + 32 * eps) * abs(want) + 0.25 * eps * np.sqrt(36)
+        worst = max(worst, float(abs(got - want) / tol))
+    assert worst <= 1.0
