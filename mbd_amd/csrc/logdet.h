@@ -12,7 +12,11 @@ namespace mbd {
 // D = diag(omega^2); one more entry, t = -lo without a weight, whose factorisation proves that
 // every eigenvalue of C lies above lo.
 constexpr int kLdMaxNodes = 20;
-constexpr long kLdMaxOrder = 16384;
+// Order of the coupled matrix up to which its energy is by log-determinants.  They cost 12 n^3 / 3
+// operations on the GEMM, the band reduction 4 n^3 / 3 behind panels and a bulge chase whose share falls
+// with n: order 16800 299 / 366 ms, 20001 488 / 542, 24576 865 / 823, 30000 (two passes within
+// 64 GB) 1574 / 1341.
+constexpr long kLdMaxOrder = 22000;
 struct LdNodes {
   int n = 0;  // nodes; entry n is the proof's shift
   double t[kLdMaxNodes + 1];

@@ -389,3 +389,22 @@ def test_small_energies_against_80_bits():
         tol = (2e-14 + 32 * eps) * abs(want) + 0.25 * eps * np.sqrt(36)
         worst = max(worst, float(abs(got - want) / tol))
     assert worst <= 1.0
+
+
+def test_largest_orders(monkeypatch):
+    """Order 16803: log-determinants, which the band reduction overtakes past 22000."""
+    n = 5601
+    geo = _spread(n, n)
+    free = np.array([engine.free_atom_params(s) for s in geo.names])
+    a, c = free[:, 1] * geo.hirshfeld, free[:, 0] * geo.hirshfeld ** 2
+    with engine.MbdEngine(0) as eng:
+        eng.set_geometry(geo, Settings())
+        monkeypatch.setenv("MBD_EIG_METHOD", "2")
+        want, om, _, dw = eng.energy(a, c)
+        monkeypatch.delenv("MBD_EIG_METHOD")
+        eng.profile_enable(True)
+        got, _, _, dg = eng.energy(a, c)
+        prof = eng.profile_read()
+    assert prof["logdet_diag"]["launches"] > 0 and prof["bisect"]["launches"] == 0
+    assert dg["n_negative"] == dw["n_negative"] == 0
+    assert abs(got - want) <= 2.2e-16 * 3 * n * 1.5 * np.sum(om)
