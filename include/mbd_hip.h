@@ -183,6 +183,8 @@ int mbd_debug_cfdm_matrix(mbd_handle *h, const double *alpha_eff,
  * consecutive) with the device factorisation; info[batch]. */
 int mbd_debug_cholesky(int device, int n, int batch, const double *A,
                        double *L, int *info);
+int mbd_debug_cholesky_fp32(int device, int n, int batch, const float *A,
+                            float *L, int *info);
 
 /* All eigenvalues (ascending) of a symmetric n x n matrix (lower triangle
  * read) with the device tridiagonalisation + bisection. */

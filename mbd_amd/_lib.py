@@ -89,6 +89,7 @@ def lib():
     L.mbd_debug_relay_matrix.argtypes = [h, ctypes.c_int, ctypes.c_int, _D]
     L.mbd_debug_cfdm_matrix.argtypes = [h, _D, _D, _D, _D]
     L.mbd_debug_cholesky.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, _D, _D, _I]
+    L.mbd_debug_cholesky_fp32.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, _F, _F, _I]
     L.mbd_debug_sym_eigvals.argtypes = [ctypes.c_int, ctypes.c_int, _D, _D]
     L.mbd_debug_lu_solve.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, _D, _D, _I]
     L.mbd_debug_gemm_nt.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,

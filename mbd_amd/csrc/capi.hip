@@ -1141,6 +1141,42 @@ bool valid_mode(int mode) {
 
 }  // namespace
 
+namespace {
+
+template <typename T>
+int debug_cholesky(int device, int n, int batch, const T *A, T *L, int *info) {
+  if (n <= 0) return -2;
+  if (batch <= 0) return -3;
+  if (!A) return -4;
+  if (!L) return -5;
+  if (!info) return -6;
+  T *dA = nullptr, *dinv = nullptr;
+  int *dinfo = nullptr;
+  int rc = 0;
+  try {
+    MBD_HIP(hipSetDevice(device));
+    const long sA = (long)n * n;
+    const long sinv = (long)ceil_div(n, kCholNB) * kCholNB * kCholNB;
+    MBD_HIP(hipMalloc(&dA, sizeof(T) * sA * batch));
+    MBD_HIP(hipMalloc(&dinv, sizeof(T) * sinv * batch));
+    MBD_HIP(hipMalloc(&dinfo, sizeof(int) * batch));
+    MBD_HIP(hipMemcpy(dA, A, sizeof(T) * sA * batch, hipMemcpyHostToDevice));
+    MBD_HIP(hipMemset(dinfo, 0, sizeof(int) * batch));
+    potrf_batched<T>(nullptr, n, dA, n, sA, batch, dinv, sinv, dinfo);
+    MBD_HIP(hipDeviceSynchronize());
+    MBD_HIP(hipMemcpy(L, dA, sizeof(T) * sA * batch, hipMemcpyDeviceToHost));
+    MBD_HIP(hipMemcpy(info, dinfo, sizeof(int) * batch, hipMemcpyDeviceToHost));
+  } catch (const HipError &e) {
+    rc = fail(nullptr, e);
+  }
+  if (dA) (void)hipFree(dA);
+  if (dinv) (void)hipFree(dinv);
+  if (dinfo) (void)hipFree(dinfo);
+  return rc;
+}
+
+}  // namespace
+
 extern "C" {
 
 int mbd_create(int device, mbd_handle **out) {
@@ -1792,37 +1828,11 @@ int mbd_debug_cfdm_matrix(mbd_handle *h, const double *alpha_eff, const double *
 }
 
 int mbd_debug_cholesky(int device, int n, int batch, const double *A, double *L, int *info) {
-  if (n <= 0) return -2;
-  if (batch <= 0) return -3;
-  if (!A) return -4;
-  if (!L) return -5;
-  if (!info) return -6;
-  double *dA = nullptr, *dinv = nullptr;
-  int *dinfo = nullptr;
-  try {
-    MBD_HIP(hipSetDevice(device));
-    const long sA = (long)n * n;
-    const int nblk = ceil_div(n, kCholNB);
-    const long sinv = (long)nblk * kCholNB * kCholNB;
-    MBD_HIP(hipMalloc(&dA, sizeof(double) * sA * batch));
-    MBD_HIP(hipMalloc(&dinv, sizeof(double) * sinv * batch));
-    MBD_HIP(hipMalloc(&dinfo, sizeof(int) * batch));
-    MBD_HIP(hipMemcpy(dA, A, sizeof(double) * sA * batch, hipMemcpyHostToDevice));
-    MBD_HIP(hipMemset(dinfo, 0, sizeof(int) * batch));
-    potrf_batched<double>(nullptr, n, dA, n, sA, batch, dinv, sinv, dinfo);
-    MBD_HIP(hipDeviceSynchronize());
-    MBD_HIP(hipMemcpy(L, dA, sizeof(double) * sA * batch, hipMemcpyDeviceToHost));
-    MBD_HIP(hipMemcpy(info, dinfo, sizeof(int) * batch, hipMemcpyDeviceToHost));
-  } catch (const HipError &e) {
-    if (dA) (void)hipFree(dA);
-    if (dinv) (void)hipFree(dinv);
-    if (dinfo) (void)hipFree(dinfo);
-    return fail(nullptr, e);
-  }
-  (void)hipFree(dA);
-  (void)hipFree(dinv);
-  (void)hipFree(dinfo);
-  return 0;
+  return debug_cholesky<double>(device, n, batch, A, L, info);
+}
+
+int mbd_debug_cholesky_fp32(int device, int n, int batch, const float *A, float *L, int *info) {
+  return debug_cholesky<float>(device, n, batch, A, L, info);
 }
 
 int mbd_debug_sym_eigvals(int device, int n, const double *A, double *w) {

@@ -307,16 +307,20 @@ class MbdEngine:
         return C.reshape(nm, nm).T.copy()
 
 
-def device_cholesky(A_batch: np.ndarray, device: int = 0):
-    """Lower Cholesky factors of a (batch, n, n) stack on the device."""
-    A = np.asarray(A_batch, dtype=np.float64)
+def device_cholesky(A_batch: np.ndarray, device: int = 0, fp32: bool = False):
+    """Lower Cholesky factors of a (batch, n, n) stack on the device, in FP64
+    or FP32 (arrays of that type)."""
+    A = np.asarray(A_batch, dtype=np.float32 if fp32 else np.float64)
     if A.ndim == 2:
         A = A[None]
     b, n, _ = A.shape
     src = np.ascontiguousarray(np.transpose(A, (0, 2, 1)))  # column-major per matrix
     L = np.zeros_like(src)
     info = np.zeros(b, dtype=np.int32)
-    rc = _lib.lib().mbd_debug_cholesky(device, n, b, dptr(src), dptr(L), iptr(info))
+    if fp32:
+        rc = _lib.lib().mbd_debug_cholesky_fp32(device, n, b, fptr(src), fptr(L), iptr(info))
+    else:
+        rc = _lib.lib().mbd_debug_cholesky(device, n, b, dptr(src), dptr(L), iptr(info))
     if rc != 0:
         raise MbdError(f"mbd_debug_cholesky failed ({rc})")
     return np.tril(np.transpose(L, (0, 2, 1))), info

@@ -65,3 +65,46 @@ def test_cholesky_pivot_rounding():
     want = A[:, 1:, 0].astype(np.longdouble) / np.sqrt(A[:, 0, 0].astype(np.longdouble))[:, None]
     err = np.abs(L[:, 1:, 0] - want) / np.abs(want)
     assert err.max() <= 2.5 * 2.0 ** -53 * (1 + 1e-6)
+
+
+# one short of, at and one past outer blocks of 512 columns, and the FP32 form
+# (the mixed solve's factor) at the edges of sub-blocks and diagonal blocks too
+@pytest.mark.parametrize("n,fp32", [(511, False), (512, False), (513, False), (640, False), (1025, False)] +
+                         [(n, True) for n in (1, 31, 33, 64, 97, 128, 129, 257, 511, 512, 513, 1025)])
+def test_cholesky_outer_blocks_and_fp32(n, fp32):
+    from mbd_amd import engine
+    t = np.float32 if fp32 else np.float64
+    A = np.array([_spd(n, n), _spd(n, n + 1)]).astype(t)
+    L, info = engine.device_cholesky(A, fp32=fp32)
+    assert L.dtype == t and list(info) == [0, 0]
+    for b in range(2):
+        # as above: n eps cond(A) |L|
+        want = np.linalg.cholesky(A[b].astype(np.float64))
+        assert np.allclose(L[b], want, rtol=0, atol=n * (1.2e-7 if fp32 else 2.3e-16) * 10 * 2)
+
+
+@pytest.mark.parametrize("at,fp32", [(512, False), (513, False), (700, False), (1, True), (33, True),
+                                     (128, True), (129, True), (513, True), (700, True)])
+def test_cholesky_reports_pivot_past_outer_block(at, fp32):
+    from mbd_amd import engine
+    A = _spd(700, at)
+    A[at - 1, at - 1] = -1.0
+    _, info = engine.device_cholesky(np.array([A, _spd(700, 1)]), fp32=fp32)
+    assert list(info) == [at, 0]
+
+
+def test_cholesky_pivot_rounding_fp32():
+    """As test_cholesky_pivot_rounding, in units of 2^-24."""
+    from mbd_amd import engine
+    rng = np.random.default_rng(0)
+    b, n = 640, 32
+    A = np.zeros((b, n, n), np.float32)
+    A[:, np.arange(n), np.arange(n)] = 1e4
+    A[:, 0, 0] = np.exp(rng.uniform(-4, 4, b))
+    A[:, 1:, 0] = rng.uniform(-1, 1, (b, n - 1))
+    A[:, 0, 1:] = A[:, 1:, 0]
+    L, info = engine.device_cholesky(A, fp32=True)
+    assert not info.any()
+    want = A[:, 1:, 0].astype(np.float64) / np.sqrt(A[:, 0, 0].astype(np.float64))[:, None]
+    err = np.abs(L[:, 1:, 0] - want) / np.abs(want)
+    assert err.max() <= 2.5 * 2.0 ** -24 * (1 + 1e-6)
