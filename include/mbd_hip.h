@@ -110,8 +110,9 @@ int mbd_scs(mbd_handle *h, int mode, double *alpha_eff, double *coupled_pol,
 /* E_MBD from alpha_eff[n] and c6_eff[n] (UTILS.f90:700-879): builds the
  * coupled-QHO matrix over the supercell and, in FP64,
  * E = 1/2 sum_{l>=0} sqrt(l) / Ncell - 3/2 sum w, from log-determinants of
- * shifted matrices where all eigenvalues l are proved positive, from the
- * eigenvalues otherwise.  omega[n], reff[n] may be NULL.  Returns 0 or MBD_ERR_*; d->info_eig and d->n_negative report. */
+ * shifted matrices where all w are positive and all eigenvalues l are proved
+ * positive, from the eigenvalues otherwise.  omega[n], reff[n] may be NULL.
+ * Returns 0 or MBD_ERR_*; d->info_eig and d->n_negative report. */
 int mbd_energy(mbd_handle *h, const double *alpha_eff, const double *c6_eff,
                double *e_mbd, double *omega, double *reff, mbd_diag *d);
 

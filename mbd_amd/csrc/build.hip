@@ -28,7 +28,7 @@ namespace mbd {
 
 namespace {
 
-constexpr int kFullTiles = 512;  // tiles that fill the 256 CUs with one workgroup each
+constexpr int kFullTiles = 512;  // tiles that fill the 256 CUs with two workgroups each
 constexpr int kFreqGroup = 7;   // grid points per image scan of the SCS builder
 constexpr int TILE = 16;        // atoms (sites) per tile edge
 constexpr int TB = 3 * TILE;    // matrix rows per tile edge
@@ -67,7 +67,9 @@ __device__ inline bool in_sphere(double dx, double dy, double dz, double rc, dou
 // wave so runs the tensor once per marked image of its fullest pair in each
 // chunk rather than once per image marked by any of its 64 pairs (at a 100 A
 // cutoff in a 38 A cell about 76 of 343 images per pair, scattered
-// differently over the lanes).  Each pair still sums its images in table order.
+// differently over the lanes).  Each pair sums its images in table order, or
+// with several slices of a workgroup (k_scs_build) each slice's in that order
+// and then the slices.
 constexpr int kImgChunk = 32;
 // NEAR: near is set if an image's r^2 is so close to rc^2 that another
 // rounding of the same displacement could decide otherwise.
