@@ -513,15 +513,15 @@ void cfdm_cells(hipStream_t s, int N, int ncell, const double *xyz, const int *c
 // Phases of the cells' Fourier transform, (nreal + npair) x ncell cosines and
 // then the pairs' sines: every k.a / S is a multiple of 1 / L, L the least
 // common multiple of the cells along the axes, whose cosines and sines cs
-// holds.  kv: the wave vectors, real ones first.
+// holds, then the wave vectors, real ones first (one upload).
 __global__ __launch_bounds__(256) void k_cell_phase(int s1, int s2, int s3, int L, int nreal, int npair,
-                                                    const int *__restrict__ kv,
                                                     const double *__restrict__ cs,
                                                     double *__restrict__ phase) {
   const int nc = s1 * s2 * s3, a = blockIdx.x * 256 + threadIdx.x, k = blockIdx.y;
   if (a >= nc) return;
-  const int m1 = kv[3 * k] * (a % s1) % s1 * (L / s1), m2 = kv[3 * k + 1] * (a / s1 % s2) % s2 * (L / s2),
-            m3 = kv[3 * k + 2] * (a / s1 / s2) % s3 * (L / s3);
+  const double *kv = cs + 2 * L + 3 * k;
+  const int m1 = (int)kv[0] * (a % s1) % s1 * (L / s1), m2 = (int)kv[1] * (a / s1 % s2) % s2 * (L / s2),
+            m3 = (int)kv[2] * (a / s1 / s2) % s3 * (L / s3);
   const int m = (m1 + m2 + m3) % L;
   phase[(long)k * nc + a] = cs[m];
   if (k >= nreal) phase[(long)(k + npair) * nc + a] = cs[L + m];
@@ -568,12 +568,12 @@ __global__ __launch_bounds__(256) void k_cell_dft(int n, int ncell, int nreal, i
   }
 }
 
-void cell_dft(hipStream_t s, int n, const int *cells, int L, int nreal, int npair, const int *kv,
-              const double *cs, double *phase, const double *B, double *Hr, double *Hp) {
+void cell_dft(hipStream_t s, int n, const int *cells, int L, int nreal, int npair, const double *cs,
+              double *phase, const double *B, double *Hr, double *Hp) {
   const int nc = cells[0] * cells[1] * cells[2], nk = nreal + npair;
   ProfScope ps(K_CFDM_BUILD, s, 4.0 * n * (n + 1.0) * (nc + nreal + 4.0 * npair), 0.0);
   hipLaunchKernelGGL(k_cell_phase, dim3(ceil_div(nc, 256), nk), dim3(256), 0, s, cells[0], cells[1],
-                     cells[2], L, nreal, npair, kv, cs, phase);
+                     cells[2], L, nreal, npair, cs, phase);
   // 8 workgroups per CU, half of them above the diagonal
   const int nz = std::min(nk, ceil_div(8 * 256, ceil_div(n, 256) * n));
   hipLaunchKernelGGL(k_cell_dft, dim3(ceil_div(n, 256), n, nz), dim3(256), 0, s, n, nc, nreal, npair,

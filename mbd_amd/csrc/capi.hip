@@ -289,7 +289,7 @@ struct mbd_handle {
   DevBuf<int> ldInfo;
   // supercells by cell differences: blocks, their Fourier transform, phases
   DevBuf<double> cellB, cellH, cellPh;
-  DevBuf<int> cellNear, cellK;
+  DevBuf<int> cellNear;
   bool cells_cover = false;  // the image box covers the cutoff sphere for every pair
   // result of the last run_energy
   double e_val = 0.0;
@@ -682,14 +682,13 @@ bool use_logdet() { return !getenv("MBD_EIG_METHOD"); }
 constexpr int kLzMinOrder = 7000;
 // From this n^3 (summed over the matrices) on, a guess of the lower end after
 // one that failed is proved before its nodes are factored (the matrix most
-// likely has an eigenvalue that is not positive), and a set's products end
-// once its proof has failed.  Energies of matrices with negative eigenvalues
-// (a factorisation of order 3000 fails at row 231), without either / proof
-// first / both / by eigenvalues alone: order 2100 31.3 / 30.3 / 27.8 / 25.1
-// ms, 3000 47.8 / 44.5 / 40.1 / 36.3, 6000 130 / 107 / 85 / 77, 6900 168 / 134
-// / 101 / 92.  Below, one matrix takes about as long as a set (order 900: 31.5
-// / 31.3 / 30.7 / 29.2), and the products' look at the proof 1 % of a
-// molecule of order 1584.
+// likely has an eigenvalue that is not positive), and a set's updates end once
+// its proof has failed.  Energies of matrices with negative eigenvalues (a
+// factorisation of order 3000 fails at row 231), without either / proof first /
+// both / by eigenvalues alone: order 2100 31.3 / 30.3 / 28.5 / 25.1 ms, 3000
+// 47.8 / 44.5 / 41.3 / 36.3, 6000 130 / 107 / 88 / 77, 6900 168 / 134 / 104 /
+// 92.  Below, one matrix takes about as long as a set (order 900: 31.5 / 31.3 /
+// 30.7 / 29.2).
 constexpr double kLdProofWork = 2048.0 * 2048.0 * 2048.0;
 void fetch(mbd_handle *h, double *dst, const double *src, size_t count);
 
@@ -912,23 +911,22 @@ ByCells energy_by_cells(mbd_handle *h, const double *alpha_eff_d) {
   const int nr = (int)kv.size() / 3, np = (int)pair.size() / 3;
   kv.insert(kv.end(), pair.begin(), pair.end());
   const int L = std::lcm(S[0], std::lcm(S[1], S[2]));
-  std::vector<double> cs(2 * (size_t)L);
+  std::vector<double> cs(2 * (size_t)L);  // and the wave vectors
   for (int m = 0; m < L; ++m) {
     cs[m] = std::cos(2.0 * kPi * m / L);
     cs[L + m] = std::sin(2.0 * kPi * m / L);
   }
+  cs.insert(cs.end(), kv.begin(), kv.end());
   h->cellPh.ensure(cs.size() + (size_t)(nr + 2 * np) * nc);
-  h->cellK.ensure(kv.size());
   h->cellB.ensure(nc * nn);
   h->cellH.ensure((nr + 4 * (size_t)np) * nn);
   h->cellNear.ensure(1);
   MBD_HIP(hipMemcpyAsync(h->cellPh.p, cs.data(), 8 * cs.size(), hipMemcpyHostToDevice, s));
-  MBD_HIP(hipMemcpyAsync(h->cellK.p, kv.data(), sizeof(int) * kv.size(), hipMemcpyHostToDevice, s));
   batch_zero(s, h->cellNear.p, 1);
   cfdm_cells(s, N, nc, h->xyz.p, h->cell.p, h->lat_d.p, h->nimg_cfdm, h->nimg_cfdm / 2, h->img_cfdm.p,
              h->rc_cfdm / kBohr, h->beta, alpha_eff_d, h->om_at.p, h->reff.p, h->cellB.p,
              h->cellNear.p);
-  cell_dft(s, n, S, L, nr, np, h->cellK.p, h->cellPh.p, h->cellPh.p + 2 * L, h->cellB.p, h->cellH.p,
+  cell_dft(s, n, S, L, nr, np, h->cellPh.p, h->cellPh.p + cs.size(), h->cellB.p, h->cellH.p,
            h->cellH.p + nr * nn);
   int near = 0;
   MBD_HIP(hipMemcpyAsync(&near, h->cellNear.p, sizeof near, hipMemcpyDeviceToHost, s));
@@ -1257,7 +1255,6 @@ int mbd_destroy(mbd_handle *h) {
   h->cellH.release();
   h->cellPh.release();
   h->cellNear.release();
-  h->cellK.release();
   batch_release(h);
   if (h->trd_exec) (void)hipGraphExecDestroy(h->trd_exec);
   if (h->stream2) (void)hipStreamSynchronize(h->stream2);

@@ -270,7 +270,8 @@ __global__ __launch_bounds__(256) void k_potrf_diag_mols(int k0, const MolInfo *
 
 // energy: matrices of log-determinants.  proof > 0: of every `proof`
 // consecutive ones the others are useless if the last is not positive definite,
-// and their products are left out once it has shown that.
+// and their updates are left out once it has shown that (not the short panel
+// products: the look took 2 % of them).
 template <typename T>
 void potrf_batched(hipStream_t s, int n, T *A, int lda, long sA, int batch,
                    T *inv, long sinv_blk, int *info, bool energy, int proof) {
@@ -305,7 +306,7 @@ void potrf_batched(hipStream_t s, int n, T *A, int lda, long sA, int batch,
       {
         ProfScope ps(energy ? K_LD_TRSM : K_CHOL_TRSM, s, 0.0, batch * (double)m2 * kb * kb);
         gemm_nt(s, false, m2, kb, kb, T(1), A21, lda, sA, invk, NB, sinv_blk,
-                T(0), A21, lda, sA, batch, stop, per);
+                T(0), A21, lda, sA, batch);
       }
       // the rest of the outer block's columns, on and below the diagonal
       const int w2 = o1 - k1;

@@ -48,8 +48,8 @@ struct MatBatch {
 // C[m x n] = alpha * A[m x k] * B[n x k]^T + beta * C, batched over
 // blockIdx.z; lower != 0 restricts to tiles that touch the lower triangle
 // (row tile >= column tile), for symmetric rank-k updates.  With stop (device,
-// one entry per matrix; tall-skinny single products do not look at it), `per`
-// consecutive matrices are left as they are where the last one's entry is set.
+// one entry per matrix), `per` consecutive matrices may be left as they are by
+// a symmetric update where the last one's entry is set.
 void gemm_nt(hipStream_t s, bool lower, int m, int n, int k, double alpha,
              const double *A, int lda, long sA, const double *B, int ldb,
              long sB, double beta, double *C, int ldc, long sC, int batch,

@@ -56,11 +56,13 @@ struct Vec16<float> {
 // compiler wait for each one.
 // ml, nl: rows of A and of B that may be read (m, n or more).  A wave whose
 // 64 x 64 sub-tile lies past m or n computes nothing.
-template <typename T, bool LOWER, bool GEN>
+// STOP: *stop set leaves the tile as it is (looked at behind the first loads,
+// whose latency covers the look's).
+template <typename T, bool LOWER, bool GEN, bool STOP = false>
 __device__ __forceinline__ void gemm_tile(int m, int n, int ml, int nl, int k, T alpha,
                                           const T *__restrict__ A, int lda, const T *__restrict__ B,
                                           int ldb, T beta, T *__restrict__ C, int ldc, int tm, int tn,
-                                          int ta, int tb) {
+                                          int ta, int tb, const int *stop = nullptr) {
   using vec = typename Vec16<T>::t;
   constexpr int V = Vec16<T>::n, G = 4 / V;  // row groups of a wave
   constexpr int NV = BM * BK / V / NT;       // operand vectors per thread
@@ -157,7 +159,12 @@ __device__ __forceinline__ void gemm_tile(int m, int n, int ml, int nl, int k, T
 
   const bool idle = row0 + wm * 64 >= m || col0 + wn * 64 >= n;
   const int nk = (k + BK - 1) / BK;
+  const int halt = STOP ? *stop : 0;
   gload(0);
+  if (STOP) {
+    __builtin_amdgcn_sched_barrier(0);
+    if (halt) return;
+  }
   sstore(0, 0);
   __syncthreads();
   for (int kt = 0; kt < nk; ++kt) {
@@ -238,12 +245,13 @@ __device__ __forceinline__ void gemm_tile(int m, int n, int ml, int nl, int k, T
 }
 
 // One uniform batch: matrix blockIdx.z of each operand, tile blockIdx.x.
-template <typename T, bool LOWER, bool GEN>
+// STOP: nothing for the matrices whose entry of stop says so (an instance of
+// its own: the look alone costs the short products of every other caller 1 to 2 %).
+template <typename T, bool LOWER, bool GEN, bool STOP>
 __global__ __launch_bounds__(NT, 2) void k_gemm_nt(
     int m, int n, int k, T alpha, const T *__restrict__ A, int lda, long sA,
     const T *__restrict__ B, int ldb, long sB, T beta, T *__restrict__ C,
     int ldc, long sC, int tiles_n, int ta, int tb, const int *stop, int per) {
-  if (stop && stop[(blockIdx.z / per + 1) * per - 1]) return;
   int tm, tn;
   const int idx = blockIdx.x;
   if (LOWER && idx < tiles_n * (tiles_n + 1) / 2) {
@@ -257,8 +265,9 @@ __global__ __launch_bounds__(NT, 2) void k_gemm_nt(
     tn = rest % tiles_n;
   }
   const long bz = blockIdx.z;
-  gemm_tile<T, LOWER, GEN>(m, n, m, n, k, alpha, A + bz * sA, lda, B + bz * sB, ldb, beta, C + bz * sC,
-                           ldc, tm, tn, ta, tb);
+  gemm_tile<T, LOWER, GEN, STOP>(m, n, m, n, k, alpha, A + bz * sA, lda, B + bz * sB, ldb, beta,
+                                 C + bz * sC, ldc, tm, tn, ta, tb,
+                                 STOP ? stop + (bz / per + 1) * per - 1 : nullptr);
 }
 
 // The two products of a left-looking Cholesky's block column k0 over matrices
@@ -383,8 +392,9 @@ void launch(hipStream_t s, bool lower, int m, int n, int k, T alpha,
   const int tmn = ceil_div(m, BM), tnn = ceil_div(n, BN);
   const bool gen = ta || tb || m < Vec16<T>::n || n < Vec16<T>::n;
   const dim3 grid(lower ? tnn * (tnn + 1) / 2 + (tmn - tnn) * tnn : tmn * tnn, 1, batch);
-  auto *f = lower ? (gen ? k_gemm_nt<T, true, true> : k_gemm_nt<T, true, false>)
-                  : (gen ? k_gemm_nt<T, false, true> : k_gemm_nt<T, false, false>);
+  auto *f = lower ? (gen ? k_gemm_nt<T, true, true, false> : k_gemm_nt<T, true, false, false>)
+                  : (gen ? k_gemm_nt<T, false, true, false> : k_gemm_nt<T, false, false, false>);
+  if (stop && lower && !gen) f = k_gemm_nt<T, true, false, true>;
   hipLaunchKernelGGL(f, grid, dim3(NT), 0, s, m, n, k, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc,
                      sC, tnn, ta, tb, stop, per);
   MBD_LAUNCH_CHECK();

@@ -32,8 +32,8 @@ void cfdm_cells(hipStream_t s, int N, int ncell, const double *xyz, const int *c
                 const double *lat, int nimg, int center, const double *img, double rc_bohr,
                 double beta, const double *alpha_eff, const double *omega, const double *reff,
                 double *B, int *near);
-void cell_dft(hipStream_t s, int n, const int *cells, int L, int nreal, int npair, const int *kv,
-              const double *cs, double *phase, const double *B, double *Hr, double *Hp);
+void cell_dft(hipStream_t s, int n, const int *cells, int L, int nreal, int npair, const double *cs,
+              double *phase, const double *B, double *Hr, double *Hp);
 
 // chol.hip
 template <typename T>

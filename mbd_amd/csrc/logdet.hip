@@ -394,14 +394,15 @@ void ld_sums_mols(hipStream_t s, int nmat, const MolInfo *mols, const MolMat *ma
 // of 12 (order 36) 1.7e-13 / 3.6e-13 / 1.3e-14 / 1.0e-14, order 42 1.1e-13 /
 // 1.5e-13 / 1.5e-14 / 6.5e-15, 1584 2.5e-14 / 1.8e-14 / 5.6e-15 / 4.6e-15,
 // periodic of order 3993 2.6e-14 / 8.8e-14 / 7e-16 / 1.4e-15; 88 matrices of
-// order 3072 16 us / 176 us / 0.8 ms of a pass of 34 ms.
+// order 3072 16 us / 169 us / 0.8 ms of a pass of 34 ms.
 constexpr int kLdRowNodes = 2;
-__global__ __launch_bounds__(64 * GW) void k_ld_sums(int n, const double *__restrict__ H, long ld, long sH,
+constexpr int SW = 16;  // waves of a sums workgroup
+__global__ __launch_bounds__(64 * SW) void k_ld_sums(int n, const double *__restrict__ H, long ld, long sH,
                                                      const double *__restrict__ L, long lda, long sA,
                                                      LdNodes nd, int b0, int nb,
                                                      const double *__restrict__ omega, int N, int cells,
                                                      double *__restrict__ g) {
-  __shared__ double part[GW][GB];
+  __shared__ double part[SW][GB];
   const int m = blockIdx.y, b = b0 + m % nb, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   if (b == nd.n) return;  // the proof has no weight
   const int r0 = blockIdx.x * GB, row = min(r0 + lane, n - 1), end = min(r0 + GB - 1, n - 1);
@@ -409,12 +410,12 @@ __global__ __launch_bounds__(64 * GW) void k_ld_sums(int n, const double *__rest
   const bool rows = b >= nd.n - kLdRowNodes;
   double s = 0.0;
   if (rows) {
-    for (int c = w; c < end; c += 8 * GW) {
+    for (int c = w; c < end; c += 8 * SW) {
       double v[8];
 #pragma unroll
-      for (int q = 0; q < 8; ++q) v[q] = M[(long)min(c + q * GW, end) * lda];
+      for (int q = 0; q < 8; ++q) v[q] = M[(long)min(c + q * SW, end) * lda];
 #pragma unroll
-      for (int q = 0; q < 8; ++q) s = c + q * GW < row ? fma(v[q], v[q], s) : s;
+      for (int q = 0; q < 8; ++q) s = c + q * SW < row ? fma(v[q], v[q], s) : s;
     }
     part[w][lane] = s;
     __syncthreads();
@@ -422,7 +423,7 @@ __global__ __launch_bounds__(64 * GW) void k_ld_sums(int n, const double *__rest
   if (w) return;
   const double om = omega[(row % (3 * N * cells)) / (3 * cells)], w2 = om * om, d = w2 + nd.t[b];
   if (rows) {
-    for (int i = 1; i < GW; ++i) s += part[i][lane];
+    for (int i = 1; i < SW; ++i) s += part[i][lane];
     s = log1p(((H[(long)(m / nb) * sH + row + row * ld] - w2) - s) / d);
   } else {
     const double l = M[row * lda];
@@ -435,7 +436,7 @@ __global__ __launch_bounds__(64 * GW) void k_ld_sums(int n, const double *__rest
 
 void ld_sums(hipStream_t s, int n, const double *H, long ld, long sH, const double *L, long lda, long sA,
              int batch, const LdNodes &nd, int b0, int nb, const double *omega, int N, int cells, double *g) {
-  hipLaunchKernelGGL(k_ld_sums, dim3(ceil_div(n, GB), batch * nb), dim3(64 * GW), 0, s, n, H, ld, sH, L, lda,
+  hipLaunchKernelGGL(k_ld_sums, dim3(ceil_div(n, GB), batch * nb), dim3(64 * SW), 0, s, n, H, ld, sH, L, lda,
                      sA, nd, b0, nb, omega, N, cells, g);
   MBD_LAUNCH_CHECK();
 }
