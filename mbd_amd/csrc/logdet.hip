@@ -393,7 +393,7 @@ void ld_sums_mols(hipStream_t s, int nmat, const MolInfo *mols, const MolMat *ma
 // path / all nodes by the diagonal / the last two by rows / all by rows: ring
 // of 12 (order 36) 1.7e-13 / 3.6e-13 / 1.3e-14 / 1.0e-14, order 42 1.1e-13 /
 // 1.5e-13 / 1.5e-14 / 6.5e-15, 1584 2.5e-14 / 1.8e-14 / 5.6e-15 / 4.6e-15,
-// periodic of order 3993 2.6e-14 / 8.8e-14 / 7e-16 / 1.4e-15; 88 matrices of
+// periodic of order 3993 2.6e-14 / 8.8e-14 / 7e-16 / 1.4e-15; 104 matrices of
 // order 3072 16 us / 169 us / 0.8 ms of a pass of 34 ms.
 constexpr int kLdRowNodes = 2;
 constexpr int SW = 16;  // waves of a sums workgroup
