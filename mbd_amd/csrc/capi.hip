@@ -682,8 +682,9 @@ bool use_logdet() { return !getenv("MBD_EIG_METHOD"); }
 constexpr int kLzMinOrder = 7000;
 // From this n^3 (summed over the matrices) on, a guess of the lower end after
 // one that failed is proved before its nodes are factored (the matrix most
-// likely has an eigenvalue that is not positive), and a set's updates end once
-// its proof has failed.  Energies of matrices with negative eigenvalues (a
+// likely has an eigenvalue that is not positive), and, without Ritz values, a
+// set's updates end once its proof has failed (the look costs the updates of a
+// positive definite matrix 0.2 %).  Energies of matrices with negative eigenvalues (a
 // factorisation of order 3000 fails at row 231), without either / proof first /
 // both / by eigenvalues alone: order 2100 31.3 / 30.3 / 28.5 / 25.1 ms, 3000
 // 47.8 / 44.5 / 41.3 / 36.3, 6000 130 / 107 / 88 / 77, 6900 168 / 134 / 104 /
@@ -742,9 +743,10 @@ double ld_work(const std::vector<LdGroup> &groups) {
 
 // Factors entries b0 ... b1 - 1 of `nd` for every matrix of `groups` and adds
 // the nodes' terms to e.  1: done; 0: a matrix is not positive definite; -1:
-// no room for one shifted matrix.
+// no room for one shifted matrix.  watch: updates end once the proof, if it is
+// among the entries, has failed.
 int ld_factor(mbd_handle *h, const std::vector<LdGroup> &groups, int cells, const LdNodes &nd, int b0,
-              int b1, double &e) {
+              int b1, bool watch, double &e) {
   hipStream_t s = h->stream;
   const size_t budget = mem_budget();
   const int all = b1 - b0;
@@ -753,7 +755,6 @@ int ld_factor(mbd_handle *h, const std::vector<LdGroup> &groups, int cells, cons
     nmat += (size_t)g.batch * all;
     npart += (size_t)g.batch * all * ceil_div(g.n, 64);
   }
-  const double work = ld_work(groups);
   h->ldG.ensure(npart);
   h->ldInfo.ensure(nmat);
   batch_zero(s, h->ldInfo.p, (int)nmat);
@@ -788,7 +789,7 @@ int ld_factor(mbd_handle *h, const std::vector<LdGroup> &groups, int cells, cons
         const size_t m0 = node.size();
         ld_shift(s, g.n, g.H + r0 * sH, g.n, sH, rn, nd, q0, nb, h->A64.p, lda, sA);
         potrf_batched<double>(s, g.n, h->A64.p, lda, sA, rn * nb, h->inv64.p, sinv,
-                              h->ldInfo.p + m0, true, work >= kLdProofWork && q0 + nb == nd.n + 1 ? nb : 0);
+                              h->ldInfo.p + m0, true, watch && q0 + nb == nd.n + 1 ? nb : 0);
         ld_sums(s, g.n, g.H + r0 * sH, g.n, sH, h->A64.p, lda, sA, rn, nd, q0, nb, h->om_at.p, h->N, cells,
                 h->ldG.p + p0);
         for (int m = 0; m < rn * nb; ++m) node.push_back(q0 + m % nb);
@@ -854,6 +855,8 @@ bool energy_by_logdet(mbd_handle *h, const std::vector<LdGroup> &groups, int cel
     const double up = std::max(w2max, std::min(top, rhi + 0.2 * (rhi - rlo)));
     guess.insert(guess.begin(), {0.65 * std::min(rlo, w2min), up});
   }
+  // (with Ritz values above zero a proof hardly fails: no watching)
+  const bool big = ld_work(groups) >= kLdProofWork, watch = big && above == INFINITY;
   bool failed = false;
   for (const auto &[lo, up] : guess) {
     if (lo >= above) continue;  // its proof cannot hold
@@ -861,11 +864,11 @@ bool energy_by_logdet(mbd_handle *h, const std::vector<LdGroup> &groups, int cel
     if (!ld_nodes(lo, up, nd)) return false;
     double e = 0.0;
     int pd = 1;
-    if (failed && ld_work(groups) >= kLdProofWork) {
-      pd = ld_factor(h, groups, cells, nd, nd.n, nd.n + 1, e);
-      if (pd > 0) pd = ld_factor(h, groups, cells, nd, 0, nd.n, e);
+    if (failed && big) {
+      pd = ld_factor(h, groups, cells, nd, nd.n, nd.n + 1, watch, e);
+      if (pd > 0) pd = ld_factor(h, groups, cells, nd, 0, nd.n, false, e);
     } else {
-      pd = ld_factor(h, groups, cells, nd, 0, nd.n + 1, e);
+      pd = ld_factor(h, groups, cells, nd, 0, nd.n + 1, watch, e);
     }
     if (pd < 0 || !std::isfinite(e)) return false;
     if (pd) {
